@@ -637,7 +637,7 @@ def kernel_times(h):
     kern = {
         "dyn_adv": ["k_dyn_keg_zad"], "dyn_vor": ["k_dyn_vor"], "dyn_zdf": ["k_dyn_zdf"],
         "dyn_spg_ts": ["k_spg_cor1", "k_spg_cor2", "k_spg_init", "k_spg_p1a", "k_spg_p1b", "k_spg_s1", "k_spg_s2", "k_spg_s3",
-                       "k_spg_loop", "k_spg_p3a", "k_spg_p3b"],
+                       "k_spg_loop", "k_spg_blk", "k_spg_p3a", "k_spg_p3b"],
         "tra_adv_trp": ["k_tra_adv_trp"],
         "tra_adv_fct": ["k_fct_fused", "k_fct_cpt_fwd", "k_fct_h", "k_fct_hh", "k_fct_v", "k_fct_vz_reg", "k_fct_lim", "k_fct_vlim",
                         "k_fct_beta", "k_fct_final", "k_fct_low", "k_fct_ad"],
@@ -1070,6 +1070,9 @@ KERNEL_BYTES = {
     # S2: reads zwx zwy zssh_frc r1_e1e2t sshn_e sshb_e sshbb_e ssha; writes
     # ssha_e ssha zsshp2_e: 8 + 3 arrays
     "k_spg_s2": lambda w, i, j, k, f: 11 * 8 * i * j,
+    # a block of sub-steps: reads nine levels, seventeen constants and five
+    # sums, writes the levels and sums
+    "k_spg_blk": lambda w, i, j, k, f: 45 * 8 * i * j,
     # fused momentum step
     "k_step_dyn1": _b(5),        # r un vn wn, w ua va
     "k_step_dyn2": _b(11),       # r ua va un vn ub vb avm, w ua va un vn

@@ -539,8 +539,9 @@ static int register_domain(const nemo_hip_domain_t *h)
     if ((rc = dev_alloc((void **)&g_c->spg_bar, 64))) return rc;
     HIPCHK(hipMemset(g_c->spg_bar, 0, 64));
     if ((rc = dev_alloc((void **)&g_c->hsb_buf, dia_hsb_scratch_bytes() + 16 * sizeof(double)))) return rc;
-    HIPCHK(hipDeviceSynchronize());
     g_c->dom = d;
+    if ((rc = launch_spg_register())) return rc;
+    HIPCHK(hipDeviceSynchronize());
     g_c->have_domain = true;
     g_c->r2dt_tra = g_c->r2dt_zdf = g_c->r2dt_dyn = 2.0 * h->rdt;
     spg_ts_reset();

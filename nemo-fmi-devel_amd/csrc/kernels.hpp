@@ -30,6 +30,7 @@ template <typename T>
 int launch_dyn_zdf(double r2dt, const T *ub, const T *vb, T *ua, T *va, const T *avm, const double *rCdU_bot,
                    const double *ua_b, const double *va_b, const double *utau, const double *utau_b,
                    const double *vtau, const double *vtau_b);
+int launch_spg_register();   // once per registered domain
 int spg_ts_weights(const DevDomain &d, int ll_av, int ll_fw, int *jpit, double *zwgt1, double *zwgt2);
 // fused = 1: the 3D parts of phases 1 and 3 are left to the fused step kernels
 template <typename T> int launch_dyn_spg_ts(int kt, const nemo_hip_spg_ts_t *st, int fused = 0);

@@ -7,7 +7,10 @@
 // Phase 1 (3D -> 2D) is one column kernel (vertical sums of the trends,
 // removal of their mean, bottom baroclinic velocity) plus one 2D kernel (the
 // barotropic Coriolis / drag / wind forcing).  Phase 2 runs the `icycle`
-// dependent sub-steps as two 2D kernels each:
+// dependent sub-steps in blocks of several per launch, held on chip
+// (k_spg_blk, below).  Two cases take the sub-steps one by one, as two 2D
+// kernels each: ln_bt_av = F, whose levels carry over between calls, and the
+// t-point Coriolis term (ENT), which reads the extrapolated velocities:
 //   S2 (k_spg_s2)  the after sea level (flux divergence, lbc fill), its ssha
 //                  sum and the AB3-AM4 interpolated level zsshp2_e;
 //   S3 (k_spg_s3)  the after velocities (Coriolis, drag, pressure gradient,
@@ -635,7 +638,10 @@ struct S_spg_p3a {
     {
         THREAD_IJ_V(vb_, 1, 1);
         if (i > d.jpi || j > d.jpj) return;
-        const size_t ij = IJ(i, j);
+        point(d, first_euler, un_adv, vn_adv, ub2_b, vb2_b, un_bf, vn_bf, IJ(i, j));
+    }
+    __device__ __forceinline__ static void point(const DevDomain &d, int first_euler, double *un_adv, double *vn_adv, double *ub2_b, double *vb2_b, double *un_bf, double *vn_bf, size_t ij)
+    {
         const double r1_2 = 0.5, atfp = d.rn_atfp;
         const double zwx = un_adv[ij], zwy = vn_adv[ij];
         if (!first_euler) {
@@ -655,6 +661,258 @@ KERNEL void k_spg_p3a(DevDomain d, int first_euler, double * __restrict__ un_adv
                           double * __restrict__ vb2_b, double * __restrict__ un_bf, double * __restrict__ vn_bf)
 {
     S_spg_p3a::run(vb_hw(), d, first_euler, un_adv, vn_adv, ub2_b, vb2_b, un_bf, vn_bf);
+}
+
+// ---------------------------------------------------------------------------
+// Phase 2 by blocks of sub-steps: one launch makes `n` sub-steps of a region of
+// SPB x SPB points held on chip and writes the points the workgroup owns.
+//
+// The two kernels above move 45 arrays of FP64 per sub-step (17 of them
+// constants) and cost two launches.  Here a point's three time levels,
+// constants and time sums stay in its thread's registers for n sub-steps;
+// LDS passes the fluxes and zsshp2_e to the neighbours.  A sub-step reads one
+// point further, so a region carries a halo of n points on each side that has
+// a neighbour region (the halo's values go stale from the outside in, one
+// point per sub-step, and are never stored), recomputed with the operations of
+// the two-kernel loop: the results are its bits.
+//
+// Cyclic sides: the region's columns (rows) run on past the domain's last one
+// to its first, ring points included, each with its own constants.  A ring
+// point takes its after values from its lbc source, two points away across the
+// seam, so the halo is two points wider for every seam it can hold (spg_halo1d).
+//
+// Regions without a wet point: their levels are zero after three sub-steps and
+// stay zero, and their sums stay as they are, so they only store those zeros.
+//
+// 100 VGPRs (a region's 1024 threads may have 128), so one workgroup per CU.
+// A launch is bound by its loads (31 arrays of the region: about 9 us when
+// every CU loads one) and by the chain of each sub-step (two barriers, some 80
+// FP64 operations: 2.2 us with every CU busy, 1.1 us for one region alone).
+// All sub-steps of a call (44 at nn_baro = 30), two kernels each -> in blocks:
+// 1024x1024 2720 -> 1460 us, 512x512 793 -> 427 us, 251x333 500 -> 172 us,
+// 182x149 cyclic EEN 438 -> 126 us, 32x22 366 -> 51 us (one launch).
+// ---------------------------------------------------------------------------
+#define SPB 32                 // region edge: one point per thread of 1024
+#define SPB_MAXN 48            // sub-steps of one launch (the weights in its arguments)
+#define SPB_PAD 72             // LDS margin: neighbour and lbc-source offsets stay inside the arrays
+struct SpgLev {                // the levels now, before, before-before of u, v and the sea level
+    double *u[3], *v[3], *h[3];
+};
+struct SpgBlk {
+    int n, jn0, hx, hy, first, last, euler;
+    double rdtbt;
+    double wgt1[SPB_MAXN], wgt2[SPB_MAXN];
+    SpgLev in, out;
+    const double *un_b, *vn_b, *sshn, *hu, *hv, *r1_hu, *r1_hv;
+    double *ua_b, *va_b, *ssha, *un_adv, *vn_adv, *ub2_b, *vb2_b, *un_bf, *vn_bf;
+};
+// tile t along one direction: the region starts at x0 and owns o0..o1
+__host__ __device__ inline void spg_tile1d(int t, int h, int len, int per, int &x0, int &o0, int &o1)
+{
+    const int w = SPB - 2 * h;
+    if (per) {
+        o0 = 1 + t * w;
+        x0 = o0 - h;
+        o1 = o0 + w - 1 < len ? o0 + w - 1 : len;
+    } else {                   // no halo is needed at the domain's closed sides
+        x0 = 1 + t * w;
+        o0 = t == 0 ? 1 : x0 + h;
+        o1 = x0 + SPB - 1 >= len ? len : x0 + SPB - 1 - h;
+    }
+}
+// halo for n sub-steps along a direction of len points
+inline int spg_halo1d(int n, int len, int per)
+{
+    if (!per) return len <= SPB ? 0 : n;    // one region: no neighbour to read from
+    int m = 1;                              // seams in a halo of n + 2 m points
+    while (m < 1 + (n + 2 * m - 1) / len) m++;
+    return n + 2 * m;
+}
+inline int spg_ntiles1d(int h, int len, int per)
+{
+    const int w = SPB - 2 * h;
+    if (per) return (len + w - 1) / w;
+    return len <= SPB ? 1 : 1 + (len - SPB + w - 1) / w;
+}
+
+// SCH: the barotropic Coriolis term: 0 ENE and MIX, 1 ENS, 2 EEN and EET
+template <int SCH>
+struct S_spg_blk {
+    static constexpr int NTHR = SPB * SPB, WAVES = 4;
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const SpgBlk &a, const SpgWork &w)
+    {
+        constexpr int N = SPB * SPB + 2 * SPB_PAD;
+        __shared__ double sx[2][N], sy[2][N], sp[N], s1[N], s2[N];
+        unsigned bx, by;
+        xcd_tile_v(vb_, bx, by);
+        const int tid = (int)threadIdx.x, lx = tid % SPB, ly = tid / SPB, q = tid + SPB_PAD;
+        int x0, y0, ox0, ox1, oy0, oy1;
+        spg_tile1d((int)bx, a.hx, d.jpi, d.iper, x0, ox0, ox1);
+        spg_tile1d((int)by, a.hy, d.jpj, d.jper, y0, oy0, oy1);
+        int i = x0 + lx, j = y0 + ly;
+        const bool own = i >= ox0 && i <= ox1 && j >= oy0 && j <= oy1;
+        if (d.iper) i = ((i - 1) % d.jpi + d.jpi) % d.jpi + 1;
+        if (d.jper) j = ((j - 1) % d.jpj + d.jpj) % d.jpj + 1;
+        const bool ex = i >= 1 && i <= d.jpi && j >= 1 && j <= d.jpj;
+        const bool inner = ex && is_interior(d, i, j);
+        // a ring point with an lbc source: its place in the region
+        int si = i, sj = j, src = q;
+        const bool ring = ex && !inner && lbc_src(d, 'T', i, j, si, sj);
+        if (ring) src = q + (si == i ? 0 : i == 1 ? -2 : 2) + SPB * (sj == j ? 0 : j == 1 ? -2 : 2);
+        const bool cyc = (d.iper || d.jper) && __syncthreads_or(ring);
+        const size_t ij = ex ? IJ(i, j) : 0;
+        double ssm = 0.0, ssu = 0.0, ssv = 0.0;
+        if (ex) {
+            ssm = SSMASK(ij);
+            ssu = SSUMASK(ij);
+            ssv = SSVMASK(ij);
+        }
+        const bool dry = !__syncthreads_or(ssm != 0.0 || ssu != 0.0 || ssv != 0.0);
+        double u0 = 0.0, u1 = 0.0, u2 = 0.0, v0 = 0.0, v1 = 0.0, v2 = 0.0, h0 = 0.0, h1 = 0.0, h2 = 0.0;
+        double sum_h = 0.0, sum_u = 0.0, sum_v = 0.0, adv_u = 0.0, adv_v = 0.0;
+        const bool idle = dry && a.jn0 >= 3;
+        if (own && (!idle || a.last) && !a.first) {
+            sum_h = a.ssha[ij];
+            sum_u = a.ua_b[ij];
+            sum_v = a.va_b[ij];
+            adv_u = a.un_adv[ij];
+            adv_v = a.vn_adv[ij];
+        }
+        if (!idle) {
+            const Metrics<double> &m = d.md;
+            double hu = 0.0, hv = 0.0, e2u = 0.0, e1v = 0.0, r1_e2u = 0.0, r1_e1v = 0.0;
+            double r1_e1e2t = 0.0, fs = 0.0, r1_e1u = 0.0, r1_e2v = 0.0, cdu = 0.0, cdv = 0.0, r1_hu = 0.0, r1_hv = 0.0;
+            double fu = 0.0, fv = 0.0;
+            double c[SCH == 2 ? 7 : 3] = {};
+            if (ex) {
+                if (a.first) {
+                    u0 = a.un_b[ij];
+                    v0 = a.vn_b[ij];
+                    h0 = a.sshn[ij];
+                } else {
+                    u0 = a.in.u[0][ij]; u1 = a.in.u[1][ij]; u2 = a.in.u[2][ij];
+                    v0 = a.in.v[0][ij]; v1 = a.in.v[1][ij]; v2 = a.in.v[2][ij];
+                    h0 = a.in.h[0][ij]; h1 = a.in.h[1][ij]; h2 = a.in.h[2][ij];
+                }
+                hu = a.hu[ij]; hv = a.hv[ij];
+                e2u = m.e2u[ij]; e1v = m.e1v[ij];
+                if (own) {
+                    r1_e2u = m.r1_e2u[ij];
+                    r1_e1v = m.r1_e1v[ij];
+                }
+            }
+            if (inner) {
+                r1_e1e2t = m.r1_e1e2t[ij];
+                fs = w.zssh_frc[ij];
+                r1_e1u = m.r1_e1u[ij]; r1_e2v = m.r1_e2v[ij];
+                cdu = w.zCdU_u[ij]; cdv = w.zCdU_v[ij];
+                r1_hu = a.r1_hu[ij]; r1_hv = a.r1_hv[ij];
+                fu = w.zu_frc[ij]; fv = w.zv_frc[ij];
+                if constexpr (SCH == 2) {
+                    c[0] = A2(w.ftne, i, j); c[1] = A2(w.ftnw, i + 1, j); c[2] = A2(w.ftse, i, j);
+                    c[3] = A2(w.ftsw, i + 1, j); c[4] = A2(w.ftsw, i, j + 1); c[5] = A2(w.ftse, i, j + 1);
+                    c[6] = A2(w.ftnw, i, j);
+                } else {
+                    c[0] = A2(w.zwz, i, j); c[1] = A2(w.zwz, i, j - 1); c[2] = A2(w.zwz, i - 1, j);
+                }
+            }
+            for (int n = 0; n < a.n; n++) {
+                const int jn = a.jn0 + n + 1, b = n & 1;
+                double *X = sx[b], *Y = sy[b];
+                // extrapolated velocities and their fluxes, the un_adv sum (k_spg_s1)
+                double za1 = 1.781105, za2 = -1.06221, za3 = 0.281105;
+                if (jn < 3) { za1 = 1.0; za2 = 0.0; za3 = 0.0; }
+                const double ue = za1 * u0 + za2 * u1 + za3 * u2;
+                const double ve = za1 * v0 + za2 * v1 + za3 * v2;
+                const double x = e2u * ue * hu, y = e1v * ve * hv;
+                adv_u = adv_u + a.wgt2[n] * x * r1_e2u;
+                adv_v = adv_v + a.wgt2[n] * y * r1_e1v;
+                X[q] = x;
+                Y[q] = y;
+                __syncthreads();
+                // after sea level and zsshp2_e (k_spg_s2)
+                double zb0 = 0.614, zb1 = 0.285, zb2 = 0.088, zb3 = 0.013;
+                if (jn == 1) { zb0 = 1.0; zb1 = 0.0; zb2 = 0.0; zb3 = 0.0; }
+                else if (jn == 2) { zb0 = 1.0833333333333; zb1 = -0.1666666666666; zb2 = 0.0833333333333; zb3 = 0.0; }
+                double ha = 0.0;
+                if (inner) {
+                    const double zhdiv = (x - X[q - 1] + y - Y[q - SPB]) * r1_e1e2t;
+                    ha = (h0 - a.rdtbt * (fs + zhdiv)) * ssm;
+                }
+                double p = zb0 * ha + zb1 * h0 + zb2 * h1 + zb3 * h2;
+                if (cyc) {     // the ring's after sea level is its source's
+                    s1[q] = ha;
+                    __syncthreads();
+                    if (ring) {
+                        ha = s1[src];
+                        p = zb0 * ha + zb1 * h0 + zb2 * h1 + zb3 * h2;
+                    }
+                }
+                sp[q] = p;
+                __syncthreads();
+                // after velocities (k_spg_s3)
+                double nu = 0.0, nv = 0.0;
+                if (inner) {
+                    double zu_trd, zv_trd;
+                    if constexpr (SCH == 0) {
+                        const double zy1 = (Y[q - SPB] + Y[q - SPB + 1]) * r1_e1u, zy2 = (y + Y[q + 1]) * r1_e1u;
+                        const double zx1 = (X[q - 1] + X[q + SPB - 1]) * r1_e2v, zx2 = (x + X[q + SPB]) * r1_e2v;
+                        zu_trd = 0.25 * (c[1] * zy1 + c[0] * zy2);
+                        zv_trd = -(0.25 * (c[2] * zx1 + c[0] * zx2));
+                    } else if constexpr (SCH == 1) {
+                        const double zy1 = 0.125 * (Y[q - SPB] + Y[q - SPB + 1] + y + Y[q + 1]) * r1_e1u;
+                        const double zx1 = -(0.125 * (X[q - 1] + X[q + SPB - 1] + x + X[q + SPB]) * r1_e2v);
+                        zu_trd = zy1 * (c[1] + c[0]);
+                        zv_trd = zx1 * (c[2] + c[0]);
+                    } else {
+                        const double r1_12 = 1.0 / 12.0;
+                        zu_trd = r1_12 * r1_e1u * (c[0] * y + c[1] * Y[q + 1] + c[2] * Y[q - SPB] + c[3] * Y[q - SPB + 1]);
+                        zv_trd = -(r1_12 * r1_e2v *
+                                   (c[4] * X[q + SPB - 1] + c[5] * X[q + SPB] + c[6] * X[q - 1] + c[0] * x));
+                    }
+                    zu_trd = zu_trd + cdu * u0 * r1_hu;
+                    zv_trd = zv_trd + cdv * v0 * r1_hv;
+                    const double zu_spg = -(d.grav * (sp[q + 1] - p) * r1_e1u);
+                    const double zv_spg = -(d.grav * (sp[q + SPB] - p) * r1_e2v);
+                    nu = (u0 + a.rdtbt * ((1.0 - d.rn_scal_load) * zu_spg + zu_trd + fu)) * ssu;
+                    nv = (v0 + a.rdtbt * ((1.0 - d.rn_scal_load) * zv_spg + zv_trd + fv)) * ssv;
+                }
+                if (cyc) {
+                    s1[q] = nu;
+                    s2[q] = nv;
+                    __syncthreads();
+                    if (ring) {
+                        nu = s1[src];
+                        nv = s2[src];
+                    }
+                }
+                if (a.wgt1[n] != 0.0) {   // a zero weight leaves the sums as they are
+                    sum_h = sum_h + a.wgt1[n] * ha;
+                    sum_u = sum_u + a.wgt1[n] * nu;
+                    sum_v = sum_v + a.wgt1[n] * nv;
+                }
+                u2 = u1; u1 = u0; u0 = nu;
+                v2 = v1; v1 = v0; v0 = nv;
+                h2 = h1; h1 = h0; h0 = ha;
+            }
+        }
+        if (!own) return;
+        a.out.u[0][ij] = u0; a.out.u[1][ij] = u1; a.out.u[2][ij] = u2;
+        a.out.v[0][ij] = v0; a.out.v[1][ij] = v1; a.out.v[2][ij] = v2;
+        a.out.h[0][ij] = h0; a.out.h[1][ij] = h1; a.out.h[2][ij] = h2;
+        if (idle && !a.last) return;
+        a.ssha[ij] = sum_h;
+        a.ua_b[ij] = sum_u;
+        a.va_b[ij] = sum_v;
+        a.un_adv[ij] = adv_u;
+        a.vn_adv[ij] = adv_v;
+        if (a.last) S_spg_p3a::point(d, a.euler, a.un_adv, a.vn_adv, a.ub2_b, a.vb2_b, a.un_bf, a.vn_bf, ij);
+    }
+};
+template <int SCH>
+__global__ __launch_bounds__(SPB * SPB, 4) void k_spg_blk(DevDomain d, SpgBlk a, SpgWork w)
+{
+    S_spg_blk<SCH>::run(vb_hw(), d, a, w);
 }
 
 template <typename T>
@@ -818,6 +1076,57 @@ static bool spg_loop_coop(const DevDomain &d, const SpgWork &w, const nemo_hip_s
     return true;
 }
 
+// sub-steps per launch and halo of k_spg_blk.  Long blocks save launches and
+// re-reads, short ones halo: the block is the one with the least modelled time,
+//   launches * (launch + rounds * (load + sub-steps * sub-step)),
+// rounds being the regions over the CUs (one region's workgroup fills a CU).
+// Measured, us per call for 2, 3, ... 8, 10 sub-steps per launch:
+//   1024x1024  2134 1638 1473 1495 1546 1624 1795 2554   (chosen: 4)
+//   251x333     296  234  197  181  179  173  236  324   (7)
+//   512x512     712  483  437  517  501  488  492  752   (4)
+//   182x149 EEN 285  221  184  163  147  132  123  130   (9)
+// Members of a plan share one length, so that their launches batch.
+struct SpgBlkShape {
+    int n, hx, hy, ntx, nty;
+};
+static SpgBlkShape spg_blk_shape(const DevDomain &d, int icycle, bool plan)
+{
+    const double t_launch = 4.0, t_load = 8.0, t_sub = 1.3;   // us
+    const int ncu = 256;
+    SpgBlkShape best{};
+    double tb = 1e30;
+    for (int n = 1; n <= SPB_MAXN && n <= icycle; n++) {
+        if (plan && n != (icycle < 4 ? icycle : 4)) continue;
+        const int hx = spg_halo1d(n, d.jpi, d.iper), hy = spg_halo1d(n, d.jpj, d.jper);
+        if (2 * hx > SPB - 2 || 2 * hy > SPB - 2) break;
+        const int ntx = spg_ntiles1d(hx, d.jpi, d.iper), nty = spg_ntiles1d(hy, d.jpj, d.jper);
+        const int nl = (icycle + n - 1) / n;
+        const double rounds = (double)((ntx * nty + ncu - 1) / ncu);
+        const double t = nl * (t_launch + rounds * (t_load + n * t_sub));
+        if (t < tb) {
+            tb = t;
+            best = SpgBlkShape{n, hx, hy, ntx, nty};
+        }
+    }
+    return best;
+}
+
+// the domain's part of the barotropic Coriolis term that no field enters
+// (ENE, ENS, MIX: ff_f over the mean depth of the f-point's column, lines
+// 300-342): made once when the domain is registered
+int launch_spg_register()
+{
+    const DevDomain &d = nh::dom();
+    if (d.nvor_scheme != NEMO_NP_ENE && d.nvor_scheme != NEMO_NP_ENS && d.nvor_scheme != NEMO_NP_MIX) return 0;
+    SpgWork w{};
+    w.zwz = nh::scratch2(7);
+    w.zhf = nh::scratch2(8);
+    Grid2 g = grid2(d.jpi, d.jpj);
+    LAUNCH("dyn_spg_ts", k_spg_cor1, g, d, (const double *)nullptr, w);
+    LAUNCH("dyn_spg_ts", k_spg_cor2, g, d, (const double *)nullptr, w);
+    return 0;
+}
+
 template <typename T>
 int launch_dyn_spg_ts(int kt, const nemo_hip_spg_ts_t *st, int fused)
 {
@@ -844,8 +1153,8 @@ int launch_dyn_spg_ts(int kt, const nemo_hip_spg_ts_t *st, int fused)
     if (rc) return rc;
 
     Grid2 g = grid2(d.jpi, d.jpj);
-    LAUNCHB("dyn_spg_ts", k_spg_cor1, (S_spg_cor1), g, d, st->ht_n, w);
-    LAUNCHB("dyn_spg_ts", k_spg_cor2, (S_spg_cor2), g, d, st->ht_n, w);
+    if (d.nvor_scheme == NEMO_NP_EEN) LAUNCHB("dyn_spg_ts", k_spg_cor1, (S_spg_cor1), g, d, st->ht_n, w);
+    if (d.nvor_scheme == NEMO_NP_EEN || d.nvor_scheme == NEMO_NP_EET) LAUNCHB("dyn_spg_ts", k_spg_cor2, (S_spg_cor2), g, d, st->ht_n, w);
     if (d.nvor_scheme == NEMO_NP_EEN) LAUNCHB("dyn_spg_ts", k_spg_cor3, (S_spg_cor3), g, d, w);
     if (!fused)
         LAUNCHB("dyn_spg_ts", k_spg_p1a<T>, (S_spg_p1a<T>), g, d, ua, va, (const T *)un, (const T *)vn, st->r1_hu_n, st->r1_hv_n,
@@ -865,6 +1174,49 @@ int launch_dyn_spg_ts(int kt, const nemo_hip_spg_ts_t *st, int fused)
     } else if (nh::capturing()) {
         return nh::set_error(NEMO_HIP_ERR_STATE,
                              "dyn_spg_ts: ln_bt_av = F carries the barotropic levels between calls; not recordable");
+    }
+    // by blocks of sub-steps: levels set afresh, and a Coriolis term that reads
+    // the fluxes (the t-point one of ENT reads the extrapolated velocities)
+    if (ll_init && d.nvor_scheme != NEMO_NP_ENT && !nh::tune(nh::T_SPG_PERSISTENT)) {
+        const SpgBlkShape sh = spg_blk_shape(d, icycle, nh::planning());
+        const int nl = (icycle + sh.n - 1) / sh.n;
+        const SpgLev lev[2] = {{{ube[0], ube[1], ube[2]}, {vbe[0], vbe[1], vbe[2]}, {sse[0], sse[1], sse[2]}},
+                               {{s2[13], s2[14], s2[15]}, {s2[16], s2[17], s2[29]}, {s2[30], s2[31], nh::scratch2(32)}}};
+        Grid2 gb;
+        gb.block = dim3(SPB * SPB, 1, 1);
+        gb.grid = dim3((unsigned)sh.ntx, (unsigned)sh.nty, 1);
+        int jn = 0;
+        for (int l = 0; l < nl; l++) {
+            SpgBlk a{};
+            a.n = (icycle - jn + nl - l - 1) / (nl - l);   // equal shares, none above sh.n
+            a.jn0 = jn;
+            a.hx = sh.hx; a.hy = sh.hy;
+            a.first = l == 0;
+            a.last = l == nl - 1;
+            a.euler = kt == d.nit000 && d.neuler == 0;
+            a.rdtbt = rdtbt;
+            for (int n = 0; n < a.n; n++) {
+                a.wgt1[n] = wgt1[jn + n];
+                a.wgt2[n] = wgt2[jn + n];
+            }
+            a.out = lev[(nl - 1 - l) & 1];   // the last one leaves the levels where the next call looks for them
+            a.in = lev[(nl - l) & 1];
+            a.un_b = st->un_b; a.vn_b = st->vn_b; a.sshn = st->sshn;
+            a.hu = st->hu_n; a.hv = st->hv_n; a.r1_hu = st->r1_hu_n; a.r1_hv = st->r1_hv_n;
+            a.ua_b = st->ua_b; a.va_b = st->va_b; a.ssha = st->ssha; a.un_adv = st->un_adv; a.vn_adv = st->vn_adv;
+            a.ub2_b = st->ub2_b; a.vb2_b = st->vb2_b; a.un_bf = st->un_bf; a.vn_bf = st->vn_bf;
+            switch (d.nvor_scheme) {
+            case NEMO_NP_ENE:
+            case NEMO_NP_MIX: LAUNCHB("dyn_spg_ts", (k_spg_blk<0>), (S_spg_blk<0>), gb, d, a, w); break;
+            case NEMO_NP_ENS: LAUNCHB("dyn_spg_ts", (k_spg_blk<1>), (S_spg_blk<1>), gb, d, a, w); break;
+            default: LAUNCHB("dyn_spg_ts", (k_spg_blk<2>), (S_spg_blk<2>), gb, d, a, w); break;
+            }
+            jn += a.n;
+        }
+        if (!fused)
+            LAUNCHB("dyn_spg_ts", k_spg_p3b<T>, (S_spg_p3b<T>), g, d, r1_2dt_b, ua, va, un, vn, st->ua_b, st->va_b, st->ub_b, st->vb_b,
+                   st->un_adv, st->vn_adv, st->r1_hu_n, st->r1_hv_n, st->un_b, st->vn_b);
+        return 0;
     }
     LAUNCHB("dyn_spg_ts", k_spg_init, (S_spg_init), g, d, ll_init, st->un_b, st->vn_b, st->sshn, ube[ru[0]], vbe[ru[0]], sse[rs[0]],
            ube[ru[1]], vbe[ru[1]], sse[rs[1]], ube[ru[2]], vbe[ru[2]], sse[rs[2]], st->ua_b, st->va_b, st->ssha,
