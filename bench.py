@@ -641,7 +641,7 @@ def kernel_times(h):
         "tra_adv_trp": ["k_tra_adv_trp"],
         "tra_adv_fct": ["k_fct_fused", "k_fct_cpt_fwd", "k_fct_h", "k_fct_hh", "k_fct_v", "k_fct_vz_reg", "k_fct_lim", "k_fct_vlim",
                         "k_fct_beta", "k_fct_final", "k_fct_low", "k_fct_ad"],
-        "tra_ldf_iso": ["k_ldf_iso_coef", "k_tra_ldf_iso", "k_fill3", "k_copy3"], "tra_zdf": ["k_tra_zdf", "k_tra_zdf_reg", "k_clamp_ring"],
+        "tra_ldf_iso": ["k_ldf_iso_coef", "k_tra_ldf_iso", "k_fill3"], "tra_zdf": ["k_tra_zdf", "k_tra_zdf_reg", "k_clamp_ring"],
         "lbc_lnk": ["k_lbc"],
         "step_dyn": ["k_step_dyn1", "k_step_dyn2"],
         "step_tra": ["k_fct_fused", "k_fct_cpt_fwd", "k_fct_h", "k_fct_hh", "k_fct_v", "k_fct_vz_reg", "k_fct_lim", "k_fct_vlim",

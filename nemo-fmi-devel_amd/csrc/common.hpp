@@ -91,7 +91,6 @@ __device__ __forceinline__ T &at32(T *p, uint32_t e)
 }
 #define IJK32(i, j, k) ((((uint32_t)((k) - 1) * (uint32_t)d.jpj + (uint32_t)((j) - 1)) * (uint32_t)d.jpi) + (uint32_t)((i) - 1))
 #define A3(p, i, j, k) at32((p), IJK32(i, j, k))
-#define E3(p, ij, k) (p)[(size_t)((k) - 1) * d.e3_sk + (size_t)(ij) * d.e3_sij]
 
 // Plane-relative access for k-marched kernels: the level base pointer is
 // uniform across the wave (kept in SGPRs), the lane's in-plane offset is a
@@ -118,6 +117,9 @@ __device__ __forceinline__ void stp(T *pl, uint32_t ij, T v)
 {
     *(T *)((char *)pl + (uint32_t)(ij * (uint32_t)sizeof(T))) = v;
 }
+// vertical scale factors: the level's base is uniform, the in-plane offset (0
+// for a horizontally uniform coordinate) is fixed for a column
+#define E3(p, ij, k) ldp((p) + (size_t)((k) - 1) * d.e3_sk, (uint32_t)(ij) * (uint32_t)d.e3_sij)
 #define IJ32(i, j) ((uint32_t)((j) - 1) * (uint32_t)d.jpi + (uint32_t)((i) - 1))
 
 template <typename T>
@@ -168,6 +170,27 @@ __device__ __forceinline__ double psurf(const uint32_t *p, uint32_t ij)
 #define WMASK(T_, i, j, k) wpmask<T_, 0>(d.ktu, IJ32(i, j), k)
 #define WUMASK(T_, i, j, k) wpmask<T_, 16>(d.ktu, IJ32(i, j), k)
 #define WVMASK(T_, i, j, k) wpmask<T_, 0>(d.kvf, IJ32(i, j), k)
+
+// Level ranges of a wave (call with all 64 lanes active).  A wave's columns are
+// 64 neighbours along i, so most waves are wet, or dry, in all of them: a march
+// runs mask-free down to the last level where every mask of its stencil is 1,
+// with masks down to its deepest wet level, and stops there where the levels
+// below are known to give zeros.
+__device__ __forceinline__ int wave_max(int v)
+{
+#pragma unroll
+    for (int o = 32; o; o >>= 1) v = max(v, __shfl_xor(v, o));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ int wave_min(int v) { return -wave_max(-v); }
+
+// 1 / max(n, 1) for a sum n of up to four masks (0 or 1 each): the quotients the
+// division gives, without it
+template <typename T>
+__device__ __forceinline__ T rmask4(T n)
+{
+    return n > T(3.5) ? T(0.25) : n > T(2.5) ? T(1) / T(3) : n > T(1.5) ? T(0.5) : T(1);
+}
 
 // A column Thomas solve may keep the FP64 pivot of every ZDF_SEG-th level
 // only (a checkpoint in scratch): the back substitution then recomputes the
