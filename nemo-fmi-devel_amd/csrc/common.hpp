@@ -120,6 +120,15 @@ __device__ __forceinline__ void stp(T *pl, uint32_t ij, T v)
 // vertical scale factors: the level's base is uniform, the in-plane offset (0
 // for a horizontally uniform coordinate) is fixed for a column
 #define E3(p, ij, k) ldp((p) + (size_t)((k) - 1) * d.e3_sk, (uint32_t)(ij) * (uint32_t)d.e3_sij)
+// element k of a table no kernel writes, k uniform: a scalar load.  (A plain load
+// becomes a vector one where the compiler cannot rule out that a store of the
+// kernel reached the table.)
+template <typename T>
+__device__ __forceinline__ T uld(const T *p, int k)
+{
+    typedef const T __attribute__((address_space(4))) *cp;
+    return ((cp)(uintptr_t)p)[k];
+}
 #define IJ32(i, j) ((uint32_t)((j) - 1) * (uint32_t)d.jpi + (uint32_t)((i) - 1))
 
 template <typename T>

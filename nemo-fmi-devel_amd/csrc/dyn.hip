@@ -455,13 +455,47 @@ template int launch_dyn_vor<float>(const float *, const float *, float *, float 
 struct PreIdentity {
     template <typename T>
     __device__ __forceinline__ T operator()(int, T x) const { return x; }
+    template <typename T>
+    __device__ __forceinline__ T wet(T x) const { return x; }   // where the level's mask is 1
 };
-template <typename T, typename Pre = PreIdentity>
+// the levels of a wave's u (comp 0) or v (comp 1) columns, called with all 64
+// lanes active (on: the lane has a column).  all: the last level above which
+// every lane's masks are 1 and no bottom drag enters; end: the deepest level
+// with a mask or a drag that is not zero.  Below it every row is x = 0.
+struct ZdfLev {
+    int all, end;
+};
+__device__ __forceinline__ ZdfLev zdf_levels(const DevDomain &d, int comp, int i, int j, bool on)
+{
+    int a = d.jpk, e = 1;
+    if (on) {
+        const uint32_t ij = IJ32(i, j);
+        const KRange &kr = comp ? d.kV : d.kU;
+        const int x0 = kr.k0[ij], x1 = kr.k1[ij];
+        e = max(x1, 1);
+        if (is_interior(d, i, j)) {
+            const int ikb = comp ? d.mbkv[ij] : d.mbku[ij];
+            e = max(e, ikb);
+            a = x0 > 1 ? 0 : min(x1, ikb);
+        }
+    }
+    const int all = wave_min(a) - 1, end = min(wave_max(e), d.jpk - 1);
+    return ZdfLev{min(all, end - 1), end};
+}
+//
+// The sweeps run from the surface to the wave's deepest masked or dragged level
+// (zdf_levels), above its first bottom without mask tests; below, every row is
+// x = 0 and is only stored.  A segment's operands are loaded together, and
+// horizontally uniform scale factors (E3U) are scalar loads.
+// k_step_dyn2, 1024x1024x75 FP32 (47 % of the cells dry): 1526 -> 1036 us (4.5
+// TB/s); k_dyn_zdf, 512x512x75 FP64: 590 -> 413 us; reading the next segment
+// ahead as well, 20 VGPRs more, gives 1202 and 437.
+template <bool E3U, typename T, typename Pre = PreIdentity>
 __device__ __forceinline__ void zdf_column(const DevDomain &d, double r2dt, int comp, int i, int j,
                                            const T *__restrict__ pb, T *__restrict__ pa, const T *__restrict__ avm,
                                            const double *__restrict__ rCdU_bot, const double *__restrict__ pa_b,
                                            const double *__restrict__ tau, const double *__restrict__ tau_b,
-                                           double *__restrict__ zwd_s, Pre pre = Pre())
+                                           double *__restrict__ zwd_s, const ZdfLev lv, Pre pre = Pre())
 {
     const Metrics<T> &m = met<T>(d);
     const int jpk = d.jpk;
@@ -478,46 +512,77 @@ __device__ __forceinline__ void zdf_column(const DevDomain &d, double r2dt, int 
     const bool inner = is_interior(d, i, j);
     const bool rm_b = d.ln_drgimp && d.ln_dynspg_ts;
     const double ab = rm_b ? pa_b[ij] : 0.0;
+    const auto dry = [&]() {   // the levels below the wave's deepest one
+        for (int k = lv.end + 1; k <= jpk - 1; k++) stp(plane_ptr(pa, plane, k), ij, T(0));
+    };
     if (!inner) {
-        for (int k = 1; k <= jpk - 1; k++) {
+        for (int k = 1; k <= lv.end; k++) {
             const double xm = xmask(k);
             double a = ((double)ldp(plane_ptr(pb, plane, k), ij) +
                         r2dt * (double)pre(k, ldp((const T *)plane_ptr(pa, plane, k), ij))) * xm;
             if (rm_b) a = (a - ab) * xm;
             stp(plane_ptr(pa, plane, k), ij, (T)a);
         }
+        dry();
         return;
     }
     const int ikb = comp ? d.mbkv[ij] : d.mbku[ij];
     const double csum = rCdU_bot[ijn] + rCdU_bot[ij];
     const double zdt = r2dt * 0.5;
-    // off-diagonal at w-level k (k >= 2), lines 208-243
-    auto zzw = [&](int k, double ze3) {
-        const T *ak = plane_ptr(avm, plane, k);
-        return -(zdt * ((double)ldp(ak, ijn) + (double)ldp(ak, ij)) / (ze3 * (double)E3(e3xw, ij, k)) * wxmask(k));
+    // off-diagonal at w-level k (k >= 2), lines 208-243, from loaded operands:
+    // avm at the face's two t-points, e3xw.  WET: its mask is 1
+    auto zzw_v = [&](auto wet, int k, double ze3, T a_n, T a_c, T e3w) {
+        const double q = zdt * ((double)a_n + (double)a_c) / (ze3 * (double)e3w);
+        return decltype(wet)::value ? -q : -(q * wxmask(k));
     };
-    // zzw from loaded operands: avm at the face's two t-points, e3xw
-    auto zzw_v = [&](int k, double ze3, T a_n, T a_c, T e3w) {
-        return -(zdt * ((double)a_n + (double)a_c) / (ze3 * (double)e3w) * wxmask(k));
-    };
-    auto ld_avm = [&](int k, T &a_n, T &a_c, T &e3w) {   // level k <= jpk
+    // level k <= jpk; the scale factors by vector load with the level's other
+    // operands or, horizontally uniform, by scalar load where used
+    auto ld_avm = [&](int k, T &a_n, T &a_c, T &e3w) {
         const T *ak = plane_ptr(avm, plane, k);
         a_n = ldp(ak, ijn);
         a_c = ldp(ak, ij);
-        e3w = E3(e3xw, ij, k);
+        if constexpr (!E3U) e3w = E3(e3xw, ij, k);
+    };
+    auto zz = [&](auto wet, int k, double ze3, T a_n, T a_c, T e3w) {
+        return zzw_v(wet, k, ze3, a_n, a_c, E3U ? uld(e3xw, k - 1) : e3w);
+    };
+    auto ze3_of = [&](int k, T v) {
+        const double e = (double)(E3U ? uld(e3x, k - 1) : v);
+        return (1.0 - r_vvl) * e + r_vvl * e;
+    };
+    const std::false_type masked{};
+    const std::true_type unmasked{};
+    const int kend = lv.end;
+    // the operands of ZDF_SEG levels from k0 (pb, pa, e3x) and of the w-levels
+    // under them (avm, e3xw); levels past kend load kend's and are not used.
+    // A segment's operands are loaded together (a load issued after a store to
+    // pa waits for it)
+    struct Seg {
+        T b[ZDF_SEG], t[ZDF_SEG], e[ZDF_SEG], wn[ZDF_SEG], wc[ZDF_SEG], we[ZDF_SEG];
+    };
+    auto fetch = [&](int k0, Seg &g, bool with_b) {
+#pragma unroll
+        for (int q = 0; q < ZDF_SEG; q++) {
+            const int k = min(k0 + q, kend);
+            g.t[q] = ldp((const T *)plane_ptr(pa, plane, k), ij);
+            if (with_b) g.b[q] = ldp(plane_ptr(pb, plane, k), ij);
+            if constexpr (!E3U) g.e[q] = E3(e3x, ij, k);
+            ld_avm(k + 1, g.wn[q], g.wc[q], g.we[q]);
+        }
     };
     double zws_prev, zwd_prev, a_prev;
-    // the operands of level k (pb, pa, e3x) and of w-level k + 1 (avm, e3xw)
-    // are loaded one level ahead
-    T w1n, w1c, w1e;   // w-level k + 1 of the current level
+    T w1n, w1c, w1e = T(1);   // w-level k of the level to come
+    Seg cur;
     ld_avm(2, w1n, w1c, w1e);
     {   // k = 1: surface row with the wind stress
         const double xm = xmask(1);
         double a = ((double)ldp(pb, ij) + r2dt * (double)pre(1, ldp((const T *)pa, ij))) * xm;
         if (rm_b) a = (a - ab) * xm;
-        const double ze3 = (1.0 - r_vvl) * (double)E3(e3x, ij, 1) + r_vvl * (double)E3(e3x, ij, 1);
+        T e1 = T(1);
+        if constexpr (!E3U) e1 = E3(e3x, ij, 1);
+        const double ze3 = ze3_of(1, e1);
         if (rm_b && 1 == ikb) a = a + r2dt * 0.5 * csum * ab / ze3;
-        const double zws = zzw_v(2, ze3, w1n, w1c, w1e);
+        const double zws = zz(masked, 2, ze3, w1n, w1c, w1e);
         double zwd = 1.0 - zws;
         if (d.ln_drgimp && 1 == ikb) zwd = zwd - r2dt * 0.5 * csum / ze3;
         a = a + r2dt * 0.5 * (tau_b[ij] + tau[ij]) / (ze3 * d.rau0) * xm;
@@ -526,28 +591,27 @@ __device__ __forceinline__ void zdf_column(const DevDomain &d, double r2dt, int 
         zwd_prev = zwd;
         a_prev = a;
     }
-    {
-        T b_c = ldp(plane_ptr(pb, plane, 2), ij), t_c = ldp((const T *)plane_ptr(pa, plane, 2), ij);
-        T e_c = E3(e3x, ij, 2);
-        T w0n = w1n, w0c = w1c, w0e = w1e;   // w-level k
-        ld_avm(3 <= jpk ? 3 : jpk, w1n, w1c, w1e);
-#pragma unroll 4
-        for (int k = 2; k <= jpk - 1; k++) {
-            // level k + 1's operands (within the arrays: levels <= jpk)
-            const int kn = k + 1, kw = k + 2 <= jpk ? k + 2 : jpk;
-            const T b_n = ldp(plane_ptr(pb, plane, kn), ij), t_n = ldp((const T *)plane_ptr(pa, plane, kn), ij);
-            const T e_n = E3(e3x, ij, kn);
-            T w2n, w2c, w2e;
-            ld_avm(kw, w2n, w2c, w2e);
-            const double xm = xmask(k);
-            double a = ((double)b_c + r2dt * (double)pre(k, t_c)) * xm;
-            if (rm_b) a = (a - ab) * xm;
-            const double ze3 = (1.0 - r_vvl) * (double)e_c + r_vvl * (double)e_c;
-            if (rm_b && k == ikb) a = a + r2dt * 0.5 * csum * ab / ze3;
-            const double zwi = zzw_v(k, ze3, w0n, w0c, w0e);
-            const double zws = zzw_v(k + 1, ze3, w1n, w1c, w1e);
+    auto down = [&](auto wet, int k0) {   // ZDF_SEG levels of the forward sweep
+        constexpr bool WET = decltype(wet)::value;
+#pragma unroll
+        for (int q = 0; q < ZDF_SEG; q++) {
+            const int k = k0 + q;
+            if (!WET && k > kend) break;
+            double a;
+            if constexpr (WET) {
+                a = (double)cur.b[q] + r2dt * (double)pre.wet(cur.t[q]);
+                if (rm_b) a = a - ab;
+            } else {
+                const double xm = xmask(k);
+                a = ((double)cur.b[q] + r2dt * (double)pre(k, cur.t[q])) * xm;
+                if (rm_b) a = (a - ab) * xm;
+            }
+            const double ze3 = ze3_of(k, cur.e[q]);
+            if (!WET && rm_b && k == ikb) a = a + r2dt * 0.5 * csum * ab / ze3;
+            const double zwi = zz(wet, k, ze3, w1n, w1c, w1e);
+            const double zws = zz(wet, k + 1, ze3, cur.wn[q], cur.wc[q], cur.we[q]);
             double zwd = 1.0 - zwi - zws;
-            if (d.ln_drgimp && k == ikb) zwd = zwd - r2dt * 0.5 * csum / ze3;
+            if (!WET && d.ln_drgimp && k == ikb) zwd = zwd - r2dt * 0.5 * csum / ze3;
             zwd = zwd - zwi * zws_prev / zwd_prev;
             a = a - zwi / zwd_prev * a_prev;
             if (k % ZDF_SEG == 0) stp(plane_ptr(zwd_s, plane, k), ij, zwd);   // checkpoint pivots only
@@ -555,68 +619,80 @@ __device__ __forceinline__ void zdf_column(const DevDomain &d, double r2dt, int 
             zws_prev = zws;
             zwd_prev = zwd;
             a_prev = a;
-            b_c = b_n; t_c = t_n; e_c = e_n;
-            w0n = w1n; w0c = w1c; w0e = w1e;
-            w1n = w2n; w1c = w2c; w1e = w2e;
+            w1n = cur.wn[q]; w1c = cur.wc[q]; w1e = cur.we[q];
         }
+    };
+    int k0 = 2;
+    for (; k0 + ZDF_SEG - 1 <= lv.all; k0 += ZDF_SEG) {
+        fetch(k0, cur, true);
+        down(unmasked, k0);
     }
-    double x = a_prev / zwd_prev;
-    stp(plane_ptr(pa, plane, jpk - 1), ij, (T)x);
-    // levels jpk-2 .. 1 by segments of ZDF_SEG levels, bottom segment first:
+    for (; k0 <= kend; k0 += ZDF_SEG) {
+        fetch(k0, cur, true);
+        down(masked, k0);
+    }
+    // levels kend-1 .. 1 by segments of ZDF_SEG levels, bottom segment first:
     // the forward sweep kept the pivot of every ZDF_SEG-th level only, so a
     // segment first recomputes its pivots from the one above it (the
-    // operations of the forward sweep), then substitutes back.  Each
-    // segment's operands are loaded together, from levels within the arrays.
-    const int kl = jpk - 2;
-    for (int s = (kl + ZDF_SEG - 1) / ZDF_SEG - 1; s >= 0; s--) {
-        const int k0 = s * ZDF_SEG + 1;
-        T e[ZDF_SEG], t[ZDF_SEG], wn[ZDF_SEG], wc[ZDF_SEG], we[ZDF_SEG];   // level k, w-level k + 1
-#pragma unroll
-        for (int q = 0; q < ZDF_SEG; q++) {
-            const int k = k0 + q <= kl ? k0 + q : kl;
-            e[q] = E3(e3x, ij, k);
-            t[q] = ldp((const T *)plane_ptr(pa, plane, k), ij);
-            ld_avm(k + 1, wn[q], wc[q], we[q]);
-        }
-        double zwd_p = 0.0, zws_p = 0.0;
-        T an = T(0), ac = T(0), aw = T(0);   // w-level k0
-        if (s > 0) {
-            zwd_p = ldp((const double *)plane_ptr(zwd_s, plane, k0 - 1), ij);
-            const T ep = E3(e3x, ij, k0 - 1);
-            ld_avm(k0, an, ac, aw);
-            const double ze3p = (1.0 - r_vvl) * (double)ep + r_vvl * (double)ep;
-            zws_p = zzw_v(k0, ze3p, an, ac, aw);
-        }
+    // operations of the forward sweep), then substitutes back
+    const int kl = kend - 1;
+    int s = (kl + ZDF_SEG - 1) / ZDF_SEG - 1;
+    T an, ac, aw = T(1), ep = T(1);   // w-level k0 of the segment, e3x above it, and the checkpoint pivot
+    double ckp = 1.0;
+    auto fetch_top = [&](int kt) {
+        if (kt == 1) return;
+        ld_avm(kt, an, ac, aw);
+        if constexpr (!E3U) ep = E3(e3x, ij, kt - 1);
+        ckp = ldp((const double *)plane_ptr(zwd_s, plane, kt - 1), ij);
+    };
+    an = ac = T(0);
+    // the last row of the whole column divides the value in hand, any other the
+    // one rounded to storage, as if it had been stored and the zero below
+    // substituted
+    double x = (kend == jpk - 1 ? a_prev : (double)(T)a_prev) / zwd_prev;
+    stp(plane_ptr(pa, plane, kend), ij, (T)x);
+    dry();
+    auto up = [&](auto wet) {
+        constexpr bool WET = decltype(wet)::value;
+        const int kt = s * ZDF_SEG + 1;
+        fetch(kt, cur, false);
+        fetch_top(kt);
+        T pn = an, pc = ac, pw = aw;
+        double zwd_p = ckp, zws_p = 0.0;
+        if (s > 0) zws_p = zz(wet, kt, ze3_of(kt - 1, ep), an, ac, aw);
         double piv[ZDF_SEG], zsv[ZDF_SEG];
 #pragma unroll
         for (int q = 0; q < ZDF_SEG; q++) {
-            const int k = k0 + q;
-            const double ze3 = (1.0 - r_vvl) * (double)e[q] + r_vvl * (double)e[q];
-            const double zws = zzw_v(k + 1, ze3, wn[q], wc[q], we[q]);
+            const int k = kt + q;
+            const double ze3 = ze3_of(k, cur.e[q]);
+            const double zws = zz(wet, k + 1, ze3, cur.wn[q], cur.wc[q], cur.we[q]);
             double zwd;
             if (k == 1) {
                 zwd = 1.0 - zws;
-                if (d.ln_drgimp && 1 == ikb) zwd = zwd - r2dt * 0.5 * csum / ze3;
+                if (!WET && d.ln_drgimp && 1 == ikb) zwd = zwd - r2dt * 0.5 * csum / ze3;
             } else {
-                const double zwi = q == 0 ? zzw_v(k, ze3, an, ac, aw) : zzw_v(k, ze3, wn[q - 1], wc[q - 1], we[q - 1]);
+                const double zwi = zz(wet, k, ze3, pn, pc, pw);
                 zwd = 1.0 - zwi - zws;
-                if (d.ln_drgimp && k == ikb) zwd = zwd - r2dt * 0.5 * csum / ze3;
+                if (!WET && d.ln_drgimp && k == ikb) zwd = zwd - r2dt * 0.5 * csum / ze3;
                 zwd = zwd - zwi * zws_p / zwd_p;
             }
             piv[q] = zwd;
             zsv[q] = zws;
             zws_p = zws;
             zwd_p = zwd;
+            pn = cur.wn[q]; pc = cur.wc[q]; pw = cur.we[q];
         }
 #pragma unroll
         for (int q = ZDF_SEG - 1; q >= 0; q--) {
-            const int k = k0 + q;
-            if (k <= kl) {
-                x = ((double)t[q] - zsv[q] * x) / piv[q];
+            const int k = kt + q;
+            if (WET || k <= kl) {
+                x = ((double)cur.t[q] - zsv[q] * x) / piv[q];
                 stp(plane_ptr(pa, plane, k), ij, (T)x);
             }
         }
-    }
+    };
+    for (; s >= 0 && (s + 1) * ZDF_SEG > lv.all; s--) up(masked);
+    for (; s >= 0; s--) up(unmasked);
 }
 
 // The same column solve in the FP32 storage form with jpk <= KMAX: the
@@ -761,28 +837,31 @@ __device__ __forceinline__ void zdf_column_reg(const DevDomain &d, double r2dt, 
 // 75 of the full-size configurations
 #define ZDF_REG_KMAX 76
 
-template <typename T, bool REG>
+template <typename T, bool REG, bool E3U>
 struct S_dyn_zdf {
     static constexpr int NTHR = NH_BLOCK, WAVES = 2;
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double r2dt, const T * __restrict__ ub, const T * __restrict__ vb, T * __restrict__ ua, T * __restrict__ va, const T * __restrict__ avm, const double * __restrict__ rCdU_bot, const double * __restrict__ ua_b, const double * __restrict__ va_b, const double * __restrict__ utau, const double * __restrict__ utau_b, const double * __restrict__ vtau, const double * __restrict__ vtau_b, double * __restrict__ zwd_s)
     {
         THREAD_IJ_V(vb_, 1, 1);
-        if (i > d.jpi || j > d.jpj) return;
+        const bool on = i <= d.jpi && j <= d.jpj;
         if constexpr (REG) {
+            if (!on) return;
             zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b);
             zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b);
         } else {
-            zdf_column(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b, zwd_s);
-            zdf_column(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b, zwd_s);
+            const ZdfLev lu = zdf_levels(d, 0, i, j, on), lv = zdf_levels(d, 1, i, j, on);
+            if (!on) return;
+            zdf_column<E3U>(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b, zwd_s, lu);
+            zdf_column<E3U>(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b, zwd_s, lv);
         }
     }
 };
-template <typename T, bool REG>
+template <typename T, bool REG, bool E3U>
 KERNEL_W(2) void k_dyn_zdf(DevDomain d, double r2dt, const T * __restrict__ ub, const T * __restrict__ vb, T * __restrict__ ua, T * __restrict__ va, const T * __restrict__ avm,
                           const double * __restrict__ rCdU_bot, const double * __restrict__ ua_b, const double * __restrict__ va_b, const double * __restrict__ utau,
                           const double * __restrict__ utau_b, const double * __restrict__ vtau, const double * __restrict__ vtau_b, double * __restrict__ zwd_s)
 {
-    S_dyn_zdf<T, REG>::run(vb_hw(), d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau, utau_b, vtau, vtau_b, zwd_s);
+    S_dyn_zdf<T, REG, E3U>::run(vb_hw(), d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau, utau_b, vtau, vtau_b, zwd_s);
 }
 // the register form applies: FP32 storage, jpk <= ZDF_REG_KMAX, switch zdf_reg
 template <typename T>
@@ -802,13 +881,17 @@ int launch_dyn_zdf(double r2dt, const T *ub, const T *vb, T *ua, T *va, const T 
     // forward-substituted values stay in ua/va at storage precision
     if constexpr (sizeof(T) == 4) {
         if (zdf_reg<T>(d)) {
-            LAUNCHB("dyn_zdf", (k_dyn_zdf<T, true>), (S_dyn_zdf<T, true>), g, d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau,
+            LAUNCHB("dyn_zdf", (k_dyn_zdf<T, true, false>), (S_dyn_zdf<T, true, false>), g, d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau,
                    utau_b, vtau, vtau_b, zwd);
             return 0;
         }
     }
-    LAUNCHB("dyn_zdf", (k_dyn_zdf<T, false>), (S_dyn_zdf<T, false>), g, d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau, utau_b,
-           vtau, vtau_b, zwd);
+#define ZDF_LAUNCH(U) \
+    LAUNCHB("dyn_zdf", (k_dyn_zdf<T, false, U>), (S_dyn_zdf<T, false, U>), g, d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau, \
+           utau_b, vtau, vtau_b, zwd)
+    if (d.e3_sij == 0) ZDF_LAUNCH(true);
+    else ZDF_LAUNCH(false);
+#undef ZDF_LAUNCH
     return 0;
 }
 template int launch_dyn_zdf<double>(double, const double *, const double *, double *, double *, const double *,
@@ -969,29 +1052,48 @@ struct PreSpg {
         if (inner) x = (T)((double)x - s * xm);
         return (T)((double)x + dd);
     }
+    __device__ __forceinline__ T wet(T x) const { return (T)((double)(T)((double)x - s) + dd); }
 };
 
-template <typename T, bool REG>
+template <typename T, bool REG, bool E3U>
 struct S_step_dyn2 {
     static constexpr int NTHR = NH_BLOCK, WAVES = 2;
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double r2dt, double r1_2dt_b, const T *__restrict__ ub, const T *__restrict__ vb, T *__restrict__ ua, T *__restrict__ va, T *__restrict__ un, T *__restrict__ vn, const T *__restrict__ avm, const double *__restrict__ rCdU_bot, const double *__restrict__ ua_b, const double *__restrict__ va_b, const double *__restrict__ ub_b, const double *__restrict__ vb_b, const double *__restrict__ un_adv, const double *__restrict__ vn_adv, const double *__restrict__ r1_hu_n, const double *__restrict__ r1_hv_n, const double *__restrict__ un_b, const double *__restrict__ vn_b, const double *__restrict__ su_s, const double *__restrict__ sv_s, const double *__restrict__ utau, const double *__restrict__ utau_b, const double *__restrict__ vtau, const double *__restrict__ vtau_b, double *__restrict__ zwd_s)
     {
         THREAD_IJ_V(vb_, 1, 1);
-        if (i > d.jpi || j > d.jpj) return;
+        const bool on = i <= d.jpi && j <= d.jpj;
+        const ZdfLev lu = zdf_levels(d, 0, i, j, on), lv = zdf_levels(d, 1, i, j, on);
+        if (!on) return;
         const size_t ij = IJ(i, j);
         const size_t plane = d.n2;
         const uint32_t ij32 = IJ32(i, j);
-        // phase 3 on the now velocities, lines 1254-1259
+        // phase 3 on the now velocities, lines 1254-1259: zero where masked
         {
             const double cu = un_adv[ij] * r1_hu_n[ij], cv = vn_adv[ij] * r1_hv_n[ij];
             const double ubn = un_b[ij], vbn = vn_b[ij];
             const int u0 = d.kU.k0[ij], u1 = d.kU.k1[ij], v0 = d.kV.k0[ij], v1 = d.kV.k1[ij];
-    #pragma unroll 4
-            for (int k = 1; k <= d.jpk - 1; k++) {
-                T *uk = plane_ptr(un, plane, k), *vk = plane_ptr(vn, plane, k);
-                const double um = (k >= u0 && k <= u1) ? 1.0 : 0.0, vm = (k >= v0 && k <= v1) ? 1.0 : 0.0;
-                stp(uk, ij32, (T)(((double)ldp((const T *)uk, ij32) + cu - ubn) * um));
-                stp(vk, ij32, (T)(((double)ldp((const T *)vk, ij32) + cv - vbn) * vm));
+            const int ke = max(lu.end, lv.end);
+            constexpr int KB = 8;   // levels loaded together, ahead of the stores
+            for (int k0 = 1; k0 <= ke; k0 += KB) {
+                T uo[KB], vo[KB];
+    #pragma unroll
+                for (int q = 0; q < KB; q++) {
+                    const int k = min(k0 + q, ke);
+                    uo[q] = ldp((const T *)plane_ptr(un, plane, k), ij32);
+                    vo[q] = ldp((const T *)plane_ptr(vn, plane, k), ij32);
+                }
+    #pragma unroll
+                for (int q = 0; q < KB; q++) {
+                    const int k = k0 + q;
+                    if (k > ke) break;
+                    const double um = (k >= u0 && k <= u1) ? 1.0 : 0.0, vm = (k >= v0 && k <= v1) ? 1.0 : 0.0;
+                    stp(plane_ptr(un, plane, k), ij32, (T)(((double)uo[q] + cu - ubn) * um));
+                    stp(plane_ptr(vn, plane, k), ij32, (T)(((double)vo[q] + cv - vbn) * vm));
+                }
+            }
+            for (int k = ke + 1; k <= d.jpk - 1; k++) {
+                stp(plane_ptr(un, plane, k), ij32, T(0));
+                stp(plane_ptr(vn, plane, k), ij32, T(0));
             }
         }
         const bool inner = is_interior(d, i, j);
@@ -1001,12 +1103,12 @@ struct S_step_dyn2 {
             zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b, pu);
             zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b, pv);
         } else {
-            zdf_column(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b, zwd_s, pu);
-            zdf_column(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b, zwd_s, pv);
+            zdf_column<E3U>(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b, zwd_s, lu, pu);
+            zdf_column<E3U>(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b, zwd_s, lv, pv);
         }
     }
 };
-template <typename T, bool REG>
+template <typename T, bool REG, bool E3U>
 KERNEL_W(2) void k_step_dyn2(DevDomain d, double r2dt, double r1_2dt_b, const T *__restrict__ ub, const T *__restrict__ vb,
                         T *__restrict__ ua, T *__restrict__ va, T *__restrict__ un, T *__restrict__ vn,
                         const T *__restrict__ avm, const double *__restrict__ rCdU_bot,
@@ -1020,7 +1122,7 @@ KERNEL_W(2) void k_step_dyn2(DevDomain d, double r2dt, double r1_2dt_b, const T 
                         const double *__restrict__ vtau, const double *__restrict__ vtau_b,
                         double *__restrict__ zwd_s)
 {
-    S_step_dyn2<T, REG>::run(vb_hw(), d, r2dt, r1_2dt_b, ub, vb, ua, va, un, vn, avm, rCdU_bot, ua_b, va_b, ub_b, vb_b, un_adv, vn_adv, r1_hu_n, r1_hv_n, un_b, vn_b, su_s, sv_s, utau, utau_b, vtau, vtau_b, zwd_s);
+    S_step_dyn2<T, REG, E3U>::run(vb_hw(), d, r2dt, r1_2dt_b, ub, vb, ua, va, un, vn, avm, rCdU_bot, ua_b, va_b, ub_b, vb_b, un_adv, vn_adv, r1_hu_n, r1_hv_n, un_b, vn_b, su_s, sv_s, utau, utau_b, vtau, vtau_b, zwd_s);
 }
 
 template <typename T, int ADV, int KEG, int SCHEME>
@@ -1084,15 +1186,19 @@ int launch_step_dyn(int kt, double r2dt, const T *ub, const T *vb, const T *wn, 
     double *zwd = (double *)nh::scratch3(nh::S_ZWT);
     if constexpr (sizeof(T) == 4) {
         if (zdf_reg<T>(d)) {
-            LAUNCHB("step_dyn", (k_step_dyn2<T, true>), (S_step_dyn2<T, true>), g, d, r2dt, 1.0 / z2dt_bf, ub, vb, ua, va, un, vn, avm,
+            LAUNCHB("step_dyn", (k_step_dyn2<T, true, false>), (S_step_dyn2<T, true, false>), g, d, r2dt, 1.0 / z2dt_bf, ub, vb, ua, va, un, vn, avm,
                    st->rCdU_bot, st->ua_b, st->va_b, st->ub_b, st->vb_b, st->un_adv, st->vn_adv, st->r1_hu_n,
                    st->r1_hv_n, st->un_b, st->vn_b, w[2], w[3], st->utau, utau_b, st->vtau, vtau_b, zwd);
             return 0;
         }
     }
-    LAUNCHB("step_dyn", (k_step_dyn2<T, false>), (S_step_dyn2<T, false>), g, d, r2dt, 1.0 / z2dt_bf, ub, vb, ua, va, un, vn, avm,
-           st->rCdU_bot, st->ua_b, st->va_b, st->ub_b, st->vb_b, st->un_adv, st->vn_adv, st->r1_hu_n, st->r1_hv_n,
-           st->un_b, st->vn_b, w[2], w[3], st->utau, utau_b, st->vtau, vtau_b, zwd);
+#define DYN2_LAUNCH(U) \
+    LAUNCHB("step_dyn", (k_step_dyn2<T, false, U>), (S_step_dyn2<T, false, U>), g, d, r2dt, 1.0 / z2dt_bf, ub, vb, ua, va, un, vn, avm, \
+           st->rCdU_bot, st->ua_b, st->va_b, st->ub_b, st->vb_b, st->un_adv, st->vn_adv, st->r1_hu_n, st->r1_hv_n, \
+           st->un_b, st->vn_b, w[2], w[3], st->utau, utau_b, st->vtau, vtau_b, zwd)
+    if (d.e3_sij == 0) DYN2_LAUNCH(true);
+    else DYN2_LAUNCH(false);
+#undef DYN2_LAUNCH
     return 0;
 }
 template int launch_step_dyn<double>(int, double, const double *, const double *, const double *, const double *,

@@ -1079,8 +1079,8 @@ enum { QC = 0, QW = 1, QE = 2, QS = 3, QN = 4 };
 // neighbouring workgroups instead (the tracer is the lowest digit of the
 // XCD-ordered tile index, so the workgroups of one tile run on one XCD at
 // the same time and share the coefficient loads in its L2)
-// E3U: horizontally uniform scale factors, read by level where used (scalar
-// loads) instead of with the window
+// E3U: horizontally uniform scale factors, one value per level read where used
+// instead of five with the window
 template <typename T, int MODE, int NT, int TSPLIT, bool E3U>
 struct S_tra_ldf_iso {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
@@ -1390,21 +1390,32 @@ template int launch_tra_ldf_iso<float>(int, double, const float *, const float *
 // the upper diagonal and, segment by segment from those checkpoints, the
 // other pivots, with the operations of the forward sweep.
 // ---------------------------------------------------------------------------
-// NT tracers share the matrix.  The forward sweep is unrolled by four with
-// the pointers declared non-aliasing, so the loads of four levels are issued
-// together ahead of the serial FP64 recurrence; the backward sweep loads a
-// segment's operands together.
-template <typename T, int NT>
+// NT tracers share the matrix.  Both sweeps work on segments of ZDF_SEG levels,
+// the next segment's operands in flight while the serial FP64 recurrence runs
+// through the current one: a load issued after a store to pta waits for it
+// (the compiler cannot tell the two levels apart), so they are read ahead of it.
+//
+// The sweeps run over the levels 1..kend down to the wave's deepest wet one:
+// below, tmask sets every solved value to zero, so the row at kend has nothing
+// to substitute, and the dry levels are only stored.  zwi(k) is zws(k-1), the
+// same quotient.  The kernel is bound by HBM (5.7 TB/s over every level):
+// 1024x1024x75 FP32, 47 % of the cells dry:
+// 983 -> 792 us (4.9 TB/s); 512x512x75 FP64: 373 -> 296; 32x22x31 FP64: 34 -> 27.
+template <typename T, int NT, bool E3U>
 struct S_tra_zdf {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double p2dt, const T * __restrict__ ptb, T * __restrict__ pta, int jn0, const T * __restrict__ src, int l_ldfslp, const T * __restrict__ add, double * __restrict__ zwt, int clamp_jn)
     {
         THREAD_IJ_V(vb_, 2, 2);
-        if (i > d.jpi - 1 || j > d.jpj - 1) return;
-        const uint32_t ij = IJ32(i, j);
+        const bool on = i <= d.jpi - 1 && j <= d.jpj - 1;
+        const int jpk = d.jpk;
+        const uint32_t ij = on ? IJ32(i, j) : 0u;
+        const uint32_t tw = on ? d.ktu[ij] : 1u;
+        const int t0 = (int)(tw & 255u), t1 = (int)((tw >> 8) & 255u);
+        const int kend = min(wave_max(t1), jpk - 1);
+        if (!on) return;
         const size_t plane = d.n2, n3 = d.n3;
         const Metrics<T> &m = met<T>(d);
-        const int jpk = d.jpk;
         const T *tb[NT];
         T *ta[NT];
     #pragma unroll
@@ -1412,136 +1423,158 @@ struct S_tra_zdf {
             tb[n] = ptb + (size_t)(jn0 + n) * n3;
             ta[n] = pta + (size_t)(jn0 + n) * n3;
         }
-        // zwt(k) of trazdf.F90:153-176: avt/avs, 0 at the surface, plus the
-        // iso-neutral contribution on 2..jpkm1.  Both loads are unconditional
-        // (levels 1 <= k <= jpk, the second clamped to jpkm1), so the march can
-        // keep several levels of loads in flight; the conditions only select.
-        const T *addp = l_ldfslp ? add : src;
-        auto coef = [&](int k) -> double {
-            const double sv = (double)ldp(plane_ptr(src, plane, k), ij);
-            const double av = (double)ldp(plane_ptr(addp, plane, k <= jpk - 1 ? k : jpk - 1), ij);
-            double c = sv;
-            if (l_ldfslp && k <= jpk - 1) c = c + av;
-            return k <= 1 ? 0.0 : c;
-        };
-        // only checkpoint pivots (every ZDF_SEG-th level) are stored; the back
-        // substitution recomputes the others segment by segment
-        double prev[NT];
-        double zws_prev, zwt_prev, zc_k;
-        // k = 1 (zwi = 0)
-        {
-            const double zc_kp1 = coef(2);
-            const double e3t = (double)E3(m.e3t, ij, 1);
-            const double zwi = -(p2dt * 0.0 / (double)E3(m.e3w, ij, 1));
-            const double zws = -(p2dt * zc_kp1 / (double)E3(m.e3w, ij, 2));
-            const double zwd = e3t - zwi - zws;
+        if (kend >= 1) {
+            // zwt(k) of trazdf.F90:153-176: avt/avs, 0 at the surface, plus the
+            // iso-neutral contribution on 2..jpkm1.  Both loads are unconditional
+            // (levels 1 <= k <= jpk, the second clamped to jpkm1), so the march can
+            // keep several levels of loads in flight; the conditions only select.
+            const T *addp = l_ldfslp ? add : src;
+            const T *const pe3t = m.e3t, *const pe3w = m.e3w;
+            // w-level k <= jpk.  e3w, e3t: a vector load with the level's other
+            // operands, or, horizontally uniform, a scalar load where used
+            auto ld_w = [&](int k, T &sv_, T &av_, T &e3w_) {
+                sv_ = ldp(plane_ptr(src, plane, k), ij);
+                av_ = ldp(plane_ptr(addp, plane, k <= jpk - 1 ? k : jpk - 1), ij);
+                if constexpr (!E3U) e3w_ = E3(m.e3w, ij, k);
+            };
+            auto e3t_of = [&](int k, T v) -> double { return (double)(E3U ? uld(pe3t, k - 1) : v); };
+            auto off = [&](int k, T sv_, T av_, T e3w_) -> double {   // -p2dt zwt / e3w at w-level k
+                double c = (double)sv_;
+                if (l_ldfslp && k <= jpk - 1) c = c + (double)av_;
+                return -(p2dt * (k <= 1 ? 0.0 : c) / (double)(E3U ? uld(pe3w, k - 1) : e3w_));
+            };
+            // the operands of ZDF_SEG levels from k0 and of the w-levels under
+            // them (levels past kend load kend's and are not used)
+            struct Seg {
+                T b[NT][ZDF_SEG], a[NT][ZDF_SEG], sv[ZDF_SEG], av[ZDF_SEG], e3t[ZDF_SEG], e3w[ZDF_SEG];
+            };
+            auto fetch = [&](int k0, Seg &g, bool with_tb) {
     #pragma unroll
-            for (int n = 0; n < NT; n++) {
-                const double v = e3t * (double)ldp(tb[n], ij) + p2dt * e3t * (double)ldp((const T *)ta[n], ij);
-                prev[n] = v;
-                stp(ta[n], ij, (T)v);
-            }
-            zws_prev = zws;
-            zwt_prev = zwd;
-            zc_k = zc_kp1;
-        }
-    #pragma unroll 4
-        for (int k = 2; k <= jpk - 1; k++) {
-            const double zc_kp1 = coef(k + 1);
-            const double e3t = (double)E3(m.e3t, ij, k);
-            const double zwi = -(p2dt * zc_k / (double)E3(m.e3w, ij, k));
-            const double zws = -(p2dt * zc_kp1 / (double)E3(m.e3w, ij, k + 1));
-            const double zwd = e3t - zwi - zws;
-            const double zwt_k = zwd - zwi * zws_prev / zwt_prev;
-            if (k % ZDF_SEG == 0 && k <= jpk - 2) stp(plane_ptr(zwt, plane, k), ij, zwt_k);
-    #pragma unroll
-            for (int n = 0; n < NT; n++) {
-                const double zrhs = e3t * (double)ldp(plane_ptr(tb[n], plane, k), ij) +
-                                    p2dt * e3t * (double)ldp((const T *)plane_ptr(ta[n], plane, k), ij);
-                const double v = zrhs - zwi / zwt_prev * prev[n];
-                prev[n] = v;
-                stp(plane_ptr(ta[n], plane, k), ij, (T)v);
-            }
-            zws_prev = zws;
-            zwt_prev = zwt_k;
-            zc_k = zc_kp1;
-        }
-        // back substitution, the result is the after tracer
-        {
-            const double tm = TMASK(double, i, j, jpk - 1);
-    #pragma unroll
-            for (int n = 0; n < NT; n++) {
-                const double v = prev[n] / zwt_prev * tm;
-                prev[n] = v;
-                T out = (T)v;
-                if (jn0 + n == clamp_jn && out < T(0)) out = T(0.1);
-                stp(plane_ptr(ta[n], plane, jpk - 1), ij, out);
-            }
-        }
-        const int t0 = d.kT.k0[ij], t1 = d.kT.k1[ij];
-        const int kl = jpk - 2;
-        // each segment's operands are loaded together, from levels within the
-        // arrays (clamped to kl; the values of levels past kl are not used)
-        auto ld_w = [&](int k, T &sv_, T &av_, T &e3w_) {   // w-level k <= jpk
-            sv_ = ldp(plane_ptr(src, plane, k), ij);
-            av_ = ldp(plane_ptr(addp, plane, k <= jpk - 1 ? k : jpk - 1), ij);
-            e3w_ = E3(m.e3w, ij, k);
-        };
-        auto coef_v = [&](int k, T sv_, T av_) -> double {
-            double c = (double)sv_;
-            if (l_ldfslp && k <= jpk - 1) c = c + (double)av_;
-            return k <= 1 ? 0.0 : c;
-        };
-        for (int s = (kl + ZDF_SEG - 1) / ZDF_SEG - 1; s >= 0; s--) {
-            const int k0 = s * ZDF_SEG + 1;
-            T e3t_[ZDF_SEG], sv_[ZDF_SEG], av_[ZDF_SEG], e3w_[ZDF_SEG], ta_[NT][ZDF_SEG];   // level k, w-level k + 1
-    #pragma unroll
-            for (int q = 0; q < ZDF_SEG; q++) {
-                const int k = k0 + q <= kl ? k0 + q : kl;
-                e3t_[q] = E3(m.e3t, ij, k);
-                ld_w(k + 1, sv_[q], av_[q], e3w_[q]);
-    #pragma unroll
-                for (int n = 0; n < NT; n++) ta_[n][q] = ldp((const T *)plane_ptr(ta[n], plane, k), ij);
-            }
-            T svp, avp, e3wp;   // w-level k0
-            ld_w(k0, svp, avp, e3wp);
-            double piv[ZDF_SEG], zsv[ZDF_SEG];
-            double zc = coef_v(k0, svp, avp);
-            double zwt_p = 1.0, zws_p = 0.0;
-            if (k0 > 1) {
-                zwt_p = ldp((const double *)plane_ptr(zwt, plane, k0 - 1), ij);
-                zws_p = -(p2dt * zc / (double)e3wp);
-            }
-    #pragma unroll
-            for (int q = 0; q < ZDF_SEG; q++) {
-                const int k = k0 + q;
-                const double zc_kp1 = coef_v(k + 1, sv_[q], av_[q]);
-                const double e3t = (double)e3t_[q];
-                const double zwi = -(p2dt * zc / (double)(q == 0 ? e3wp : e3w_[q > 0 ? q - 1 : 0]));
-                const double zws = -(p2dt * zc_kp1 / (double)e3w_[q]);
-                const double zwd = e3t - zwi - zws;
-                piv[q] = k == 1 ? zwd : zwd - zwi * zws_p / zwt_p;
-                zsv[q] = zws;
-                zws_p = zws;
-                zwt_p = piv[q];
-                zc = zc_kp1;
-            }
-    #pragma unroll
-            for (int q = ZDF_SEG - 1; q >= 0; q--) {
-                const int k = k0 + q;
-                if (k <= kl) {
-                    const double tm = (k >= t0 && k <= t1) ? 1.0 : 0.0;
+                for (int q = 0; q < ZDF_SEG; q++) {
+                    const int k = min(k0 + q, kend);
+                    if constexpr (!E3U) g.e3t[q] = E3(m.e3t, ij, k);
+                    ld_w(k + 1, g.sv[q], g.av[q], g.e3w[q]);
     #pragma unroll
                     for (int n = 0; n < NT; n++) {
-                        const double v = ((double)ta_[n][q] - zsv[q] * prev[n]) / piv[q] * tm;
-                        prev[n] = v;
-                        T out = (T)v;
-                        if (jn0 + n == clamp_jn && out < T(0)) out = T(0.1);
-                        stp(plane_ptr(ta[n], plane, k), ij, out);
+                        g.a[n][q] = ldp((const T *)plane_ptr(ta[n], plane, k), ij);
+                        if (with_tb) g.b[n][q] = ldp(plane_ptr(tb[n], plane, k), ij);
                     }
                 }
+            };
+            // only checkpoint pivots (every ZDF_SEG-th level) are stored; the back
+            // substitution recomputes the others segment by segment
+            double prev[NT];
+            double zws_prev, zwt_prev;
+            Seg cur, nxt;
+            fetch(2, cur, true);
+            // k = 1 (zwi = 0)
+            {
+                T sv, av, e3w = T(1), e1 = T(1), e3 = T(1);
+                ld_w(2, sv, av, e3w);
+                if constexpr (!E3U) { e1 = E3(m.e3w, ij, 1); e3 = E3(m.e3t, ij, 1); }
+                const double e3t = e3t_of(1, e3);
+                const double zwi = -(p2dt * 0.0 / (double)(E3U ? uld(pe3w, 0) : e1));
+                const double zws = off(2, sv, av, e3w);
+                zwt_prev = e3t - zwi - zws;
+                zws_prev = zws;
+    #pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    const double v = e3t * (double)ldp(tb[n], ij) + p2dt * e3t * (double)ldp((const T *)ta[n], ij);
+                    prev[n] = v;
+                    stp(ta[n], ij, (T)v);
+                }
+            }
+            for (int k0 = 2; k0 <= kend; k0 += ZDF_SEG) {
+                fetch(k0 + ZDF_SEG, nxt, true);
+    #pragma unroll
+                for (int q = 0; q < ZDF_SEG; q++) {
+                    const int k = k0 + q;
+                    if (k > kend) break;
+                    const double e3t = e3t_of(k, cur.e3t[q]);
+                    const double zwi = zws_prev;
+                    const double zws = off(k + 1, cur.sv[q], cur.av[q], cur.e3w[q]);
+                    const double zwd = e3t - zwi - zws;
+                    const double zwt_k = zwd - zwi * zws_prev / zwt_prev;
+                    if (k % ZDF_SEG == 0) stp(plane_ptr(zwt, plane, k), ij, zwt_k);
+    #pragma unroll
+                    for (int n = 0; n < NT; n++) {
+                        const double zrhs = e3t * (double)cur.b[n][q] + p2dt * e3t * (double)cur.a[n][q];
+                        const double v = zrhs - zwi / zwt_prev * prev[n];
+                        prev[n] = v;
+                        stp(plane_ptr(ta[n], plane, k), ij, (T)v);
+                    }
+                    zws_prev = zws;
+                    zwt_prev = zwt_k;
+                }
+                cur = nxt;
+            }
+            // back substitution, the result is the after tracer.  The last row of
+            // the whole column divides the value in hand, any other the one rounded
+            // to storage, as if it had been stored and the zero below substituted
+            const int kl = kend - 1;
+            int s = (kl + ZDF_SEG - 1) / ZDF_SEG - 1;
+            T svp, avp, e3wp = T(1);   // w-level k0 of the segment, and its checkpoint pivot
+            double ckp = 1.0;
+            auto fetch_top = [&](int k0) {
+                ld_w(k0, svp, avp, e3wp);
+                if (k0 > 1) ckp = ldp((const double *)plane_ptr(zwt, plane, k0 - 1), ij);
+            };
+            if (s >= 0) {
+                fetch(s * ZDF_SEG + 1, cur, false);
+                fetch_top(s * ZDF_SEG + 1);
+            }
+            {
+                const double tm = (kend >= t0 && kend <= t1) ? 1.0 : 0.0;
+    #pragma unroll
+                for (int n = 0; n < NT; n++) {
+                    const double v = (kend == jpk - 1 ? prev[n] : (double)(T)prev[n]) / zwt_prev * tm;
+                    prev[n] = v;
+                    T out = (T)v;
+                    if (jn0 + n == clamp_jn && out < T(0)) out = T(0.1);
+                    stp(plane_ptr(ta[n], plane, kend), ij, out);
+                }
+            }
+            for (; s >= 0; s--) {
+                const int k0 = s * ZDF_SEG + 1;
+                double piv[ZDF_SEG], zsv[ZDF_SEG];
+                double zwt_p = ckp, zws_p = off(k0, svp, avp, e3wp);
+                if (s > 0) {
+                    fetch(k0 - ZDF_SEG, nxt, false);
+                    fetch_top(k0 - ZDF_SEG);
+                }
+    #pragma unroll
+                for (int q = 0; q < ZDF_SEG; q++) {
+                    const int k = k0 + q;
+                    const double e3t = e3t_of(k, cur.e3t[q]);
+                    const double zwi = zws_p;
+                    const double zws = off(k + 1, cur.sv[q], cur.av[q], cur.e3w[q]);
+                    const double zwd = e3t - zwi - zws;
+                    piv[q] = k == 1 ? zwd : zwd - zwi * zws_p / zwt_p;
+                    zsv[q] = zws;
+                    zws_p = zws;
+                    zwt_p = piv[q];
+                }
+    #pragma unroll
+                for (int q = ZDF_SEG - 1; q >= 0; q--) {
+                    const int k = k0 + q;
+                    if (k <= kl) {
+                        const double tm = (k >= t0 && k <= t1) ? 1.0 : 0.0;
+    #pragma unroll
+                        for (int n = 0; n < NT; n++) {
+                            const double v = ((double)cur.a[n][q] - zsv[q] * prev[n]) / piv[q] * tm;
+                            prev[n] = v;
+                            T out = (T)v;
+                            if (jn0 + n == clamp_jn && out < T(0)) out = T(0.1);
+                            stp(plane_ptr(ta[n], plane, k), ij, out);
+                        }
+                    }
+                }
+                cur = nxt;
             }
         }
+        for (int k = kend + 1; k <= jpk - 1; k++)
+    #pragma unroll
+            for (int n = 0; n < NT; n++) stp(plane_ptr(ta[n], plane, k), ij, T(0));
     #pragma unroll
         for (int n = 0; n < NT; n++) {
             if (jn0 + n == clamp_jn) {
@@ -1551,12 +1584,12 @@ struct S_tra_zdf {
         }
     }
 };
-template <typename T, int NT>
+template <typename T, int NT, bool E3U>
 KERNEL void k_tra_zdf(DevDomain d, double p2dt, const T * __restrict__ ptb, T * __restrict__ pta, int jn0,
                       const T * __restrict__ src, int l_ldfslp, const T * __restrict__ add,
                       double * __restrict__ zwt, int clamp_jn)
 {
-    S_tra_zdf<T, NT>::run(vb_hw(), d, p2dt, ptb, pta, jn0, src, l_ldfslp, add, zwt, clamp_jn);
+    S_tra_zdf<T, NT, E3U>::run(vb_hw(), d, p2dt, ptb, pta, jn0, src, l_ldfslp, add, zwt, clamp_jn);
 }
 
 // FP32 storage with at most KMAX - 1 solved levels: the same solve with the
@@ -1756,7 +1789,8 @@ static int zdf_group(const char *name, const DevDomain &d, Grid2 g, double p2dt,
             return 0;
         }
     }
-    LAUNCHB(name, (k_tra_zdf<T, NT>), (S_tra_zdf<T, NT>), g, d, p2dt, ptb, pta, jn, src, l_ldfslp, add, zwt, clamp_jn);
+    if (d.e3_sij == 0) LAUNCHB(name, (k_tra_zdf<T, NT, true>), (S_tra_zdf<T, NT, true>), g, d, p2dt, ptb, pta, jn, src, l_ldfslp, add, zwt, clamp_jn);
+    else LAUNCHB(name, (k_tra_zdf<T, NT, false>), (S_tra_zdf<T, NT, false>), g, d, p2dt, ptb, pta, jn, src, l_ldfslp, add, zwt, clamp_jn);
     return 0;
 }
 
