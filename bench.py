@@ -642,13 +642,13 @@ def kernel_times(h):
         "tra_adv_fct": ["k_fct_fused", "k_fct_cpt_fwd", "k_fct_h", "k_fct_hh", "k_fct_v", "k_fct_vz_reg", "k_fct_lim", "k_fct_vlim",
                         "k_fct_beta", "k_fct_final", "k_fct_low", "k_fct_ad"],
         "tra_ldf_iso": ["k_ldf_iso_coef", "k_tra_ldf_iso", "k_fill3"], "tra_zdf": ["k_tra_zdf", "k_tra_zdf_reg", "k_clamp_ring"],
-        "lbc_lnk": ["k_lbc"],
+        "lbc_lnk": ["k_lbc", "k_lbc4"],
         "step_dyn": ["k_step_dyn1", "k_step_dyn2"],
         "step_tra": ["k_fct_fused", "k_fct_cpt_fwd", "k_fct_h", "k_fct_hh", "k_fct_v", "k_fct_vz_reg", "k_fct_lim", "k_fct_vlim",
                      "k_fct_beta", "k_fct_final", "k_zero_ring", "k_tra_zdf", "k_tra_zdf_reg"],
         "div_hor": ["k_div_hor"], "ssh_nxt": ["k_ssh_nxt"], "wzv": ["k_wzv"], "ssh_swp": ["k_ssh_swp"],
         "tra_nxt": ["k_tra_nxt"], "dyn_nxt": ["k_dyn_nxt1", "k_dyn_nxt2"],
-        "ldf_slp": ["k_slp_mxl", "k_slp_uv_raw", "k_slp_uv_filt", "k_slp_w_raw", "k_slp_w_filt"],
+        "ldf_slp": ["k_slp_mxl", "k_slp"],
     }
     for n in names:
         out[n] = h.timing_get(n)

@@ -86,5 +86,35 @@ int launch_lbc(T *p, int nk, char nat, T pval)
     LAUNCHB("lbc_lnk", k_lbc<T>, (S_lbc<T>), g, d, p, nk, nat, pval);
     return 0;
 }
+
+// the fill of four arrays of nk levels in one launch (grid.y: the array), for
+// the point types whose rule is the same (T, U, V, W; zero on closed sides): a
+// launch of one array is too small to fill the chip and costs about 5 us
+template <typename T>
+struct S_lbc4 {
+    static constexpr int NTHR = NH_BLOCK, WAVES = 1;
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, T *__restrict__ p0, T *__restrict__ p1, T *__restrict__ p2, T *__restrict__ p3, int nk)
+    {
+        T *p = vb_.y == 0 ? p0 : vb_.y == 1 ? p1 : vb_.y == 2 ? p2 : p3;
+        S_lbc<T>::run(vb_, d, p, nk, 'T', T(0));
+    }
+};
+template <typename T>
+KERNEL void k_lbc4(DevDomain d, T *__restrict__ p0, T *__restrict__ p1, T *__restrict__ p2, T *__restrict__ p3, int nk)
+{
+    S_lbc4<T>::run(vb_hw(), d, p0, p1, p2, p3, nk);
+}
+template <typename T>
+int launch_lbc4(T *p0, T *p1, T *p2, T *p3, int nk)
+{
+    const DevDomain &d = nh::dom();
+    Grid2 g;
+    g.grid = dim3((unsigned)nk, 4, 1);
+    g.block = dim3(NH_BLOCK, 1, 1);
+    LAUNCHB("lbc_lnk", k_lbc4<T>, (S_lbc4<T>), g, d, p0, p1, p2, p3, nk);
+    return 0;
+}
+template int launch_lbc4<double>(double *, double *, double *, double *, int);
+template int launch_lbc4<float>(float *, float *, float *, float *, int);
 template int launch_lbc<double>(double *, int, char, double);
 template int launch_lbc<float>(float *, int, char, float);

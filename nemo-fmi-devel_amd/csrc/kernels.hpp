@@ -7,6 +7,8 @@ int launch_dom_msk(double *tmask, double *umask, double *vmask, double *fmask, d
                    double *wvmask, double *ssmask, double *ssumask, double *ssvmask);
 template <typename T> int launch_lbc(T *p, int nk, char nat, T pval);
 
+template <typename T> int launch_lbc4(T *p0, T *p1, T *p2, T *p3, int nk);   // T, U, V or W points, zero on closed sides
+
 template <typename T> int launch_tra_adv_trp(const T *un, const T *vn, const T *wn, T *zun, T *zvn, T *zwn);
 template <typename T>
 int launch_tra_adv_fct(double p2dt, const T *pun, const T *pvn, const T *pwn, const T *ptb, const T *ptn, T *pta,

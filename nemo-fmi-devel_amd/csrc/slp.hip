@@ -7,13 +7,11 @@
 // reference's operation order, so the FP64 form reproduces it bit for bit.
 //
 // The reference builds the unfiltered slopes in work arrays, applies
-// lbc_lnk to them, filters and applies lbc_lnk again.  Here one kernel per
-// level builds the unfiltered slopes of a tile and its halo in LDS (a halo
+// lbc_lnk to them, filters and applies lbc_lnk again.  Here one kernel marches
+// down a region of columns: it builds the unfiltered slopes of a level in LDS (a
 // point on the ring evaluates the interior formula at its lbc source, or is
 // zero on a closed boundary, which is what lbc_lnk gives), filters them and
-// writes the interior; the final lbc_lnk fills the output's ring.  The
-// horizontal and vertical density gradients (zgru, zgrv, zdzr) are
-// recomputed from prd and pn2 where used.
+// writes the interior; the final lbc_lnk fills the output's ring.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -66,9 +64,22 @@ KERNEL void k_zdf_mxl(DevDomain d, const T *__restrict__ rn2b, const T *__restri
     const int ikt = d.mbkt[ij];
     double h = 0.;
     int nm = nlb10;
-    for (int k = nlb10; k <= d.jpk - 1; k++) {
-        h = h + max2((double)A3(rn2b, i, j, k), 0.) * E3(d.md.e3w, ij, k);
-        if (h < zN2_c) nm = (k < ikt ? k : ikt) + 1;
+    // h never falls, and nm stays at ikt + 1 from there on: the march ends where
+    // every column of the wave has passed one of the two (the column read to the
+    // bottom: 33 us at 512x509x75 in FP32, 11 us at 203x157x31 in FP64)
+    constexpr int KB = 8;
+    for (int k0 = nlb10; k0 <= d.jpk - 1; k0 += KB) {
+        T n2[KB];
+#pragma unroll
+        for (int q = 0; q < KB; q++) n2[q] = A3(rn2b, i, j, min(k0 + q, d.jpk - 1));
+#pragma unroll
+        for (int q = 0; q < KB; q++) {
+            const int k = k0 + q;
+            if (k > d.jpk - 1) break;
+            h = h + max2((double)n2[q], 0.) * E3(d.md.e3w, ij, k);
+            if (h < zN2_c) nm = (k < ikt ? k : ikt) + 1;
+        }
+        if (!__any(h < zN2_c && k0 + KB - 1 < ikt)) break;
     }
     const double ss = d.ssmask[ij];
     nmln[ij] = nm;
@@ -127,187 +138,206 @@ KERNEL void k_slp_mxl(DevDomain d, SlpIn<T> in, const int32_t *__restrict__ nmln
 }
 
 // ---------------------------------------------------------------------------
-// I. unfiltered u/v slopes at the interior point (si, sj), level k, lines
-// 197-219 (zwz, zww).  P(i, j, kk) and N(i, j, kk) give prd and pn2 at the
-// levels used (prd: k, k-1; pn2: k, k+1), from global memory or from LDS.
+// The four slopes, marched down SLP_RX x SLP_RY columns, one per thread.  At each
+// level a thread shares its prd and zdzr with its neighbours through LDS, forms
+// the unfiltered slopes (zwz, zww of parts I and II) of its column from them
+// and the gradients it kept from the level above, shares those, and, inside
+// the tile (the region less two points on each side), applies the Shapiro
+// filters and tapers of lines 232-271 and 316-356.  A region point on the
+// domain's ring takes zero on a closed side, its lbc source's value on a cyclic
+// one (the reference's lbc_lnk of zwz/zww, lines 231 and 315): there the region
+// runs on past the domain's last column to its first, both ring columns
+// included, so the source is two points away across the seam and the region
+// has two more points on each side.  The output's ring is the final lbc_lnk
+// (line 361), a separate pass.
+//
+// The terms of the mixed layer (a division and the depths) are formed only at
+// levels where a column of the wave is in it, -7e3/e3 once per level where the
+// scale factors are horizontally uniform, and levels below the region's deepest
+// column are stored as the zeros the masks give.
+//
+// Bound by FP64 vector instructions (six divisions per point).  One level of
+// a 64x4 tile per workgroup, staged in LDS with its two-point halo, ran 1020
+// instructions per cell: 512x509x75 FP32 790 -> 330 us, 203x157x31 cyclic FP64
+// 74 -> 39 us.
 // ---------------------------------------------------------------------------
-template <class P, class N>
-__device__ __forceinline__ double a_dzr(const DevDomain &d, const P &prd, const N &pn2, int i, int j, int k)
-{
-    const double zm1_g = -1.0 / d.grav;
-    return zm1_g * (prd(i, j, k) + 1.) * (pn2(i, j, k) + pn2(i, j, k + 1)) * (1. - 0.5 * TMASK(double, i, j, k + 1));
-}
-template <class P>
-__device__ __forceinline__ double a_gru(const DevDomain &d, const P &prd, int i, int j, int k)
-{
-    return UMASK(double, i, j, k) * (prd(i + 1, j, k) - prd(i, j, k));
-}
-template <class P>
-__device__ __forceinline__ double a_grv(const DevDomain &d, const P &prd, int i, int j, int k)
-{
-    return VMASK(double, i, j, k) * (prd(i, j + 1, k) - prd(i, j, k));
-}
-
-template <typename T, class P, class N>
-__device__ __forceinline__ void raw_uv(const DevDomain &d, const P &prd, const N &pn2, const T *gdept,
-                                       const int32_t *nmln, const double *zsu, const double *zsv, double z1_slpmax,
-                                       int si, int sj, int k, double &zwz, double &zww)
-{
-    const Metrics<double> &m = d.md;
-    const uint32_t ij = IJ32(si, sj);
-    const double zau = a_gru(d, prd, si, sj, k) * m.r1_e1u[ij];
-    const double zav = a_grv(d, prd, si, sj, k) * m.r1_e2v[ij];
-    const double dc = a_dzr(d, prd, pn2, si, sj, k);
-    double zbu = 0.5 * (dc + a_dzr(d, prd, pn2, si + 1, sj, k));
-    double zbv = 0.5 * (dc + a_dzr(d, prd, pn2, si, sj + 1, k));
-    zbu = min3(zbu, -z1_slpmax * fabs(zau), -7.e+3 / E3(m.e3u, ij, k) * fabs(zau));
-    zbv = min3(zbv, -z1_slpmax * fabs(zav), -7.e+3 / E3(m.e3v, ij, k) * fabs(zav));
-    const double oc = oml(nmln, ij, k);
-    const double zfi = max2(oc, oml(nmln, ij + 1, k));
-    const double zfj = max2(oc, oml(nmln, ij + (uint32_t)d.jpi, k));
-    const double gc = (double)A3(gdept, si, sj, k);
-    const double zdepu = 0.5 * ((gc + (double)A3(gdept, si + 1, sj, k)) - E3(m.e3u, ij, d.miku[ij]));
-    const double zdepv = 0.5 * ((gc + (double)A3(gdept, si, sj + 1, k)) - E3(m.e3v, ij, d.mikv[ij]));
-    zwz = ((1. - zfi) * zau / (zbu - ZEPS) + zfi * zdepu * zsu[ij]) * UMASK(double, si, sj, k);
-    zww = ((1. - zfj) * zav / (zbv - ZEPS) + zfj * zdepv * zsv[ij]) * VMASK(double, si, sj, k);
-}
-
-// II. unfiltered w slopes at the interior point (si, sj), level k, lines 277-304
-template <typename T, class P, class N>
-__device__ __forceinline__ void raw_w(const DevDomain &d, const P &prd, const N &pn2, const T *gdepw,
-                                      const int32_t *nmln, const double *hmlp, const double *wiml,
-                                      const double *wjml, int si, int sj, int k, double &zwz, double &zww)
-{
-    const Metrics<double> &m = d.md;
-    const uint32_t ij = IJ32(si, sj);
-    const double zm1_2g = -0.5 / d.grav;
-    const double zbw = zm1_2g * pn2(si, sj, k) * (prd(si, sj, k) + prd(si, sj, k - 1) + 2.);
-    const double zci = max2(UMASK(double, si - 1, sj, k) + UMASK(double, si, sj, k) + UMASK(double, si - 1, sj, k - 1) +
-                                UMASK(double, si, sj, k - 1),
-                            ZEPS) * m.e1t[ij];
-    const double zcj = max2(VMASK(double, si, sj - 1, k) + VMASK(double, si, sj, k - 1) +
-                                VMASK(double, si, sj - 1, k - 1) + VMASK(double, si, sj, k),
-                            ZEPS) * m.e2t[ij];
-    const double wm = WMASK(double, si, sj, k);
-    const double zai = (a_gru(d, prd, si - 1, sj, k) + a_gru(d, prd, si, sj, k - 1) +
-                        a_gru(d, prd, si - 1, sj, k - 1) + a_gru(d, prd, si, sj, k)) / zci * wm;
-    const double zaj = (a_grv(d, prd, si, sj - 1, k) + a_grv(d, prd, si, sj, k - 1) +
-                        a_grv(d, prd, si, sj - 1, k - 1) + a_grv(d, prd, si, sj, k)) / zcj * wm;
-    const double e3w = E3(m.e3w, ij, k);
-    const double zbi = min3(zbw, -100. * fabs(zai), -7.e+3 / e3w * fabs(zai));
-    const double zbj = min3(zbw, -100. * fabs(zaj), -7.e+3 / e3w * fabs(zaj));
-    const double zfk = max2(oml(nmln, ij, k), oml(nmln, ij, k - 1));
-    const int ikt = d.mikt[ij];
-    const double gwt = (double)A3(gdepw, si, sj, ikt);
-    const double zck = ((double)A3(gdepw, si, sj, k) - gwt) / max2(hmlp[ij] - gwt, 10.);
-    zwz = (zai / (zbi - ZEPS) * (1. - zfk) + zck * wiml[ij] * zfk) * wm;
-    zww = (zaj / (zbj - ZEPS) * (1. - zfk) + zck * wjml[ij] * zfk) * wm;
-}
-
-// prd or pn2 read from global memory
+#define SLP_RX 32
+#define SLP_RY 16
+#define SLP_MAXKB 24
 template <typename T>
-struct GlobalField {
-    const T *p;
-    const DevDomain &d;
-    __device__ __forceinline__ double operator()(int i, int j, int k) const { return (double)A3(p, i, j, k); }
-};
-
-// ---------------------------------------------------------------------------
-// one level of a SLP_TX x SLP_TY tile: the four unfiltered slopes of the
-// tile and a one-point halo in LDS (a halo point on the domain's ring takes
-// its lbc source's value, or zero on a closed side: the reference's
-// lbc_lnk of zwz/zww, lines 231 and 315), then the Shapiro filters and
-// tapers of lines 232-271 and 316-356 for the tile's interior points.  The
-// output's ring is the final lbc_lnk (line 361), a separate pass.
-// ---------------------------------------------------------------------------
-#define SLP_TX 64
-#define SLP_TY 4
-template <typename T>
-__global__ __launch_bounds__(SLP_TX * SLP_TY) void k_slp(DevDomain d, SlpIn<T> in, const T *__restrict__ gdept,
-                                                          const T *__restrict__ gdepw,
-                                                          const int32_t *__restrict__ nmln,
-                                                          const double *__restrict__ zsu,
-                                                          const double *__restrict__ zsv,
-                                                          const double *__restrict__ hmlp,
-                                                          const double *__restrict__ wiml,
-                                                          const double *__restrict__ wjml, double z1_slpmax,
-                                                          T *__restrict__ uslp, T *__restrict__ vslp,
-                                                          T *__restrict__ wslpi, T *__restrict__ wslpj)
+__global__ __launch_bounds__(SLP_RX * SLP_RY, 4) void k_slp(DevDomain d, SlpIn<T> in, const T *__restrict__ gdept,
+                                                             const T *__restrict__ gdepw,
+                                                             const int32_t *__restrict__ nmln,
+                                                             const double *__restrict__ zsu,
+                                                             const double *__restrict__ zsv,
+                                                             const double *__restrict__ hmlp,
+                                                             const double *__restrict__ wiml,
+                                                             const double *__restrict__ wjml, double z1_slpmax, int kb,
+                                                             T *__restrict__ uslp, T *__restrict__ vslp,
+                                                             T *__restrict__ wslpi, T *__restrict__ wslpj)
 {
-    constexpr int LX = SLP_TX + 2, LY = SLP_TY + 2;      // the slopes: tile + 1
-    constexpr int SX = SLP_TX + 4, SY = SLP_TY + 4;      // prd, pn2: tile + 2
-    __shared__ double su[LY][LX], sv[LY][LX], swi[LY][LX], swj[LY][LX];
-    __shared__ double p0[SY][SX], pm[SY][SX], n0[SY][SX], np[SY][SX];
-    const int k = (int)blockIdx.z + 2;
-    const int ib = 2 + (int)blockIdx.x * SLP_TX, jb = 2 + (int)blockIdx.y * SLP_TY;
-    const int tid = (int)(threadIdx.y * SLP_TX + threadIdx.x);
-    // prd (k, k-1) and pn2 (k, k+1) of the tile and a two-point halo, as stored
-    for (int q = tid; q < SX * SY; q += SLP_TX * SLP_TY) {
-        const int li = q % SX, lj = q / SX;
-        const int i = ib - 2 + li, j = jb - 2 + lj;
-        double a = 0., b = 0., c = 0., e = 0.;
-        if (i >= 1 && i <= d.jpi && j >= 1 && j <= d.jpj) {
-            const uint32_t p = IJK32(i, j, k);
-            a = (double)at32(in.prd, p);
-            b = (double)at32(in.prd, p - (uint32_t)d.n2);
-            c = (double)at32(in.pn2, p);
-            e = (double)at32(in.pn2, p + (uint32_t)d.n2);
-        }
-        p0[lj][li] = a;
-        pm[lj][li] = b;
-        n0[lj][li] = c;
-        np[lj][li] = e;
+    constexpr int N = SLP_RX * SLP_RY;
+    __shared__ double sp[N], sdz[N], su[N], sv[N], swi[N], swj[N];
+    __shared__ double q3u[SLP_MAXKB], q3v[SLP_MAXKB], q3w[SLP_MAXKB];   // -7e3 / e3 of the chunk's levels
+    __shared__ int s_end;
+    const Metrics<double> &m = d.md;
+    unsigned bx, by;
+    xcd_tile(bx, by);
+    const int jpi = d.jpi, jpj = d.jpj, jpkm1 = d.jpk - 1;
+    const int q = (int)threadIdx.x, lx = q % SLP_RX, ly = q / SLP_RX;
+    // the tile of interior points the workgroup owns, and its halo
+    const int hx = d.iper ? 4 : 2, hy = d.jper ? 4 : 2, wx = SLP_RX - 2 * hx, wy = SLP_RY - 2 * hy;
+    int i = 2 + (int)bx * wx + lx - hx, j = 2 + (int)by * wy + ly - hy;
+    const bool own = lx >= hx && lx < SLP_RX - hx && ly >= hy && ly < SLP_RY - hy && i <= jpi - 1 && j <= jpj - 1;
+    if (d.iper) i = ((i - 1) % jpi + jpi) % jpi + 1;
+    if (d.jper) j = ((j - 1) % jpj + jpj) % jpj + 1;
+    const int k0 = 2 + (int)blockIdx.z * kb, k1 = min(k0 + kb - 1, jpkm1);
+    const bool uni = d.e3_sij == 0;
+    const bool inner = i >= 2 && i <= jpi - 1 && j >= 2 && j <= jpj - 1;
+    // columns off the domain read its nearest one and are not used
+    const int ic = min(max(i, 1), jpi), jc = min(max(j, 1), jpj);
+    const uint32_t c = IJ32(ic, jc);
+    const uint32_t w_ = ic > 1 ? c - 1u : c, e_ = ic < jpi ? c + 1u : c;
+    const uint32_t s_ = jc > 1 ? c - (uint32_t)jpi : c, n_ = jc < jpj ? c + (uint32_t)jpi : c;
+    const uint32_t tc = d.ktu[c], tw = d.ktu[w_], tn = d.ktu[n_], ts = d.ktu[s_];
+    const uint32_t vc = d.kvf[c], vs = d.kvf[s_], ve = d.kvf[e_], vw = d.kvf[w_];
+    if (q == 0) s_end = 0;
+    __syncthreads();
+    atomicMax(&s_end, (int)((tc >> 8) & 255u));
+    if (uni && q < k1 - k0 + 1) {
+        q3u[q] = -7.e+3 / m.e3u[k0 + q - 1];
+        q3v[q] = -7.e+3 / m.e3v[k0 + q - 1];
+        q3w[q] = -7.e+3 / m.e3w[k0 + q - 1];
     }
     __syncthreads();
-    const auto lprd = [&](int i, int j, int kk) {
-        return kk == k ? p0[j - jb + 2][i - ib + 2] : pm[j - jb + 2][i - ib + 2];
-    };
-    const auto ln2 = [&](int i, int j, int kk) {
-        return kk == k ? n0[j - jb + 2][i - ib + 2] : np[j - jb + 2][i - ib + 2];
-    };
-    const GlobalField<T> gprd{in.prd, d}, gn2{in.pn2, d};
-    for (int q = tid; q < LX * LY; q += SLP_TX * SLP_TY) {
-        const int li = q % LX, lj = q / LX;
-        const int i = ib - 1 + li, j = jb - 1 + lj;
-        double a = 0., b = 0., c = 0., e = 0.;
-        int si, sj;
-        if (i <= d.jpi && j <= d.jpj && lbc_src(d, 'U', i, j, si, sj)) {
-            if (si == i && sj == j) {   // an interior point: its neighbours are staged
-                raw_uv<T>(d, lprd, ln2, gdept, nmln, zsu, zsv, z1_slpmax, si, sj, k, a, b);
-                raw_w<T>(d, lprd, ln2, gdepw, nmln, hmlp, wiml, wjml, si, sj, k, c, e);
-            } else {                    // a ring point: its lbc source, from global memory
-                raw_uv<T>(d, gprd, gn2, gdept, nmln, zsu, zsv, z1_slpmax, si, sj, k, a, b);
-                raw_w<T>(d, gprd, gn2, gdepw, nmln, hmlp, wiml, wjml, si, sj, k, c, e);
+    const int kend = min(k1, s_end);     // below: dry in every column
+    // a ring point's lbc source, by its place in the region; raw: the thread
+    // forms unfiltered slopes
+    int si = i, sj = j;
+    const bool in_dom = i >= 1 && i <= jpi && j >= 1 && j <= jpj;
+    const bool ring = in_dom && !inner && lbc_src(d, 'U', i, j, si, sj);
+    const int src = min(max(q + (si == i ? 0 : i == 1 ? -2 : 2) + SLP_RX * (sj == j ? 0 : j == 1 ? -2 : 2), 0), N - 1);
+    const bool cyc = (d.iper || d.jper) && __syncthreads_or(ring);
+    const bool edge = lx == 0 || lx == SLP_RX - 1 || ly == 0 || ly == SLP_RY - 1;
+    const bool raw = inner && !edge;
+    const auto um = [](uint32_t x, int k) { return k >= (int)((x >> 16) & 255u) && k <= (int)((x >> 24) & 255u); };
+    const auto vm = [](uint32_t x, int k) { return k >= (int)(x & 255u) && k <= (int)((x >> 8) & 255u); };   // also tmask
+    const auto msk = [](bool on, double x) { return on ? x : 0.; };
+    const double zm1_g = -1.0 / d.grav, zm1_2g = -0.5 / d.grav, z1_16 = 1.0 / 16.;
+    if (k0 <= kend) {
+        const double r1_e1u = m.r1_e1u[c], r1_e2v = m.r1_e2v[c], e1t = m.e1t[c], e2t = m.e2t[c];
+        const int ml_c = nmln[c] - 1, ml_e = nmln[e_] - 1, ml_n = nmln[n_] - 1;   // omlmask: k <= ml
+        const size_t plane = d.n2;
+        const auto ld = [&](const T *p, int k) { return (double)ldp(plane_ptr(p, plane, k), c); };
+        double p_m = ld(in.prd, k0 - 1), p_k = ld(in.prd, k0);
+        double n_k = ld(in.pn2, k0), n_p = ld(in.pn2, k0 + 1);
+        // gradients of the level above, and its masks
+        double gu_cm, gu_wm, gv_cm, gv_sm;
+        bool um_cm = um(tc, k0 - 1), um_wm = um(tw, k0 - 1), vm_cm = vm(vc, k0 - 1), vm_sm = vm(vs, k0 - 1);
+        bool um_c = um(tc, k0), vm_c = vm(vc, k0), tm_c = vm(tc, k0), tm_m = vm(tc, k0 - 1);
+        sp[q] = p_m;
+        __syncthreads();
+        gu_cm = msk(um_cm, sp[min(q + 1, N - 1)] - p_m);
+        gu_wm = msk(um_wm, p_m - sp[max(q - 1, 0)]);
+        gv_cm = msk(vm_cm, sp[min(q + SLP_RX, N - 1)] - p_m);
+        gv_sm = msk(vm_sm, p_m - sp[max(q - SLP_RX, 0)]);
+        __syncthreads();
+        for (int k = k0; k <= kend; k++) {
+            const int kn = min(k + 1, d.jpk);
+            const double p_n = ld(in.prd, kn), n_pn = ld(in.pn2, min(k + 2, d.jpk));   // the next level's
+            const bool um_w = um(tw, k), vm_s = vm(vs, k), um_cp = um(tc, k + 1), vm_cp = vm(vc, k + 1);
+            const bool tm_p = vm(tc, k + 1), wm = tm_c && tm_m;
+            const double dz = zm1_g * (p_k + 1.) * (n_k + n_p) * (tm_p ? 0.5 : 1.);   // zdzr, lines 162-170
+            sp[q] = p_k;
+            sdz[q] = dz;
+            __syncthreads();
+            double a = 0., b = 0., e = 0., f = 0.;
+            const bool ml_uv = raw && k <= max(ml_c, max(ml_e, ml_n)), ml_w = raw && k - 1 <= ml_c;
+            const bool any_uv = __any(ml_uv), any_w = __any(ml_w);
+            if (raw) {
+                const double gu_c = msk(um_c, sp[q + 1] - p_k), gu_w = msk(um_w, p_k - sp[q - 1]);
+                const double gv_c = msk(vm_c, sp[q + SLP_RX] - p_k), gv_s = msk(vm_s, p_k - sp[q - SLP_RX]);
+                const double e3u7 = uni ? q3u[k - k0] : -7.e+3 / E3(m.e3u, c, k);
+                const double e3v7 = uni ? q3v[k - k0] : -7.e+3 / E3(m.e3v, c, k);
+                const double e3w7 = uni ? q3w[k - k0] : -7.e+3 / E3(m.e3w, c, k);
+                // I. u, v slopes, lines 197-219
+                const double zau = gu_c * r1_e1u, zav = gv_c * r1_e2v;
+                double zbu = 0.5 * (dz + sdz[q + 1]), zbv = 0.5 * (dz + sdz[q + SLP_RX]);
+                zbu = min3(zbu, -z1_slpmax * fabs(zau), e3u7 * fabs(zau));
+                zbv = min3(zbv, -z1_slpmax * fabs(zav), e3v7 * fabs(zav));
+                double tu = zau / (zbu - ZEPS), tv = zav / (zbv - ZEPS);
+                if (any_uv) {
+                    const double oc = k <= ml_c ? 1. : 0.;
+                    const double zfi = max2(oc, k <= ml_e ? 1. : 0.), zfj = max2(oc, k <= ml_n ? 1. : 0.);
+                    const double gc = ld(gdept, k);
+                    const double zdepu = 0.5 * ((gc + (double)ldp(plane_ptr(gdept, plane, k), e_)) - E3(m.e3u, c, d.miku[c]));
+                    const double zdepv = 0.5 * ((gc + (double)ldp(plane_ptr(gdept, plane, k), n_)) - E3(m.e3v, c, d.mikv[c]));
+                    tu = (1. - zfi) * zau / (zbu - ZEPS) + zfi * zdepu * zsu[c];
+                    tv = (1. - zfj) * zav / (zbv - ZEPS) + zfj * zdepv * zsv[c];
+                }
+                a = msk(um_c, tu);
+                b = msk(vm_c, tv);
+                // II. w slopes, lines 277-304
+                const double zbw = zm1_2g * n_k * (p_k + p_m + 2.);
+                const double zci = max2((double)((int)um_w + (int)um_c + (int)um_wm + (int)um_cm), ZEPS) * e1t;
+                const double zcj = max2((double)((int)vm_s + (int)vm_cm + (int)vm_sm + (int)vm_c), ZEPS) * e2t;
+                const double zai = msk(wm, (gu_w + gu_cm + gu_wm + gu_c) / zci);
+                const double zaj = msk(wm, (gv_s + gv_cm + gv_sm + gv_c) / zcj);
+                const double zbi = min3(zbw, -100. * fabs(zai), e3w7 * fabs(zai));
+                const double zbj = min3(zbw, -100. * fabs(zaj), e3w7 * fabs(zaj));
+                double ti = zai / (zbi - ZEPS), tj = zaj / (zbj - ZEPS);
+                if (any_w) {
+                    const double zfk = max2(k <= ml_c ? 1. : 0., k - 1 <= ml_c ? 1. : 0.);
+                    const double gwt = (double)A3(gdepw, ic, jc, d.mikt[c]);
+                    const double zck = (ld(gdepw, k) - gwt) / max2(hmlp[c] - gwt, 10.);
+                    ti = ti * (1. - zfk) + zck * wiml[c] * zfk;
+                    tj = tj * (1. - zfk) + zck * wjml[c] * zfk;
+                }
+                e = msk(wm, ti);
+                f = msk(wm, tj);
+                gu_cm = gu_c; gu_wm = gu_w; gv_cm = gv_c; gv_sm = gv_s;
             }
+            su[q] = a;
+            sv[q] = b;
+            swi[q] = e;
+            swj[q] = f;
+            __syncthreads();
+            if (cyc) {
+                if (ring) { a = su[src]; b = sv[src]; e = swi[src]; f = swj[src]; }
+                __syncthreads();
+                if (ring) { su[q] = a; sv[q] = b; swi[q] = e; swj[q] = f; }
+                __syncthreads();
+            }
+            if (own) {
+                const auto shapiro = [&](const double *z) {
+                    const double *t = z + q;
+                    return t[-SLP_RX - 1] + t[-SLP_RX + 1] + t[SLP_RX - 1] + t[SLP_RX + 1] +
+                           2. * (t[-SLP_RX] + t[-1] + t[1] + t[SLP_RX]) + 4. * t[0];
+                };
+                double u = z1_16 * shapiro(su), v = z1_16 * shapiro(sv);
+                const auto two = [](bool x, bool y) { return (double)((int)x + (int)y); };
+                u = u * two(um(tn, k), um(ts, k)) * 0.5 * two(um_c, um_cp) * 0.5;
+                v = v * two(vm(ve, k), vm(vw, k)) * 0.5 * two(vm_c, vm_cp) * 0.5;
+                const double zcofw = wm ? z1_16 : 0.;
+                const double zck = two(um_c, um_w) * two(vm_c, vm_s) * 0.25;
+                stp(plane_ptr(uslp, plane, k), c, (T)u);
+                stp(plane_ptr(vslp, plane, k), c, (T)v);
+                stp(plane_ptr(wslpi, plane, k), c, (T)(shapiro(swi) * zcofw * zck));
+                stp(plane_ptr(wslpj, plane, k), c, (T)(shapiro(swj) * zcofw * zck));
+            }
+            p_m = p_k; p_k = p_n;
+            n_k = n_p; n_p = n_pn;
+            um_cm = um_c; um_wm = um_w; vm_cm = vm_c; vm_sm = vm_s;
+            um_c = um_cp; vm_c = vm_cp; tm_m = tm_c; tm_c = tm_p;
         }
-        su[lj][li] = a;
-        sv[lj][li] = b;
-        swi[lj][li] = c;
-        swj[lj][li] = e;
     }
-    __syncthreads();
-    const int li = (int)threadIdx.x + 1, lj = (int)threadIdx.y + 1;
-    const int i = ib - 1 + li, j = jb - 1 + lj;
-    if (i > d.jpi - 1 || j > d.jpj - 1) return;
-    auto shapiro = [&](const double (*z)[LX]) {
-        return z[lj - 1][li - 1] + z[lj - 1][li + 1] + z[lj + 1][li - 1] + z[lj + 1][li + 1] +
-               2. * (z[lj - 1][li] + z[lj][li - 1] + z[lj][li + 1] + z[lj + 1][li]) + 4. * z[lj][li];
-    };
-    const double z1_16 = 1.0 / 16.;
-    double u = z1_16 * shapiro(su);
-    double v = z1_16 * shapiro(sv);
-    u = u * (UMASK(double, i, j + 1, k) + UMASK(double, i, j - 1, k)) * 0.5 *
-        (UMASK(double, i, j, k) + UMASK(double, i, j, k + 1)) * 0.5;
-    v = v * (VMASK(double, i + 1, j, k) + VMASK(double, i - 1, j, k)) * 0.5 *
-        (VMASK(double, i, j, k) + VMASK(double, i, j, k + 1)) * 0.5;
-    const double zcofw = WMASK(double, i, j, k) * z1_16;
-    const double zck = (UMASK(double, i, j, k) + UMASK(double, i - 1, j, k)) *
-                       (VMASK(double, i, j, k) + VMASK(double, i, j - 1, k)) * 0.25;
-    const uint32_t p = IJK32(i, j, k);
-    at32(uslp, p) = (T)u;
-    at32(vslp, p) = (T)v;
-    at32(wslpi, p) = (T)(shapiro(swi) * zcofw * zck);
-    at32(wslpj, p) = (T)(shapiro(swj) * zcofw * zck);
+    if (!own) return;
+    for (int k = max(k0, kend + 1); k <= k1; k++) {
+        stp(plane_ptr(uslp, d.n2, k), c, T(0));
+        stp(plane_ptr(vslp, d.n2, k), c, T(0));
+        stp(plane_ptr(wslpi, d.n2, k), c, T(0));
+        stp(plane_ptr(wslpj, d.n2, k), c, T(0));
+    }
 }
 
 }  // namespace
@@ -339,16 +369,20 @@ int launch_ldf_slp(const T *prd, const T *pn2, const T *gdept, const T *gdepw, c
     Grid2 g2 = grid2(d.jpi, d.jpj);
     LAUNCH("ldf_slp", k_slp_mxl<T>, g2, d, in, nmln, hmlpt, z1_slpmax, zsu, zsv, wiml, wjml);
     Grid2 g;
-    g.block = dim3(SLP_TX, SLP_TY, 1);
-    g.grid = dim3((unsigned)((d.jpi - 2 + SLP_TX - 1) / SLP_TX), (unsigned)((d.jpj - 2 + SLP_TY - 1) / SLP_TY),
-                  (unsigned)(d.jpk - 2));
+    g.block = dim3(SLP_RX * SLP_RY, 1, 1);
+    const int wx = SLP_RX - (d.iper ? 8 : 4), wy = SLP_RY - (d.jper ? 8 : 4);
+    g.grid = dim3((unsigned)((d.jpi - 2 + wx - 1) / wx), (unsigned)((d.jpj - 2 + wy - 1) / wy), 1);
+    // levels per workgroup: long marches repeat fewer first levels, short ones
+    // fill the chip (two workgroups per CU) on small domains
+    const int tiles = (int)(g.grid.x * g.grid.y), nlev = d.jpk - 2;
+    int nz = (1536 + tiles - 1) / tiles;
+    nz = nz < 1 ? 1 : nz > (nlev + 3) / 4 ? (nlev + 3) / 4 : nz;
+    if ((nlev + nz - 1) / nz > SLP_MAXKB) nz = (nlev + SLP_MAXKB - 1) / SLP_MAXKB;
+    const int kb = (nlev + nz - 1) / nz;
+    g.grid.z = (unsigned)((nlev + kb - 1) / kb);
     LAUNCH("ldf_slp", k_slp<T>, g, d, in, gdept, gdepw, nmln, (const double *)zsu, (const double *)zsv, hmlp,
-           (const double *)wiml, (const double *)wjml, z1_slpmax, uslp, vslp, wslpi, wslpj);
-    int st;
-    if ((st = launch_lbc<T>(uslp, d.jpk, 'U', T(0))) || (st = launch_lbc<T>(vslp, d.jpk, 'V', T(0))) ||
-        (st = launch_lbc<T>(wslpi, d.jpk, 'W', T(0))) || (st = launch_lbc<T>(wslpj, d.jpk, 'W', T(0))))
-        return st;
-    return 0;
+           (const double *)wiml, (const double *)wjml, z1_slpmax, kb, uslp, vslp, wslpi, wslpj);
+    return launch_lbc4<T>(uslp, vslp, wslpi, wslpj, d.jpk);
 }
 
 #define INST(T)                                                                                                 \

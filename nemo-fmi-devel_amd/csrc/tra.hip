@@ -2156,12 +2156,7 @@ static int launch_fct_fluxes1(const DevDomain &d, double p2dt, const T *pu, cons
     else LAUNCHB(nm, (k_fct_h<0, T, 0, 0, 1>), (S_fct_h<0, T, 0, 0, 1>), g3, d, p2dt, pu, pv, pw, ptb, ptn, pta, zwi, zwx, zwy, nt);
     if (kn_v == 4) LAUNCHB(nm, (k_fct_v<0, T, 1, 1>), (S_fct_v<0, T, 1, 1>), gi, d, pw, ptb, ptn, zwz, nt);
     else LAUNCHB(nm, (k_fct_v<0, T, 0, 1>), (S_fct_v<0, T, 0, 1>), gi, d, pw, ptb, ptn, zwz, nt);
-    int st;
-    if ((st = launch_lbc<T>(zwi, d.jpk, 'T', T(0)))) return st;
-    if ((st = launch_lbc<T>(zwx, d.jpk, 'U', T(0)))) return st;
-    if ((st = launch_lbc<T>(zwy, d.jpk, 'V', T(0)))) return st;
-    if ((st = launch_lbc<T>(zwz, d.jpk, 'W', T(0)))) return st;
-    return 0;
+    return launch_lbc4<T>(zwi, zwx, zwy, zwz, d.jpk);
 }
 
 template <int TRP, typename T>
@@ -2246,10 +2241,7 @@ static int launch_fct_pairs(const DevDomain &d, double p2dt, const T *pu, const 
             else LAUNCHB(nm, (k_fct_v<TRP, T, 0, 1>), (S_fct_v<TRP, T, 0, 1>), gi, d, pw, ptb + o, ptn + o, zwz, nt);
         }
         const int nk = nt * d.jpk;
-        if ((st = launch_lbc<T>(zwi, nk, 'T', T(0)))) return st;
-        if ((st = launch_lbc<T>(zwx, nk, 'U', T(0)))) return st;
-        if ((st = launch_lbc<T>(zwy, nk, 'V', T(0)))) return st;
-        if ((st = launch_lbc<T>(zwz, nk, 'W', T(0)))) return st;
+        if ((st = launch_lbc4<T>(zwi, zwx, zwy, zwz, nk))) return st;
         if (!d.iper && !d.jper) {
             // closed domain: betas and limited divergence fused, both tracers in one launch
             constexpr int TY = FctLimTY<T>::value, NTH = FctLimTY<T>::nth;
