@@ -45,6 +45,8 @@ struct Ctx {
     double *stp_buf = nullptr;                          // stp_ctl partial maxima and results
     double *gsum_buf = nullptr;                         // glob_sum partial pairs and total
     unsigned *spg_bar = nullptr;                        // dyn_spg_ts grid barrier and status
+    int *fct_flag = nullptr;                            // FctDry's word on the device
+    int fct_gen = 0;                                    // ... and the number of the last call
     bool spg_check = false;                             // a cooperative phase 2 awaits its status check
     double *hsb_buf = nullptr;                          // dia_hsb partial pairs and sums
     std::vector<PlanRec> trace;                         // the launches traced for a plan
@@ -137,6 +139,11 @@ int tune(Tune which) { return g_tune[which]; }
 int *spg_rot_u() { return g_c->spg_rot_u; }
 int *spg_rot_s() { return g_c->spg_rot_s; }
 unsigned *spg_barrier() { return g_c->spg_bar; }
+FctDry fct_dry_next()
+{
+    g_c->fct_gen = g_c->fct_gen == 0x7fffffff ? 1 : g_c->fct_gen + 1;
+    return FctDry{g_c->fct_flag, g_c->fct_gen};
+}
 void spg_loop_launched() { g_c->spg_check = true; }
 void spg_ts_reset()
 {
@@ -213,6 +220,7 @@ static void free_domain()
     g_c->stp_buf = nullptr;
     g_c->gsum_buf = g_c->hsb_buf = nullptr;
     g_c->spg_bar = nullptr;
+    g_c->fct_flag = nullptr;
     g_c->spg_check = false;
     g_c->have_domain = false;
 }
@@ -538,6 +546,8 @@ static int register_domain(const nemo_hip_domain_t *h)
     if ((rc = dev_alloc((void **)&g_c->gsum_buf, glob_sum_scratch_bytes()))) return rc;
     if ((rc = dev_alloc((void **)&g_c->spg_bar, 64))) return rc;
     HIPCHK(hipMemset(g_c->spg_bar, 0, 64));
+    if ((rc = dev_alloc((void **)&g_c->fct_flag, 64))) return rc;
+    HIPCHK(hipMemset(g_c->fct_flag, 0, 64));
     if ((rc = dev_alloc((void **)&g_c->hsb_buf, dia_hsb_scratch_bytes() + 16 * sizeof(double)))) return rc;
     g_c->dom = d;
     if ((rc = launch_spg_register())) return rc;

@@ -301,7 +301,18 @@ __device__ __forceinline__ void xcd_tile(unsigned &bx, unsigned &by)
 // ---------------------------------------------------------------------------
 // host side: error state, stream, timing, launch wrapper
 // ---------------------------------------------------------------------------
+// whether a FCT call met transports that are not zero on dry columns: the flux
+// kernels then store the call's number in *flag.  With another number there,
+// every antidiffusive flux of a dry level is zero, and the limiter may stop at
+// the bottom.  A recorded call repeats its number: if one replay sets it, later
+// ones find it set, which only makes them march on.
+struct FctDry {
+    int *flag;
+    int gen;
+};
+
 namespace nh {
+FctDry fct_dry_next();         // for one FCT call of the current context
 int set_error(int code, const char *fmt, ...);
 hipStream_t stream();
 const DevDomain &dom();

@@ -257,11 +257,15 @@ struct S_fct_beta {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double p2dt, const T * __restrict__ pbef, const T * __restrict__ paft, const T * __restrict__ paa, const T * __restrict__ pbb, const T * __restrict__ pcc, T * __restrict__ zbetup, T * __restrict__ zbetdo)
     {
-        // one thread per interior cell column and block of KB levels
+        // one thread per interior cell column and block of KB levels; the
+        // tracers of the launch follow one another in grid.z
         THREAD_IJ_V(vb_, 2, 2);
         if (i > d.jpi - 1 || j > d.jpj - 1) return;
         const int jpk = d.jpk;
-        const int kb0 = (int)vb_.z * KB + 1;
+        const unsigned nb = (unsigned)((jpk - 1 + KB - 1) / KB);
+        const size_t o = (size_t)(vb_.z / nb) * d.n3;
+        pbef += o; paft += o; paa += o; pbb += o; pcc += o; zbetup += o; zbetdo += o;
+        const int kb0 = (int)(vb_.z % nb) * KB + 1;
         const int kb1 = kb0 + KB - 1 < jpk - 1 ? kb0 + KB - 1 : jpk - 1;
         const double zrtrn = 1.e-15;
         const size_t ij = IJ(i, j);
@@ -357,26 +361,38 @@ __device__ __forceinline__ double lim_z(const DevDomain &d, const T *pcc, const 
                        A3(bdo, i, j, k));
 }
 
-// (4) limited fluxes and final trend, traadv_fct.F90:404-426 + 288-297
+// (4) limited fluxes and final trend, traadv_fct.F90:404-426 + 288-297.  One
+// thread per interior column and block of FIN_KB levels, the limited vertical
+// flux of the lower face carried to the next level; the tracers of the launch
+// follow one another in grid.z.  (A thread per whole column and a launch per
+// tracer, 362x149x46 FP64: 193 us for both; in blocks 99 us.)
+#define FIN_KB 4
 template <typename T>
 struct S_fct_final {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const T * __restrict__ paa, const T * __restrict__ pbb, const T * __restrict__ pcc, const T * __restrict__ bup, const T * __restrict__ bdo, T * __restrict__ ta)
     {
-        // one thread per interior column, k-marched: the limited vertical flux of
-        // the lower face is carried to the next level
         THREAD_IJ_V(vb_, 2, 2);
         if (i > d.jpi - 1 || j > d.jpj - 1) return;
+        const unsigned nb = (unsigned)((d.jpk - 1 + FIN_KB - 1) / FIN_KB);
+        const size_t o = (size_t)(vb_.z / nb) * d.n3;
+        paa += o; pbb += o; pcc += o; bup += o; bdo += o; ta += o;
+        const int k0 = (int)(vb_.z % nb) * FIN_KB + 1, k1 = min(k0 + FIN_KB - 1, d.jpk - 1);
         const Metrics<T> &m = met<T>(d);
         const size_t ij = IJ(i, j);
         const T r1_e1e2t = m.r1_e1e2t[ij];
-        double lz_k = lim_z(d, pcc, bup, bdo, i, j, 1);
-        for (int k = 1; k <= d.jpk - 1; k++) {
+        double lz_k = lim_z(d, pcc, bup, bdo, i, j, k0);
+        T tv[FIN_KB];
+    #pragma unroll
+        for (int q = 0; q < FIN_KB; q++) tv[q] = A3(ta, i, j, min(k0 + q, k1));
+    #pragma unroll
+        for (int q = 0; q < FIN_KB; q++) {
+            const int k = k0 + q;
+            if (k > k1) break;
             const double lz_kp1 = lim_z(d, pcc, bup, bdo, i, j, k + 1);
             const T lx_i = (T)lim_x(d, paa, bup, bdo, i, j, k), lx_im1 = (T)lim_x(d, paa, bup, bdo, i - 1, j, k);
             const T ly_j = (T)lim_y(d, pbb, bup, bdo, i, j, k), ly_jm1 = (T)lim_y(d, pbb, bup, bdo, i, j - 1, k);
-            const size_t p = IJK(i, j, k);
-            ta[p] = ta[p] - (lx_i - lx_im1 + ly_j - ly_jm1 + (T)lz_k - (T)lz_kp1) * r1_e1e2t / E3(m.e3t, ij, k);
+            A3(ta, i, j, k) = tv[q] - (lx_i - lx_im1 + ly_j - ly_jm1 + (T)lz_k - (T)lz_kp1) * r1_e1e2t / E3(m.e3t, ij, k);
             lz_k = lz_kp1;
         }
     }
@@ -397,7 +413,12 @@ KERNEL void k_fct_final(DevDomain d, const T * __restrict__ paa, const T * __res
 // fluxes the limited divergence needs are passed on through LDS by the
 // threads that loaded them for the betas, the vertical flux of level k+1
 // stays in a register as the beta's flux of level k, and (FP32 storage) the
-// first guess of the betas comes from the plane fetched for the bounds.
+// first guess of the betas comes from the plane fetched for the bounds.  On
+// domains whose tiles leave the chip idle the levels are split over workgroups,
+// and the march ends at the tile's deepest wet level where the call's transports
+// are masked (FctDry).  Bound by vector instructions, so what the dry levels and
+// the idle chip cost counts: 1024x1024x75 FP32 2042 us over all levels, 1637 us
+// to the bottom; 512x512x75 FP64 830 and 706 us; 32x22x31 FP64 79 us unsplit, 38 us.
 // Every value is the one k_fct_beta and k_fct_final compute (same
 // expressions, same rounding to the storage type), and the ring values
 // lbc_lnk gives a closed domain (zero betas and limited fluxes) are selected
@@ -416,7 +437,7 @@ template <typename T> struct FctLimTY {
 template <typename T, int TY, int NTH = NH_BLOCK>
 struct S_fct_lim {
     static constexpr int NTHR = NTH, WAVES = NTH == 512 ? 4 : 3;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double p2dt, const T *__restrict__ pbef_, const T *__restrict__ paft_, const T *__restrict__ paa_, const T *__restrict__ pbb_, const T *__restrict__ pcc_, T *__restrict__ ta_)
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double p2dt, const T *__restrict__ pbef_, const T *__restrict__ paft_, const T *__restrict__ paa_, const T *__restrict__ pbb_, const T *__restrict__ pcc_, T *__restrict__ ta_, int nt, int kch, FctDry dry)
     {
         // bounds: FP64 with the reference's +-1e40 land sentinels; with FP32
         // storage they are exact in FP32 (max/min of stored values) and the
@@ -437,8 +458,10 @@ struct S_fct_lim {
         // paa, pbb of level k and pcc of level k+1 over the beta region, for
         // the limited divergence of level k
         __shared__ T faa_s[BY][BX], fbb_s[BY][BX], fcc_s[BY][BX];
-        // vb_.z selects the tracer of the pair
-        const size_t o = (size_t)vb_.z * d.n3;
+        __shared__ int s_bot;
+        // vb_.z selects the tracer of the pair and the chunk of kch levels
+        const size_t o = (size_t)(vb_.z % (unsigned)nt) * d.n3;
+        const int ka = (int)(vb_.z / (unsigned)nt) * kch + 1, kb = min(ka + kch - 1, d.jpk - 1);
         const T *pbef = pbef_ + o, *paft = paft_ + o, *paa = paa_ + o, *pbb = pbb_ + o, *pcc = pcc_ + o;
         T *ta = ta_ + o;
         unsigned bx, by;
@@ -639,7 +662,7 @@ struct S_fct_lim {
         };
         const int cx = tx + 1;
         const bool okxm = i - 1 >= 2;
-        auto fin_do = [&](int k) {
+        auto fin_do = [&](int k, bool store) {
             const int s0 = k & 1, s1 = (k + 1) & 1;
     #pragma unroll
             for (int r = 0; r < NR; r++) {
@@ -658,36 +681,60 @@ struct S_fct_lim {
                     okym ? lim_face<T>(fbb_s[cy - 1][cx], bdo_s[s0][cy - 1][cx], bu_c, bup_s[s0][cy - 1][cx], bd_c)
                          : 0.0;
                 const double lz_kp1 = lim_face<T>(fcc_s[cy][cx], bdo_s[s1][cy][cx], bu_c, bup_s[s1][cy][cx], bd_c);
-                A3(ta, i, j, k) = gta[r] - ((T)lx_i - (T)lx_im1 + (T)ly_j - (T)ly_jm1 + (T)lz_k[r] - (T)lz_kp1) *
+                if (store) A3(ta, i, j, k) = gta[r] - ((T)lx_i - (T)lx_im1 + (T)ly_j - (T)ly_jm1 + (T)lz_k[r] - (T)lz_kp1) *
                                                r1_e1e2t[r] / ge3t[r];
                 lz_k[r] = lz_kp1;
             }
         };
 
-        // ---- prologue: bounds of levels 1-3, betas of level 1, loads of the
-        // first iteration in flight
-        zb_fetch(1);
-        zb_store(1);
-        zb_fetch(2);
-        zb_store(2);
-        zb_fetch(3);
-        zb_store(3);
-        beta_fetch(1, true);
+        // the deepest wet level of the tile and its beta region
+        if (tid == 0) s_bot = 0;
         __syncthreads();
-        beta_make(1);
-        beta_fetch(2, false);
-        fin_fetch(1);
-        zb_fetch(4);
+        int bot = 0;
+    #pragma unroll
+        for (int r = 0; r < NB; r++)
+            if (bon[r]) bot = max(bot, (int)((d.ktu[bof[r]] >> 8) & 255u));
+        atomicMax(&s_bot, bot);
+        __syncthreads();
+        const int kdry = s_bot;
+        // A level whose fluxes are all zero leaves the trend as it is: below the
+        // deepest wet level they are, unless the call's transports are not masked
+        const int kstop = *dry.flag == dry.gen ? kb : min(kb, kdry);
+        if (kstop < ka) return;
+        // ---- prologue: bounds of levels ks-1 (the surface: 1) to ks+2, betas of
+        // level ks, loads of the first iteration in flight.  A chunk below the
+        // surface starts a level early, for the limited flux of its upper face
+        const int ks = ka > 1 ? ka - 1 : 1;
+        if (ks > 1) {
+            zb_fetch(ks - 1);
+            zb_store(ks - 1);
+        }
+        zb_fetch(ks);
+        zb_store(ks);
+        zb_fetch(ks + 1);
+        zb_store(ks + 1);
+        zb_fetch(ks + 2);
+        if (ks == 1) zb_store(3);
+        beta_fetch(ks, true);
+        __syncthreads();
+        beta_make(ks);
+        if (ks > 1) {
+            __syncthreads();
+            zb_store(ks + 2);
+        }
+        beta_fetch(ks + 1, false);
+        fin_fetch(ks);
+        zb_fetch(ks + 3);
         __syncthreads();
         // ---- march: at the top of iteration k the LDS holds the bounds of
         // levels k..k+2 and the betas of level k; the registers hold the loads
         // for the betas of level k+1, the cell of level k and the bounds of
         // level k+3
-        for (int k = 1; k <= jpk - 1; k++) {
+        for (int k = ks; k <= kstop; k++) {
             beta_make(k + 1);
             beta_fetch(k + 2, false);
             __syncthreads();
-            fin_do(k);
+            fin_do(k, k >= ka);
             fin_fetch(k + 1);
             zb_store(k + 3);
             zb_fetch(k + 4);
@@ -698,9 +745,9 @@ struct S_fct_lim {
 template <typename T, int TY, int NTH = NH_BLOCK>
 __global__ __launch_bounds__(NTH, (S_fct_lim<T, TY, NTH>::WAVES)) void k_fct_lim(DevDomain d, double p2dt, const T *__restrict__ pbef_, const T *__restrict__ paft_,
                       const T *__restrict__ paa_, const T *__restrict__ pbb_, const T *__restrict__ pcc_,
-                      T *__restrict__ ta_)
+                      T *__restrict__ ta_, int nt, int kch, FctDry dry)
 {
-    S_fct_lim<T, TY, NTH>::run(vb_hw(), d, p2dt, pbef_, paft_, paa_, pbb_, pcc_, ta_);
+    S_fct_lim<T, TY, NTH>::run(vb_hw(), d, p2dt, pbef_, paft_, paa_, pbb_, pcc_, ta_, nt, kch, dry);
 }
 
 template <typename T>
@@ -729,7 +776,9 @@ int launch_tra_adv_fct(double p2dt, const T *pun, const T *pvn, const T *pwn, co
         LAUNCHB("tra_adv_fct", (k_fct_beta<T, FctKB<T>::beta>), (S_fct_beta<T, FctKB<T>::beta>), gk, d, p2dt, tb, zwi, zwx, zwy, zwz, zbu, zbd);
         if ((st = launch_lbc<T>(zbu, d.jpk, 'T', T(0)))) return st;
         if ((st = launch_lbc<T>(zbd, d.jpk, 'T', T(0)))) return st;
-        LAUNCHB("tra_adv_fct", (k_fct_final<T>), (S_fct_final<T>), gi, d, zwx, zwy, zwz, zbu, zbd, ta);
+        Grid2 gf = gi;
+        gf.grid.z = (unsigned)((d.jpk - 1 + FIN_KB - 1) / FIN_KB);
+        LAUNCHB("tra_adv_fct", (k_fct_final<T>), (S_fct_final<T>), gf, d, zwx, zwy, zwz, zbu, zbd, ta);
     }
     return 0;
 }
@@ -1865,9 +1914,8 @@ template int launch_tra_zdf_imp<float>(double, int, const float *, float *, int,
 template <int TRP, typename T, int NH4, int TA0, int NT, int VERT = 1>
 struct S_fct_h {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double p2dt, const T *__restrict__ pu, const T *__restrict__ pv, const T *__restrict__ pw, const T *__restrict__ ptb, const T *__restrict__ ptn, T *__restrict__ pta, T *__restrict__ pzwi, T *__restrict__ pzwx, T *__restrict__ pzwy, int kjpt)
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double p2dt, const T *__restrict__ pu, const T *__restrict__ pv, const T *__restrict__ pw, const T *__restrict__ ptb, const T *__restrict__ ptn, T *__restrict__ pta, T *__restrict__ pzwi, T *__restrict__ pzwx, T *__restrict__ pzwy, FctDry dry)
     {
-        (void)kjpt;
         THREAD_IJ_V(vb_, 1, 1);
         const int k = (int)vb_.z + 1;
         if (i > d.jpi - 1 || j > d.jpj - 1) return;     // the flux loops: 1..jpim1 x 1..jpjm1
@@ -1875,15 +1923,49 @@ struct S_fct_h {
         const Metrics<T> &m = met<T>(d);
         const size_t n3 = d.n3;
         const T zp2dt = (T)p2dt;
+        const uint32_t c = IJ32(i, j);
+        const uint32_t tc = d.ktu[c];
         const T u = tr_u<TRP>(d, pu, i, j, k), v = tr_v<TRP>(d, pv, i, j, k);
         T um = T(0), vm = T(0), e3t = T(1), tm = T(0), r1_e1e2t = T(0);
         if (inner) {
             um = tr_u<TRP>(d, pu, i - 1, j, k);
             vm = tr_v<TRP>(d, pv, i, j - 1, k);
-            const size_t ij = IJ(i, j);
-            e3t = E3(m.e3t, ij, k);
-            tm = TMASK(T, i, j, k);
-            r1_e1e2t = m.r1_e1e2t[ij];
+        }
+        // a transport through the face of a dry cell: the limiter may not stop early
+        const bool wet = kin<0>(tc, k);
+        if ((!(u == T(0)) && !(wet && kin<0>(d.ktu[c + 1u], k))) || (!(v == T(0)) && !(wet && kin<0>(d.ktu[c + (uint32_t)d.jpi], k))))
+            *dry.flag = dry.gen;
+        // a dry wave whose transports are zero, as they are unless a caller's are
+        // not masked: zero fluxes, and a first guess that is masked
+        if (!__any(wet) && !__any(!(u == T(0) && v == T(0) && um == T(0) && vm == T(0)))) {
+    #pragma unroll
+            for (int t = 0; t < NT; t++) {
+                A3(pzwx + t * n3, i, j, k) = T(0);
+                A3(pzwy + t * n3, i, j, k) = T(0);
+                if (!inner) continue;
+                A3(pzwi + t * n3, i, j, k) = T(0);
+                if (VERT && TA0) A3(pta + t * n3, i, j, k) = T(0);
+                if (VERT && k == d.jpk - 1) A3(pzwi + t * n3, i, j, d.jpk) = T(0);
+            }
+            return;
+        }
+        if (inner) {
+            e3t = E3(m.e3t, c, k);
+            tm = wet ? T(1) : T(0);
+            r1_e1e2t = m.r1_e1e2t[c];
+        }
+        // order 4: zltu, zltv at this point and the next.  Away from the ring their
+        // lbc sources are the points themselves, and the two share a gradient
+        const bool self = i >= 2 && i <= d.jpi - 2 && j >= 2 && j <= d.jpj - 2;
+        const uint32_t w_ = self ? c - 1u : c, s_ = self ? c - (uint32_t)d.jpi : c;
+        const uint32_t e1 = c + 1u, n1 = c + (uint32_t)d.jpi;
+        const uint32_t e2 = self ? c + 2u : e1, n2_ = self ? c + 2u * (uint32_t)d.jpi : n1;
+        T mu_w = T(0), mu_c = T(0), mu_e = T(0), mv_s = T(0), mv_c = T(0), mv_n = T(0);
+        if (NH4) {
+            mu_w = kin<16>(d.ktu[w_], k) ? T(1) : T(0); mu_c = kin<16>(tc, k) ? T(1) : T(0);
+            mu_e = kin<16>(d.ktu[e1], k) ? T(1) : T(0);
+            mv_s = kin<0>(d.kvf[s_], k) ? T(1) : T(0); mv_c = kin<0>(d.kvf[c], k) ? T(1) : T(0);
+            mv_n = kin<0>(d.kvf[n1], k) ? T(1) : T(0);
         }
     #pragma unroll
         for (int t = 0; t < NT; t++) {
@@ -1891,12 +1973,22 @@ struct S_fct_h {
             const T tbc = A3(tb, i, j, k), tbe = A3(tb, i + 1, j, k), tbn = A3(tb, i, j + 1, k);
             const T hu = T(0.5) * ((u + fabs(u)) * tbc + (u - fabs(u)) * tbe);
             const T hv = T(0.5) * ((v + fabs(v)) * tbc + (v - fabs(v)) * tbn);
-            const T c2u = A3(tn, i, j, k) + A3(tn, i + 1, j, k);
-            const T c2v = A3(tn, i, j, k) + A3(tn, i, j + 1, k);
+            const T *tk = plane_ptr(tn, d.n2, k);
+            const T tnc = ldp(tk, c), tne = ldp(tk, e1), tnn = ldp(tk, n1);
+            const T c2u = tnc + tne, c2v = tnc + tnn;
             T *zwx = pzwx + t * n3, *zwy = pzwy + t * n3;
             if (NH4) {
-                A3(zwx, i, j, k) = T(0.5) * u * (c2u + fct_zltu(d, tn, i, j, k, true) - fct_zltu(d, tn, i + 1, j, k, true)) - hu;
-                A3(zwy, i, j, k) = T(0.5) * v * (c2v + fct_zltu(d, tn, i, j, k, false) - fct_zltu(d, tn, i, j + 1, k, false)) - hv;
+                const T r1_6 = T(1) / T(6);
+                const T gu_w = (tnc - ldp(tk, w_)) * mu_w, gu_c = (tne - tnc) * mu_c, gu_e = (ldp(tk, e2) - tne) * mu_e;
+                const T gv_s = (tnc - ldp(tk, s_)) * mv_s, gv_c = (tnn - tnc) * mv_c, gv_n = (ldp(tk, n2_) - tnn) * mv_n;
+                T lu0 = (gu_c + gu_w) * r1_6, lu1 = (gu_e + gu_c) * r1_6;
+                T lv0 = (gv_c + gv_s) * r1_6, lv1 = (gv_n + gv_c) * r1_6;
+                if (!self) {
+                    lu0 = fct_zltu(d, tn, i, j, k, true); lu1 = fct_zltu(d, tn, i + 1, j, k, true);
+                    lv0 = fct_zltu(d, tn, i, j, k, false); lv1 = fct_zltu(d, tn, i, j + 1, k, false);
+                }
+                A3(zwx, i, j, k) = T(0.5) * u * (c2u + lu0 - lu1) - hu;
+                A3(zwy, i, j, k) = T(0.5) * v * (c2v + lv0 - lv1) - hv;
             } else {
                 A3(zwx, i, j, k) = T(0.5) * u * c2u - hu;
                 A3(zwy, i, j, k) = T(0.5) * v * c2v - hv;
@@ -1921,74 +2013,135 @@ struct S_fct_h {
 template <int TRP, typename T, int NH4, int TA0, int NT>
 KERNEL void k_fct_h(DevDomain d, double p2dt, const T *__restrict__ pu, const T *__restrict__ pv,
                     const T *__restrict__ pw, const T *__restrict__ ptb, const T *__restrict__ ptn, T *__restrict__ pta,
-                    T *__restrict__ pzwi, T *__restrict__ pzwx, T *__restrict__ pzwy, int kjpt)
+                    T *__restrict__ pzwi, T *__restrict__ pzwx, T *__restrict__ pzwy, FctDry dry)
 {
-    S_fct_h<TRP, T, NH4, TA0, NT, 1>::run(vb_hw(), d, p2dt, pu, pv, pw, ptb, ptn, pta, pzwi, pzwx, pzwy, kjpt);
+    S_fct_h<TRP, T, NH4, TA0, NT, 1>::run(vb_hw(), d, p2dt, pu, pv, pw, ptb, ptn, pta, pzwi, pzwx, pzwy, dry);
 }
 // the horizontal half alone (VERT = 0)
 template <int TRP, typename T, int NH4, int NT>
 KERNEL void k_fct_hh(DevDomain d, double p2dt, const T *__restrict__ pu, const T *__restrict__ pv,
                      const T *__restrict__ pw, const T *__restrict__ ptb, const T *__restrict__ ptn, T *__restrict__ pta,
-                     T *__restrict__ pzwi, T *__restrict__ pzwx, T *__restrict__ pzwy, int kjpt)
+                     T *__restrict__ pzwi, T *__restrict__ pzwx, T *__restrict__ pzwy, FctDry dry)
 {
-    S_fct_h<TRP, T, NH4, 1, NT, 0>::run(vb_hw(), d, p2dt, pu, pv, pw, ptb, ptn, pta, pzwi, pzwx, pzwy, kjpt);
+    S_fct_h<TRP, T, NH4, 1, NT, 0>::run(vb_hw(), d, p2dt, pu, pv, pw, ptb, ptn, pta, pzwi, pzwx, pzwy, dry);
 }
 
 // per interior column: the vertical antidiffusive flux zwz (lines 255-278),
 // the compact scheme's sweeps (577-614) with the table pivots
+// Levels whose operands k_fct_v loads together, ahead of their stores, which the
+// compiler will not move loads across; below a wave's deepest wet level only
+// zeros are stored.  Order 4, 362x149x46 FP64: 84 us a level at a time, 56 us.
+// Order 2 has no recurrence, so each KB levels are a workgroup's (32x22x31 FP64,
+// both tracers: 20.8 us in columns, 6.4 us).
+#define FCTV_KB 8
 template <int TRP, typename T, int NV4, int NT>
 struct S_fct_v {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
+    static constexpr int KB = FCTV_KB;
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const T *__restrict__ pw, const T *__restrict__ ptb, const T *__restrict__ ptn, T *__restrict__ pzwz, int kjpt)
     {
         (void)kjpt;
         THREAD_IJ_V(vb_, 2, 2);
-        if (i > d.jpi - 1 || j > d.jpj - 1) return;
-        const size_t n3 = d.n3;
+        const bool on = i <= d.jpi - 1 && j <= d.jpj - 1;
         const int jpk = d.jpk;
-        const int ikb = d.mbkt[IJ(i, j)];
+        const uint32_t c = on ? IJ32(i, j) : 0u;
+        const uint32_t tc = on ? d.ktu[c] : 1u;
+        // below the wave's deepest wet level the w-mask makes every flux zero
+        const int kend = min(wave_max((int)((tc >> 8) & 255u)), jpk - 1);
+        if (!on) return;
+        const size_t n3 = d.n3, plane = d.n2;
+        const int ikb = d.mbkt[c];
+        const T e1e2t = TRP ? met<T>(d).e1e2t[c] : T(1);
+        const auto wmask = [&](int k) { return (kin<0>(tc, k) && (k == 1 || kin<0>(tc, k - 1))) ? T(1) : T(0); };
+        if constexpr (!NV4) {
+            // the mean of two levels: every level for itself, KB of them per workgroup
+            const int k0 = 1 + (int)vb_.z * KB;
+    #pragma unroll
+            for (int t = 0; t < NT; t++) {
+                const T *tb = ptb + t * n3, *tn = ptn + t * n3;
+                T nv[KB + 1], wv[KB], bv[KB + 1];
+                if (k0 <= kend) {
+    #pragma unroll
+                    for (int q = 0; q <= KB; q++) {
+                        const int k = min(max(k0 - 1 + q, 1), jpk);
+                        nv[q] = ldp(plane_ptr(tn, plane, k), c);
+                        bv[q] = ldp(plane_ptr(tb, plane, k), c);
+                        if (q) wv[q - 1] = ldp(plane_ptr(pw, plane, k), c);
+                    }
+                }
+    #pragma unroll
+                for (int q = 0; q < KB; q++) {
+                    const int k = k0 + q;
+                    if (k > jpk) break;
+                    T f = T(0);
+                    if (k > 1 && k <= kend) {
+                        const T wm = wmask(k), w = TRP ? e1e2t * wv[q] : wv[q];
+                        const T upz = T(0.5) * ((w + fabs(w)) * bv[q + 1] + (w - fabs(w)) * bv[q]) * wm;
+                        f = (w * T(0.5) * (nv[q + 1] + nv[q]) - upz) * wm;
+                    }
+                    stp(plane_ptr(pzwz + t * n3, plane, k), c, f);
+                }
+            }
+            return;
+        }
     #pragma unroll
         for (int t = 0; t < NT; t++) {
             const T *tb = ptb + t * n3, *tn = ptn + t * n3;
             T *zwz = pzwz + t * n3;
             A3(zwz, i, j, 1) = T(0);
             A3(zwz, i, j, jpk) = T(0);
-            if (!NV4) {
-    #pragma unroll 4
-                for (int k = 2; k <= jpk - 1; k++)
-                    A3(zwz, i, j, k) = (tr_w<TRP>(d, pw, i, j, k) * T(0.5) * (A3(tn, i, j, k) + A3(tn, i, j, k - 1)) -
-                                        tp_upz<TRP>(d, pw, tb, i, j, k)) *
-                                       WMASK(T, i, j, k);
-                continue;
-            }
-            T zout_prev = T(0), tn_km1 = A3(tn, i, j, 1);
-    #pragma unroll 4
-            for (int k = 2; k <= jpk - 1; k++) {
-                const T tnk = A3(tn, i, j, k);
-                T zwrm, zout, zwi_c = T(0);
-                if (k == 2 || k == ikb) {
-                    zwrm = T(0.5) * (tn_km1 + tnk);
-                } else {
-                    const T wm = WMASK(T, i, j, k);
-                    zwi_c = wm;
-                    zwrm = T(3) * wm * (tnk + tn_km1);
+            T zout_prev = T(0), tn_km1 = ldp(tn, c);
+            for (int k0 = 2; k0 <= kend; k0 += KB) {
+                T tv[KB];
+    #pragma unroll
+                for (int q = 0; q < KB; q++) tv[q] = ldp(plane_ptr(tn, plane, min(k0 + q, kend)), c);
+    #pragma unroll
+                for (int q = 0; q < KB; q++) {
+                    const int k = k0 + q;
+                    if (k > kend) break;
+                    const T tnk = tv[q];
+                    T zwrm, zout, zwi_c = T(0);
+                    if (k == 2 || k == ikb) {
+                        zwrm = T(0.5) * (tn_km1 + tnk);
+                    } else {
+                        const T wm = wmask(k);
+                        zwi_c = wm;
+                        zwrm = T(3) * wm * (tnk + tn_km1);
+                    }
+                    if (k == 2) zout = zwrm;
+                    else zout = zwrm - zwi_c / cpt_piv(cpt_tab<T>(), k - 1, ikb) * zout_prev;
+                    stp(plane_ptr(zwz, plane, k), c, zout);
+                    zout_prev = zout;
+                    tn_km1 = tnk;
                 }
-                if (k == 2) zout = zwrm;
-                else zout = zwrm - zwi_c / cpt_piv(cpt_tab<T>(), k - 1, ikb) * zout_prev;
-                A3(zwz, i, j, k) = zout;
-                zout_prev = zout;
-                tn_km1 = tnk;
             }
-            T xnext = zout_prev / cpt_piv(cpt_tab<T>(), jpk - 1, ikb);
-            A3(zwz, i, j, jpk - 1) = (tr_w<TRP>(d, pw, i, j, jpk - 1) * xnext - tp_upz<TRP>(d, pw, tb, i, j, jpk - 1)) *
-                                     WMASK(T, i, j, jpk - 1);
-    #pragma unroll 4
-            for (int k = jpk - 2; k >= 2; k--) {
-                const T zws = (k == 2 || k == ikb) ? T(0) : WMASK(T, i, j, k);
-                const T x = (A3(zwz, i, j, k) - zws * xnext) / cpt_piv(cpt_tab<T>(), k, ikb);
-                A3(zwz, i, j, k) = (tr_w<TRP>(d, pw, i, j, k) * x - tp_upz<TRP>(d, pw, tb, i, j, k)) * WMASK(T, i, j, k);
-                xnext = x;
+            // fluxes from the bottom up with the back substitution (nothing
+            // enters the deepest row)
+            T xnext = T(0);
+            for (int k1 = kend; k1 >= 2; k1 -= KB) {
+                T zv[KB], wv[KB], bv[KB + 1];
+    #pragma unroll
+                for (int q = 0; q < KB; q++) {
+                    const int k = max(k1 - q, 2);
+                    zv[q] = ldp(plane_ptr((const T *)zwz, plane, k), c);
+                    wv[q] = ldp(plane_ptr(pw, plane, k), c);
+                    bv[q] = ldp(plane_ptr(tb, plane, k), c);
+                }
+                bv[KB] = ldp(plane_ptr(tb, plane, max(k1 - KB, 1)), c);
+    #pragma unroll
+                for (int q = 0; q < KB; q++) {
+                    const int k = k1 - q;
+                    if (k < 2) break;
+                    const T wm = wmask(k), w = TRP ? e1e2t * wv[q] : wv[q];
+                    const T b_km1 = k == 2 ? ldp(tb, c) : bv[q + 1];
+                    const T upz = T(0.5) * ((w + fabs(w)) * bv[q] + (w - fabs(w)) * b_km1) * wm;
+                    const T zws = (k == 2 || k == ikb) ? T(0) : wm;
+                    const T x = (zv[q] - zws * xnext) / cpt_piv(cpt_tab<T>(), k, ikb);
+                    xnext = x;
+                    stp(plane_ptr(zwz, plane, k), c, (w * x - upz) * wm);
+                }
             }
+            for (int k = max(kend, 1) + 1; k <= jpk - 1; k++) stp(plane_ptr(zwz, plane, k), c, T(0));
         }
     }
 };
@@ -2018,9 +2171,13 @@ struct S_fct_vz_reg {
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double p2dt, const float *__restrict__ pw, const float *__restrict__ ptb, const float *__restrict__ ptn, float *__restrict__ pta, float *__restrict__ pzwi, float *__restrict__ pzwz)
     {
         THREAD_IJ_V(vb_, 2, 2);
-        if (i > d.jpi - 1 || j > d.jpj - 1) return;
-        const size_t n3 = d.n3;
+        const bool on = i <= d.jpi - 1 && j <= d.jpj - 1;
         const int jpk = d.jpk;
+        // below the wave's deepest wet level the masks make zwz and zwi zero and
+        // leave the trend alone
+        const int kend = min(wave_max(on ? (int)((d.ktu[IJ32(i, j)] >> 8) & 255u) : 0), jpk - 1);
+        if (!on) return;
+        const size_t n3 = d.n3;
         const size_t ij = IJ(i, j);
         const int ikb = d.mbkt[ij];
         const Metrics<float> &m = met<float>(d);
@@ -2032,13 +2189,19 @@ struct S_fct_vz_reg {
         A3(zwz, i, j, 1) = 0.0f;
         A3(zwz, i, j, jpk) = 0.0f;
         A3(zwi, i, j, jpk) = 0.0f;
+        for (int k = kend + 1; k <= jpk - 1; k++) {
+            A3(zwz, i, j, k) = 0.0f;
+            A3(zwi, i, j, k) = 0.0f;
+            if (TA0) A3(ta, i, j, k) = 0.0f;
+        }
+        if (kend < 1) return;
         float zo[KMAX];
         // every level's loads are issued two levels ahead, from addresses
         // within the arrays, so they are in flight across the level guards
         float zout_prev = 0.0f, tn_km1 = A3(tn, i, j, 1), tn_n1 = A3(tn, i, j, 2), tn_n2 = A3(tn, i, j, jpk > 2 ? 3 : jpk);
     #pragma unroll
         for (int k = 2; k < KMAX; k++) {
-            if (k <= jpk - 1) {
+            if (k <= kend) {
                 const float tnk = tn_n1;
                 tn_n1 = tn_n2;
                 tn_n2 = A3(tn, i, j, k + 2 <= jpk ? k + 2 : jpk);
@@ -2058,7 +2221,7 @@ struct S_fct_vz_reg {
             }
         }
         // level k's operands: wn (or pwn), tb(k), the stored s, ta, e3t (and
-        // tb(k-1), level k-1's); the climb starts at level jpk - 1
+        // tb(k-1), level k-1's); the climb starts at level kend
         struct Lv { float w, tb, s, a, e3; };
         const float *wr = pw;
         const auto lv = [&](int k) {
@@ -2070,13 +2233,13 @@ struct S_fct_vz_reg {
             l.e3 = E3(m.e3t, ij, k);
             return l;
         };
-        const int kf = jpk - 1;
+        const int kf = kend;
         Lv cur = lv(kf), nx = lv(kf > 1 ? kf - 1 : 1);
         const float e1e2t = TRP ? m.e1e2t[ij] : 1.0f;
-        float xnext = 0.0f, upz_kp1 = 0.0f;   // upz(jpk) = 0
+        float xnext = 0.0f, upz_kp1 = 0.0f;   // nothing enters level kend from below
     #pragma unroll
         for (int k = KMAX - 1; k >= 1; k--) {
-            if (k <= jpk - 1) {
+            if (k <= kend) {
                 Lv nn = nx;
                 if (k >= 3) nn = lv(k - 2);
                 const float w_c = cur.w, tb_c = cur.tb, tbm_c = nx.tb, s_c = cur.s, a_c = cur.a, e3_c = cur.e3;
@@ -2086,13 +2249,8 @@ struct S_fct_vz_reg {
                 const float upz = (k == 1) ? w * tb_c : 0.5f * (zfp * tb_c + zfm * tbm_c) * WMASK(float, i, j, k);
                 if (k >= 2) {   // zwz, as k_fct_v
                     const float wm = WMASK(float, i, j, k);
-                    float x;
-                    if (k == jpk - 1) {
-                        x = zo[k] / cpt_piv(cpt_tab<float>(), k, ikb);
-                    } else {
-                        const float zws = (k == 2 || k == ikb) ? 0.0f : wm;
-                        x = (zo[k] - zws * xnext) / cpt_piv(cpt_tab<float>(), k, ikb);
-                    }
+                    const float zws = (k == 2 || k == ikb) ? 0.0f : wm;
+                    const float x = (zo[k] - zws * xnext) / cpt_piv(cpt_tab<float>(), k, ikb);
                     A3(zwz, i, j, k) = (w * x - upz) * wm;
                     xnext = x;
                 }
@@ -2149,13 +2307,15 @@ static int launch_fct_fluxes1(const DevDomain &d, double p2dt, const T *pu, cons
                               const T *ptn, T *pta, int kn_h, int kn_v, T *zwi, T *zwx, T *zwy, T *zwz,
                               const char *nm)
 {
-    Grid2 g3 = grid2(d.jpi - 1, d.jpj - 1), gi = grid2(d.jpi - 2, d.jpj - 2);
+    Grid2 g3 = grid2(d.jpi - 1, d.jpj - 1), gi = grid2(d.jpi - 2, d.jpj - 2), gw = gi;
     g3.grid.z = (unsigned)(d.jpk - 1);
+    gw.grid.z = (unsigned)((d.jpk + FCTV_KB - 1) / FCTV_KB);
     const int nt = 1;
-    if (kn_h == 4) LAUNCHB(nm, (k_fct_h<0, T, 1, 0, 1>), (S_fct_h<0, T, 1, 0, 1>), g3, d, p2dt, pu, pv, pw, ptb, ptn, pta, zwi, zwx, zwy, nt);
-    else LAUNCHB(nm, (k_fct_h<0, T, 0, 0, 1>), (S_fct_h<0, T, 0, 0, 1>), g3, d, p2dt, pu, pv, pw, ptb, ptn, pta, zwi, zwx, zwy, nt);
+    const FctDry dry = nh::fct_dry_next();
+    if (kn_h == 4) LAUNCHB(nm, (k_fct_h<0, T, 1, 0, 1>), (S_fct_h<0, T, 1, 0, 1>), g3, d, p2dt, pu, pv, pw, ptb, ptn, pta, zwi, zwx, zwy, dry);
+    else LAUNCHB(nm, (k_fct_h<0, T, 0, 0, 1>), (S_fct_h<0, T, 0, 0, 1>), g3, d, p2dt, pu, pv, pw, ptb, ptn, pta, zwi, zwx, zwy, dry);
     if (kn_v == 4) LAUNCHB(nm, (k_fct_v<0, T, 1, 1>), (S_fct_v<0, T, 1, 1>), gi, d, pw, ptb, ptn, zwz, nt);
-    else LAUNCHB(nm, (k_fct_v<0, T, 0, 1>), (S_fct_v<0, T, 0, 1>), gi, d, pw, ptb, ptn, zwz, nt);
+    else LAUNCHB(nm, (k_fct_v<0, T, 0, 1>), (S_fct_v<0, T, 0, 1>), gw, d, pw, ptb, ptn, zwz, nt);
     return launch_lbc4<T>(zwi, zwx, zwy, zwz, d.jpk);
 }
 
@@ -2165,15 +2325,17 @@ static int launch_fct_pairs(const DevDomain &d, double p2dt, const T *pu, const 
 {
     // scratch slot pairs (two tracers of either storage type each)
     T *zwi = (T *)nh::scratch3(0), *zwx = (T *)nh::scratch3(2), *zwy = (T *)nh::scratch3(4);
-    T *zwz = (T *)nh::scratch3(6), *bu = (T *)nh::scratch3(8), *bd = (T *)nh::scratch3(10);
+    T *zwz = (T *)nh::scratch3(6), *bu = (T *)nh::scratch3(8), *bd = bu + 2 * d.n3;   // four slots: bd follows two tracers' bu
     const char *nm = TRP ? "step_tra" : "tra_adv_fct";
-    Grid2 gi = grid2(d.jpi - 2, d.jpj - 2), gk = gi;
+    Grid2 gi = grid2(d.jpi - 2, d.jpj - 2), gk = gi, gw = gi;
     gk.grid.z = (unsigned)((d.jpk - 1 + FctKB<T>::beta - 1) / FctKB<T>::beta);
+    gw.grid.z = (unsigned)((d.jpk + FCTV_KB - 1) / FCTV_KB);   // k_fct_v of order 2
     const size_t n3 = d.n3;
     int st;
     for (int t0 = 0; t0 < kjpt; t0 += 2) {
         const int nt = kjpt - t0 < 2 ? kjpt - t0 : 2;
         const size_t o = (size_t)t0 * n3;
+        const FctDry dry = nh::fct_dry_next();
         if (!d.iper && !d.jper && nh::tune(nh::T_FCT_FUSED)) {
             // closed domain: the whole chain in one kernel per tile and tracer
             // (zwz's slots hold the compact scheme's forward elimination)
@@ -2189,7 +2351,7 @@ static int launch_fct_pairs(const DevDomain &d, double p2dt, const T *pu, const 
             // forward sweep, then the vertical fluxes, first guess and limiter
             // in one bottom-up march (zwi holds s, zwz the forward sweep)
 #define FH_LAUNCH2(H, N) \
-    LAUNCHB(nm, (k_fct_hh<TRP, T, H, N>), (S_fct_h<TRP, T, H, 1, N, 0>), g3, d, p2dt, pu, pv, pw, ptb + o, ptn + o, pta + o, zwi, zwx, zwy, nt)
+    LAUNCHB(nm, (k_fct_hh<TRP, T, H, N>), (S_fct_h<TRP, T, H, 1, N, 0>), g3, d, p2dt, pu, pv, pw, ptb + o, ptn + o, pta + o, zwi, zwx, zwy, dry)
             if (kn_fct_h == 4) { if (nt == 2) FH_LAUNCH2(1, 2); else FH_LAUNCH2(1, 1); }
             else { if (nt == 2) FH_LAUNCH2(0, 2); else FH_LAUNCH2(0, 1); }
 #undef FH_LAUNCH2
@@ -2208,7 +2370,7 @@ static int launch_fct_pairs(const DevDomain &d, double p2dt, const T *pu, const 
                 // horizontal fluxes per cell, then the vertical fluxes, the
                 // low-order trend and the first guess per column
 #define FH_LAUNCH2(H, N) \
-    LAUNCHB(nm, (k_fct_hh<TRP, T, H, N>), (S_fct_h<TRP, T, H, 1, N, 0>), g3, d, p2dt, pu, pv, pw, ptb + o, ptn + o, pta + o, zwi, zwx, zwy, nt)
+    LAUNCHB(nm, (k_fct_hh<TRP, T, H, N>), (S_fct_h<TRP, T, H, 1, N, 0>), g3, d, p2dt, pu, pv, pw, ptb + o, ptn + o, pta + o, zwi, zwx, zwy, dry)
                 if (kn_fct_h == 4) { if (nt == 2) FH_LAUNCH2(1, 2); else FH_LAUNCH2(1, 1); }
                 else { if (nt == 2) FH_LAUNCH2(0, 2); else FH_LAUNCH2(0, 1); }
 #undef FH_LAUNCH2
@@ -2221,7 +2383,7 @@ static int launch_fct_pairs(const DevDomain &d, double p2dt, const T *pu, const 
         }
         if (!vdone) {
 #define FH_LAUNCH2(H, Z, N) \
-    LAUNCHB(nm, (k_fct_h<TRP, T, H, Z, N>), (S_fct_h<TRP, T, H, Z, N>), g3, d, p2dt, pu, pv, pw, ptb + o, ptn + o, pta + o, zwi, zwx, zwy, nt)
+    LAUNCHB(nm, (k_fct_h<TRP, T, H, Z, N>), (S_fct_h<TRP, T, H, Z, N>), g3, d, p2dt, pu, pv, pw, ptb + o, ptn + o, pta + o, zwi, zwx, zwy, dry)
 #define FH_LAUNCH(H, Z) \
     do { if (nt == 2) FH_LAUNCH2(H, Z, 2); else FH_LAUNCH2(H, Z, 1); } while (0)
             if (kn_fct_h == 4) {
@@ -2237,8 +2399,8 @@ static int launch_fct_pairs(const DevDomain &d, double p2dt, const T *pu, const 
             if (nt == 2) LAUNCHB(nm, (k_fct_v<TRP, T, 1, 2>), (S_fct_v<TRP, T, 1, 2>), gi, d, pw, ptb + o, ptn + o, zwz, nt);
             else LAUNCHB(nm, (k_fct_v<TRP, T, 1, 1>), (S_fct_v<TRP, T, 1, 1>), gi, d, pw, ptb + o, ptn + o, zwz, nt);
         } else {
-            if (nt == 2) LAUNCHB(nm, (k_fct_v<TRP, T, 0, 2>), (S_fct_v<TRP, T, 0, 2>), gi, d, pw, ptb + o, ptn + o, zwz, nt);
-            else LAUNCHB(nm, (k_fct_v<TRP, T, 0, 1>), (S_fct_v<TRP, T, 0, 1>), gi, d, pw, ptb + o, ptn + o, zwz, nt);
+            if (nt == 2) LAUNCHB(nm, (k_fct_v<TRP, T, 0, 2>), (S_fct_v<TRP, T, 0, 2>), gw, d, pw, ptb + o, ptn + o, zwz, nt);
+            else LAUNCHB(nm, (k_fct_v<TRP, T, 0, 1>), (S_fct_v<TRP, T, 0, 1>), gw, d, pw, ptb + o, ptn + o, zwz, nt);
         }
         const int nk = nt * d.jpk;
         if ((st = launch_lbc4<T>(zwi, zwx, zwy, zwz, nk))) return st;
@@ -2248,20 +2410,27 @@ static int launch_fct_pairs(const DevDomain &d, double p2dt, const T *pu, const 
             Grid2 gl = grid2(d.jpi - 2, d.jpj - 2);
             gl.block = dim3(LIM_TX, NTH / LIM_TX, 1);
             gl.grid.y = (unsigned)((d.jpj - 2 + TY - 1) / TY);
-            gl.grid.z = (unsigned)nt;
-            LAUNCHB(nm, (k_fct_lim<T, TY, NTH>), (S_fct_lim<T, TY, NTH>), gl, d, p2dt, ptb + o, zwi, zwx, zwy, zwz, pta + o);
+            // levels per workgroup: all of them where the tiles fill the chip (three
+            // workgroups per CU), else chunks (two extra levels each) of 8 or more
+            const int wgs = (int)(gl.grid.x * gl.grid.y) * nt, nlev = d.jpk - 1;
+            int nch = nh::planning() ? 1 : 768 / wgs;
+            nch = nch < 1 ? 1 : nch > nlev / 8 ? (nlev / 8 > 0 ? nlev / 8 : 1) : nch;
+            const int kch = (nlev + nch - 1) / nch;
+            gl.grid.z = (unsigned)(nt * ((nlev + kch - 1) / kch));
+            LAUNCHB(nm, (k_fct_lim<T, TY, NTH>), (S_fct_lim<T, TY, NTH>), gl, d, p2dt, ptb + o, zwi, zwx, zwy, zwz, pta + o, nt, kch, dry);
             continue;
         }
-        for (int t = 0; t < nt; t++) {
-            const size_t q = (size_t)t * n3;
-            LAUNCHB(nm, (k_fct_beta<T, FctKB<T>::beta>), (S_fct_beta<T, FctKB<T>::beta>), gk, d, p2dt, ptb + o + q, zwi + q, zwx + q, zwy + q, zwz + q, bu + q, bd + q);
+        Grid2 gb = gk, gf = gi;
+        gb.grid.z *= (unsigned)nt;
+        gf.grid.z = (unsigned)(nt * ((d.jpk - 1 + FIN_KB - 1) / FIN_KB));
+        LAUNCHB(nm, (k_fct_beta<T, FctKB<T>::beta>), (S_fct_beta<T, FctKB<T>::beta>), gb, d, p2dt, ptb + o, zwi, zwx, zwy, zwz, bu, bd);
+        if (nt == 2) {   // both in one launch
+            if ((st = launch_lbc<T>(bu, 2 * nk, 'T', T(0)))) return st;
+        } else {
+            if ((st = launch_lbc<T>(bu, nk, 'T', T(0)))) return st;
+            if ((st = launch_lbc<T>(bd, nk, 'T', T(0)))) return st;
         }
-        if ((st = launch_lbc<T>(bu, nk, 'T', T(0)))) return st;
-        if ((st = launch_lbc<T>(bd, nk, 'T', T(0)))) return st;
-        for (int t = 0; t < nt; t++) {
-            const size_t q = (size_t)t * n3;
-            LAUNCHB(nm, (k_fct_final<T>), (S_fct_final<T>), gi, d, zwx + q, zwy + q, zwz + q, bu + q, bd + q, pta + o + q);
-        }
+        LAUNCHB(nm, (k_fct_final<T>), (S_fct_final<T>), gf, d, zwx, zwy, zwz, bu, bd, pta + o);
     }
     if (ta0) {
         Grid2 ga = grid2(d.jpi, d.jpj);
