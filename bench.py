@@ -647,7 +647,7 @@ def kernel_times(h):
         "step_tra": ["k_fct_fused", "k_fct_cpt_fwd", "k_fct_h", "k_fct_hh", "k_fct_v", "k_fct_vz_reg", "k_fct_lim", "k_fct_vlim",
                      "k_fct_beta", "k_fct_final", "k_zero_ring", "k_tra_zdf", "k_tra_zdf_reg"],
         "div_hor": ["k_div_hor"], "ssh_nxt": ["k_ssh_nxt"], "wzv": ["k_wzv"], "ssh_swp": ["k_ssh_swp"],
-        "tra_nxt": ["k_tra_nxt"], "dyn_nxt": ["k_dyn_nxt1", "k_dyn_nxt2"],
+        "tra_nxt": ["k_tra_nxt"], "dyn_nxt": ["k_dyn_nxt"],
         "ldf_slp": ["k_slp_mxl", "k_slp"],
     }
     for n in names:
@@ -1081,8 +1081,7 @@ KERNEL_BYTES = {
     "k_ssh_nxt": lambda w, i, j, k, f: 3 * w * (i - 2) * (j - 2) * (k - 1) + 4 * 8 * i * j,   # + sshb emp_b emp ssha
     "k_wzv": _b(2),              # r hdivn, w wn
     "k_tra_nxt": _b(10),         # two tracers: r tsb tsn tsa, w tsb tsn
-    "k_dyn_nxt1": _b(4),         # r ua va, w ua va
-    "k_dyn_nxt2": _b(10),        # r ua va un vn ub vb, w un vn ub vb
+    "k_dyn_nxt": _b(12),         # r ua va un vn ub vb, w ua va un vn ub vb
 }
 
 if __name__ == "__main__":

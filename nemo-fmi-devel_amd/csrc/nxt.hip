@@ -32,11 +32,23 @@ __device__ __forceinline__ void lbc_targets(const DevDomain &d, int i, int j, F 
         }
 }
 
+// levels whose loads a closure kernel issues together, ahead of their stores:
+// the compiler moves no load across a store to an array that it cannot tell
+// apart, so a loop that loads and stores level by level waits for each level.
+// Horizontally uniform scale factors (E3U) are scalar loads (uld); as plain loads
+// they would be as many vector loads as the fields.  1024x1024x75 FP32, before
+// and after both: ssh_nxt 471 -> 246 us, div_hor 389 -> 244 us, with 942 MB
+// each to move.  (wzv, one load per level, gains nothing from it.)
+#define NXT_KB 8
+// (Scale factors that vary take registers of their own: half as many levels.)
+#define NXT_E3(p, ij, k) (E3U ? uld(p, (k) - 1) : E3(p, ij, k))
+
 // horizontal divergence at the interior point (i,j), DYN/divhor.F90:79-83.
-// The column's metrics are loaded once; at(k) evaluates one level with the
-// reference's operation order.
-template <typename T>
+// The column's metrics are loaded once; levels() evaluates NXT_KB levels from
+// k0 (the last one repeated beyond kmax) with the reference's operation order.
+template <typename T, bool E3U>
 struct HdivCol {
+    static constexpr int KB = E3U ? NXT_KB : NXT_KB / 2;
     double a1, a0, b1, b0, r;
     uint32_t ij;
     const T *un, *vn;
@@ -50,25 +62,35 @@ struct HdivCol {
         b0 = A2(m.e1v, i, j - 1);
         r = A2(m.r1_e1e2t, i, j);
     }
-    __device__ __forceinline__ double at(const DevDomain &d, int k) const
+    __device__ __forceinline__ void levels(const DevDomain &d, int k0, int kmax, T (&h)[KB]) const
     {
         const Metrics<double> &m = d.md;
-        const T *u = plane_ptr(un, d.n2, k), *v = plane_ptr(vn, d.n2, k);
-        return (a1 * E3(m.e3u, ij, k) * (double)ldp(u, ij) - a0 * E3(m.e3u, ij - 1, k) * (double)ldp(u, ij - 1) +
-                b1 * E3(m.e3v, ij, k) * (double)ldp(v, ij) -
-                b0 * E3(m.e3v, ij - (uint32_t)d.jpi, k) * (double)ldp(v, ij - (uint32_t)d.jpi)) *
-               r / E3(m.e3t, ij, k);
+        const uint32_t js = ij - (uint32_t)d.jpi;
+        T u1[KB], u0[KB], v1[KB], v0[KB];
+    #pragma unroll
+        for (int q = 0; q < KB; q++) {
+            const int k = min(k0 + q, kmax);
+            const T *u = plane_ptr(un, d.n2, k), *v = plane_ptr(vn, d.n2, k);
+            u1[q] = ldp(u, ij);
+            u0[q] = ldp(u, ij - 1u);
+            v1[q] = ldp(v, ij);
+            v0[q] = ldp(v, js);
+        }
+    #pragma unroll
+        for (int q = 0; q < KB; q++) {
+            const int k = min(k0 + q, kmax);
+            h[q] = (T)((a1 * NXT_E3(m.e3u, ij, k) * (double)u1[q] - a0 * NXT_E3(m.e3u, ij - 1u, k) * (double)u0[q] +
+                        b1 * NXT_E3(m.e3v, ij, k) * (double)v1[q] - b0 * NXT_E3(m.e3v, js, k) * (double)v0[q]) *
+                       r / NXT_E3(m.e3t, ij, k));
+        }
     }
 };
 
-// levels per thread of the per-cell closure kernels
-#define NXT_KB 8
-
 // ---------------------------------------------------------------------------
 // div_hor, DYN/divhor.F90:50-110: hdivn on levels 1..jpkm1 of the interior,
-// then lbc_lnk('T') of all jpk levels.  One thread per cell.
+// then lbc_lnk('T') of all jpk levels.  One thread per NXT_KB levels.
 // ---------------------------------------------------------------------------
-template <typename T>
+template <typename T, bool E3U>
 struct S_div_hor {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const T *__restrict__ un, const T *__restrict__ vn, T *__restrict__ hdivn)
@@ -79,25 +101,31 @@ struct S_div_hor {
         int si, sj;
         const bool ok = lbc_src(d, 'T', i, j, si, sj);
         const bool ring = si != i || sj != j || !ok;
-        const HdivCol<T> c(d, un, vn, ok ? si : 2, ok ? sj : 2);
+        const HdivCol<T, E3U> c(d, un, vn, ok ? si : 2, ok ? sj : 2);
         const uint32_t ij = IJ32(i, j);
+        constexpr int KB = HdivCol<T, E3U>::KB;
     #pragma unroll
-        for (int q = 0; q < NXT_KB; q++) {
-            const int k = k0 + q;
-            if (k > d.jpk) break;
-            T *h = plane_ptr(hdivn, d.n2, k);
-            if (k == d.jpk) {   // level jpk is not computed: lbc_lnk only
-                if (ring) stp(h, ij, ok ? ldp((const T *)h, c.ij) : T(0));
-            } else {
-                stp(h, ij, ok ? (T)c.at(d, k) : T(0));
+        for (int kb = k0; kb < k0 + NXT_KB; kb += KB) {
+            T hv[KB];
+            c.levels(d, min(kb, d.jpk), d.jpk, hv);
+    #pragma unroll
+            for (int q = 0; q < KB; q++) {
+                const int k = kb + q;
+                if (k > d.jpk) break;
+                T *h = plane_ptr(hdivn, d.n2, k);
+                if (k == d.jpk) {   // level jpk is not computed: lbc_lnk only
+                    if (ring) stp(h, ij, ok ? ldp((const T *)h, c.ij) : T(0));
+                } else {
+                    stp(h, ij, ok ? hv[q] : T(0));
+                }
             }
         }
     }
 };
-template <typename T>
+template <typename T, bool E3U>
 KERNEL void k_div_hor(DevDomain d, const T *__restrict__ un, const T *__restrict__ vn, T *__restrict__ hdivn)
 {
-    S_div_hor<T>::run(vb_hw(), d, un, vn, hdivn);
+    S_div_hor<T, E3U>::run(vb_hw(), d, un, vn, hdivn);
 }
 
 // ---------------------------------------------------------------------------
@@ -105,7 +133,7 @@ KERNEL void k_div_hor(DevDomain d, const T *__restrict__ un, const T *__restrict
 // depth-integrated divergence.  One thread per column: the column computes
 // its hdivn (at its lbc source point on the ring), the integral and ssha.
 // ---------------------------------------------------------------------------
-template <typename T>
+template <typename T, bool E3U>
 struct S_ssh_nxt {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
     __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double z2dt, double zcoef, const T *__restrict__ un, const T *__restrict__ vn, T *__restrict__ hdivn, const double *__restrict__ sshb, const double *__restrict__ emp_b, const double *__restrict__ emp, double *__restrict__ ssha)
@@ -115,24 +143,37 @@ struct S_ssh_nxt {
         int si, sj;
         const bool ok = lbc_src(d, 'T', i, j, si, sj);
         const uint32_t ij = IJ32(i, j);
-        const HdivCol<T> c(d, un, vn, ok ? si : 2, ok ? sj : 2);
+        const HdivCol<T, E3U> c(d, un, vn, ok ? si : 2, ok ? sj : 2);
+        constexpr int KB = HdivCol<T, E3U>::KB;
+        const int nlev = d.jpk - 1;
         double zhdiv = 0.0;
-    #pragma unroll 2
-        for (int k = 1; k <= d.jpk - 1; k++) {
-            const T h = ok ? (T)c.at(d, k) : T(0);
-            stp(plane_ptr(hdivn, d.n2, k), ij, h);
-            zhdiv = zhdiv + E3(d.md.e3t, ij, k) * (double)h;
+        for (int k0 = 1; k0 <= nlev; k0 += KB) {
+            T hv[KB];
+            double e3[E3U ? 1 : KB];
+            if constexpr (!E3U) {
+    #pragma unroll
+                for (int q = 0; q < KB; q++) e3[q] = E3(d.md.e3t, ij, min(k0 + q, nlev));
+            }
+            c.levels(d, k0, nlev, hv);
+    #pragma unroll
+            for (int q = 0; q < KB; q++) {
+                const int k = k0 + q;
+                if (k > nlev) break;
+                const T h = ok ? hv[q] : T(0);
+                stp(plane_ptr(hdivn, d.n2, k), ij, h);
+                zhdiv = zhdiv + (E3U ? uld(d.md.e3t, k - 1) : e3[E3U ? 0 : q]) * (double)h;
+            }
         }
         if (si != i || sj != j || !ok) A3(hdivn, i, j, d.jpk) = ok ? A3(hdivn, si, sj, d.jpk) : T(0);
         ssha[ij] = (sshb[ij] - z2dt * (zcoef * (emp_b[ij] + emp[ij]) + zhdiv)) * SSMASK(ij);
     }
 };
-template <typename T>
+template <typename T, bool E3U>
 KERNEL void k_ssh_nxt(DevDomain d, double z2dt, double zcoef, const T *__restrict__ un, const T *__restrict__ vn,
                       T *__restrict__ hdivn, const double *__restrict__ sshb, const double *__restrict__ emp_b,
                       const double *__restrict__ emp, double *__restrict__ ssha)
 {
-    S_ssh_nxt<T>::run(vb_hw(), d, z2dt, zcoef, un, vn, hdivn, sshb, emp_b, emp, ssha);
+    S_ssh_nxt<T, E3U>::run(vb_hw(), d, z2dt, zcoef, un, vn, hdivn, sshb, emp_b, emp, ssha);
 }
 
 // ---------------------------------------------------------------------------
@@ -248,150 +289,179 @@ KERNEL void k_tra_nxt(DevDomain d, int euler, double atfp, T *__restrict__ tsb, 
 }
 
 // ---------------------------------------------------------------------------
-// dyn_nxt, DYN/dynnxt.F90:66-377 (linear free surface), in two column
-// kernels.
-// Part 1 (lines 111-135): with dyn_spg_ts the baroclinic ua/va get the
-// barotropic after velocity (ua - depth mean + ua_b) on the interior, written
-// also to the ring points the lbc_lnk('U'/'V') of line 139 fills from them;
-// ring points without a source are zeroed.  Without ln_bt_fw, un/vn get the
-// advective barotropic velocity (lines 127-133), every column on itself.
+// dyn_nxt, DYN/dynnxt.F90:66-377 (linear free surface).  One thread per column
+// and component (grid.z: u, v):
+//   A  lines 111-135: with dyn_spg_ts the baroclinic ua gets the barotropic
+//      after velocity (ua - depth mean + ua_b); without ln_bt_fw, un the
+//      advective barotropic velocity;
+//   B  lines 147-176: Euler swap or Asselin filter and swap;
+//   C  lines 286-297: the forward time-splitting correction of ub, with the
+//      depth mean of the filtered column; then the barotropic now and before
+//      velocities (299-347).
+// Bound by HBM.  Each pass needs a depth sum of the pass before, and a column
+// of KMAX levels or fewer keeps ua, then the filtered ub, in registers between
+// them: 12 arrays move instead of 20 (1024x1024x75 FP32: 1442 us as two
+// kernels that read the columns again, 856 us).  KMAX = 0 reads them
+// again, for deeper columns.
+// lbc_lnk('U'/'V') of line 139: ring points without a source (closed sides) are
+// columns of zeros in the same launch; the ones with a source (cyclic sides)
+// follow in a launch of their own (RING), which reads the finished source.
 // ---------------------------------------------------------------------------
-template <typename T>
-struct S_dyn_nxt1 {
+template <typename T, int KMAX, bool E3U, bool RING>
+struct S_dyn_nxt {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, int spg_ts, int bt_fw, T *__restrict__ ua, T *__restrict__ va, T *__restrict__ un, T *__restrict__ vn, const double *__restrict__ ua_b, const double *__restrict__ va_b, const double *__restrict__ un_adv, const double *__restrict__ vn_adv, const double *__restrict__ un_b, const double *__restrict__ vn_b, const double *__restrict__ r1_hu, const double *__restrict__ r1_hv)
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, int spg_ts, int bt_fw, int euler, double atfp, T *ub_, T *vb, T *un_, T *vn, T *ua_, T *va, const double *__restrict__ ua_b_, const double *__restrict__ va_b, const double *__restrict__ un_adv, const double *__restrict__ vn_adv, double *__restrict__ ub_b_, double *__restrict__ vb_b, double *__restrict__ un_b_, double *__restrict__ vn_b, const double *__restrict__ r1_hu_, const double *__restrict__ r1_hv)
     {
-        THREAD_IJ_V(vb_, 1, 1);
-        if (i > d.jpi || j > d.jpj) return;
-        const Metrics<double> &m = d.md;
-        const uint32_t ij = IJ32(i, j);
-        const int jpk = d.jpk;
-        if (spg_ts && !bt_fw) {
-            const double cu = un_adv[ij] * r1_hu[ij], cv = vn_adv[ij] * r1_hv[ij];
-            for (int k = 1; k <= jpk - 1; k++) {
-                A3(un, i, j, k) = (T)(((double)A3(un, i, j, k) - cu + un_b[ij]) * UMASK(double, i, j, k));
-                A3(vn, i, j, k) = (T)(((double)A3(vn, i, j, k) - cv + vn_b[ij]) * VMASK(double, i, j, k));
-            }
+        int i, j;
+        if constexpr (RING) {
+            const int p = (int)(vb_.x * NH_BLOCK + threadIdx.y * blockDim.x + threadIdx.x), q = p - 2 * d.jpi;
+            i = q >= 0 ? ((q & 1) ? d.jpi : 1) : p < d.jpi ? p + 1 : p - d.jpi + 1;
+            j = q >= 0 ? 2 + q / 2 : p < d.jpi ? 1 : d.jpj;
+            if (q >= 0 && j > d.jpj - 1) return;
+        } else {
+            unsigned bx, by;
+            xcd_tile_v(vb_, bx, by);
+            i = (int)(bx * blockDim.x + threadIdx.x) + 1;
+            j = (int)(by * blockDim.y + threadIdx.y) + 1;
+            if (i > d.jpi || j > d.jpj) return;
         }
-        if (!is_interior(d, i, j)) {
-            int si, sj;
-            if (lbc_src(d, 'U', i, j, si, sj)) return;   // written by the thread of (si,sj)
-            for (int k = 1; k <= jpk; k++) {
-                A3(ua, i, j, k) = T(0);
-                A3(va, i, j, k) = T(0);
-            }
-            return;
-        }
-        double zue = 0.0, zve = 0.0;
-        if (spg_ts) {
-            zue = E3(m.e3u, ij, 1) * (double)A3(ua, i, j, 1) * UMASK(double, i, j, 1);
-            zve = E3(m.e3v, ij, 1) * (double)A3(va, i, j, 1) * VMASK(double, i, j, 1);
-    #pragma unroll 4
-            for (int k = 2; k <= jpk - 1; k++) {
-                zue = zue + E3(m.e3u, ij, k) * (double)A3(ua, i, j, k) * UMASK(double, i, j, k);
-                zve = zve + E3(m.e3v, ij, k) * (double)A3(va, i, j, k) * VMASK(double, i, j, k);
-            }
-            zue = zue * r1_hu[ij];
-            zve = zve * r1_hv[ij];
-        }
-    #pragma unroll 4
-        for (int k = 1; k <= jpk; k++) {
-            T a = A3(ua, i, j, k), b = A3(va, i, j, k);
-            if (spg_ts && k < jpk) {
-                a = (T)(((double)a - zue + ua_b[ij]) * UMASK(double, i, j, k));
-                b = (T)(((double)b - zve + va_b[ij]) * VMASK(double, i, j, k));
-                A3(ua, i, j, k) = a;
-                A3(va, i, j, k) = b;
-            }
-            lbc_targets(d, i, j, [&](int ti, int tj) {
-                A3(ua, ti, tj, k) = a;
-                A3(va, ti, tj, k) = b;
-            });
-        }
-    }
-};
-template <typename T>
-KERNEL void k_dyn_nxt1(DevDomain d, int spg_ts, int bt_fw, T *__restrict__ ua, T *__restrict__ va,
-                       T *__restrict__ un, T *__restrict__ vn, const double *__restrict__ ua_b,
-                       const double *__restrict__ va_b, const double *__restrict__ un_adv,
-                       const double *__restrict__ vn_adv, const double *__restrict__ un_b,
-                       const double *__restrict__ vn_b, const double *__restrict__ r1_hu, const double *__restrict__ r1_hv)
-{
-    S_dyn_nxt1<T>::run(vb_hw(), d, spg_ts, bt_fw, ua, va, un, vn, ua_b, va_b, un_adv, vn_adv, un_b, vn_b, r1_hu, r1_hv);
-}
+        int si, sj;
+        const bool ok = lbc_src(d, 'U', i, j, si, sj);
+        const bool ring = !is_interior(d, i, j);
+        if (RING != (ring && ok)) return;
+        const bool zero = !RING && ring;
+        const bool cv = vb_.z != 0;
+        T *__restrict__ ub = cv ? vb : ub_;
+        T *__restrict__ un = cv ? vn : un_;
+        T *__restrict__ ua = cv ? va : ua_;
+        const double *e3x = cv ? d.md.e3v : d.md.e3u;
+        const uint32_t ij = IJ32(i, j), src = RING ? IJ32(si, sj) : ij;
+        const uint32_t w = cv ? d.kvf[ij] : d.ktu[ij] >> 16;
+        const int m0 = (int)(w & 255u), m1 = (int)((w >> 8) & 255u);
+        const auto mask = [&](int k) { return k >= m0 && k <= m1 ? 1.0 : 0.0; };
+        const double r1h = (cv ? r1_hv : r1_hu_)[ij];
+        const double unb = (cv ? vn_b : un_b_)[ij];
+        const int nlev = d.jpk - 1;
+        constexpr int KB = NXT_KB, NB = KMAX ? KMAX / KB : 1;
+        static_assert(KMAX % KB == 0, "whole batches");
 
-// Part 2 (lines 147-176, 286-297, 299-347): Euler swap or Asselin filter and
-// swap on every column, the forward time-splitting correction of ub/vb, and
-// the barotropic now and before velocities.  Each column reads and writes
-// only itself.  The depth mean of part 1 multiplies by r1_hu once (zue *
-// r1_hu_a) exactly as lines 119-120 do, and the same holds for line 292.
-template <typename T>
-struct S_dyn_nxt2 {
-    static constexpr int NTHR = NH_BLOCK, WAVES = 1;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, int euler, int bt_fix, double atfp, T *__restrict__ ub, T *__restrict__ vb, T *__restrict__ un, T *__restrict__ vn, const T *__restrict__ ua, const T *__restrict__ va, double *__restrict__ ub_b, double *__restrict__ vb_b, double *__restrict__ un_b, double *__restrict__ vn_b, const double *__restrict__ r1_hu, const double *__restrict__ r1_hv)
-    {
-        THREAD_IJ_V(vb_, 1, 1);
-        if (i > d.jpi || j > d.jpj) return;
-        const Metrics<double> &m = d.md;
-        const uint32_t ij = IJ32(i, j);
-        const int jpkm1 = d.jpk - 1;
-        double sun = 0.0, svn = 0.0, sub = 0.0, svb = 0.0;   // depth sums of un, vn, ub, vb
-    #pragma unroll 2
-        for (int k = 1; k <= jpkm1; k++) {
-            const double a = (double)A3(ua, i, j, k), b = (double)A3(va, i, j, k);
-            const double e3u = E3(m.e3u, ij, k), e3v = E3(m.e3v, ij, k);
-            const double mu = UMASK(double, i, j, k), mv = VMASK(double, i, j, k);
-            double fu, fv;
-            if (euler) {
-                fu = (double)A3(ub, i, j, k);
-                fv = (double)A3(vb, i, j, k);
+        // level k0 + q (0-based, the last one repeated) of a column, KB at a time
+        const auto load = [&](const T *p, uint32_t c, int k0, T *v) {
+    #pragma unroll
+            for (int q = 0; q < KB; q++) v[q] = ldp(plane_ptr(p, d.n2, min(k0 + q, nlev - 1) + 1), c);
+        };
+        // A
+        T x[NB * KB];
+        double mean = 0.0;
+        const bool fix = spg_ts && !RING;
+        const auto sum_a = [&](int k0, const T *v) {
+    #pragma unroll
+            for (int q = 0; q < KB; q++) {
+                const int k = k0 + q + 1;
+                if (k > nlev) break;
+                const double t = NXT_E3(e3x, ij, k) * (double)v[q] * mask(k);
+                mean = k == 1 ? t : mean + t;
+            }
+        };
+        if constexpr (KMAX) {
+    #pragma unroll
+            for (int b = 0; b < NB; b++)
+                if (b * KB < nlev) load(ua, src, b * KB, x + b * KB);
+            if (fix) {
+    #pragma unroll
+                for (int b = 0; b < NB; b++)
+                    if (b * KB < nlev) sum_a(b * KB, x + b * KB);
+            }
+        } else if (fix) {
+            for (int k0 = 0; k0 < nlev; k0 += KB) {
+                load(ua, src, k0, x);
+                sum_a(k0, x);
+            }
+        }
+        mean = mean * r1h;
+        const double uab = fix ? (cv ? va_b : ua_b_)[ij] : 0.0;
+        const bool adv = spg_ts && !bt_fw, bt_fix = spg_ts && bt_fw && !euler;
+        const double cu_adv = adv ? (cv ? vn_adv : un_adv)[ij] * r1h : 0.0;
+
+        // B
+        double sn = 0.0, sb = 0.0;   // depth sums of un and ub
+        const auto filter = [&](int k0, T *v) {
+            T nv[KB], bv[KB];
+            load(un, ij, k0, nv);
+            load(ub, ij, k0, bv);
+    #pragma unroll
+            for (int q = 0; q < KB; q++) {
+                const int k = k0 + q + 1;
+                if (k > nlev) break;
+                const double mk = mask(k), e3 = NXT_E3(e3x, ij, k);
+                T a = v[q];
+                if (fix) a = (T)(((double)a - mean + uab) * mk);
+                if (zero) a = T(0);
+                if (spg_ts || RING || zero) stp(plane_ptr(ua, d.n2, k), ij, a);
+                T f = bv[q];
+                if (!euler) {
+                    const double n1 = adv ? (double)(T)(((double)nv[q] - cu_adv + unb) * mk) : (double)nv[q];
+                    f = (T)(n1 + atfp * ((double)bv[q] - 2.0 * n1 + (double)a));
+                    if (KMAX == 0 || !bt_fix) stp(plane_ptr(ub, d.n2, k), ij, f);
+                }
+                stp(plane_ptr(un, d.n2, k), ij, a);
+                v[q] = f;
+                const double tn = e3 * (double)a * mk, tb = e3 * (double)f * mk;
+                sn = k == 1 ? tn : sn + tn;
+                sb = k == 1 ? tb : sb + tb;
+            }
+        };
+        if constexpr (KMAX) {
+    #pragma unroll
+            for (int b = 0; b < NB; b++)
+                if (b * KB < nlev) filter(b * KB, x + b * KB);
+        } else {
+            for (int k0 = 0; k0 < nlev; k0 += KB) {
+                load(ua, src, k0, x);
+                filter(k0, x);
+            }
+        }
+        if (zero) A3(ua, i, j, d.jpk) = T(0);
+        if (RING) A3(ua, i, j, d.jpk) = A3(ua, si, sj, d.jpk);
+
+        // C
+        if (bt_fix) {
+            const double cu = sb * r1h - unb;
+            const auto correct = [&](int k0, const T *v) {
+    #pragma unroll
+                for (int q = 0; q < KB; q++) {
+                    const int k = k0 + q + 1;
+                    if (k > nlev) break;
+                    const double mk = mask(k);
+                    const T nb = (T)((double)v[q] - cu * mk);
+                    stp(plane_ptr(ub, d.n2, k), ij, nb);
+                    const double tb = NXT_E3(e3x, ij, k) * (double)nb * mk;
+                    sb = k == 1 ? tb : sb + tb;
+                }
+            };
+            if constexpr (KMAX) {
+    #pragma unroll
+                for (int b = 0; b < NB; b++)
+                    if (b * KB < nlev) correct(b * KB, x + b * KB);
             } else {
-                const double n1 = (double)A3(un, i, j, k), n2 = (double)A3(vn, i, j, k);
-                const T zuf = (T)(n1 + atfp * ((double)A3(ub, i, j, k) - 2.0 * n1 + a));
-                const T zvf = (T)(n2 + atfp * ((double)A3(vb, i, j, k) - 2.0 * n2 + b));
-                A3(ub, i, j, k) = zuf;
-                A3(vb, i, j, k) = zvf;
-                fu = (double)zuf;
-                fv = (double)zvf;
-            }
-            A3(un, i, j, k) = A3(ua, i, j, k);
-            A3(vn, i, j, k) = A3(va, i, j, k);
-            const double tu = e3u * (double)A3(ua, i, j, k) * mu, tv = e3v * (double)A3(va, i, j, k) * mv;
-            const double bu = e3u * fu * mu, bv = e3v * fv * mv;
-            sun = k == 1 ? tu : sun + tu;
-            svn = k == 1 ? tv : svn + tv;
-            sub = k == 1 ? bu : sub + bu;
-            svb = k == 1 ? bv : svb + bv;
-        }
-        if (!euler && bt_fix) {
-            // lines 286-297: the depth mean of ub/vb set to the input un_b/vn_b
-            const double cu = sub * r1_hu[ij] - un_b[ij], cv = svb * r1_hv[ij] - vn_b[ij];
-    #pragma unroll 4
-            for (int k = 1; k <= jpkm1; k++) {
-                const double e3u = E3(m.e3u, ij, k), e3v = E3(m.e3v, ij, k);
-                const double mu = UMASK(double, i, j, k), mv = VMASK(double, i, j, k);
-                const T nb = (T)((double)A3(ub, i, j, k) - cu * mu);
-                const T nv = (T)((double)A3(vb, i, j, k) - cv * mv);
-                A3(ub, i, j, k) = nb;
-                A3(vb, i, j, k) = nv;
-                const double bu = e3u * (double)nb * mu, bv = e3v * (double)nv * mv;
-                sub = k == 1 ? bu : sub + bu;
-                svb = k == 1 ? bv : svb + bv;
+                for (int k0 = 0; k0 < nlev; k0 += KB) {
+                    load(ub, ij, k0, x);
+                    correct(k0, x);
+                }
             }
         }
-        un_b[ij] = sun * r1_hu[ij];
-        vn_b[ij] = svn * r1_hv[ij];
-        ub_b[ij] = sub * r1_hu[ij];
-        vb_b[ij] = svb * r1_hv[ij];
+        (cv ? vn_b : un_b_)[ij] = sn * r1h;
+        (cv ? vb_b : ub_b_)[ij] = sb * r1h;
     }
 };
-template <typename T>
-KERNEL void k_dyn_nxt2(DevDomain d, int euler, int bt_fix, double atfp, T *__restrict__ ub, T *__restrict__ vb,
-                       T *__restrict__ un, T *__restrict__ vn, const T *__restrict__ ua, const T *__restrict__ va,
-                       double *__restrict__ ub_b, double *__restrict__ vb_b, double *__restrict__ un_b,
-                       double *__restrict__ vn_b, const double *__restrict__ r1_hu, const double *__restrict__ r1_hv)
+template <typename T, int KMAX, bool E3U, bool RING>
+KERNEL void k_dyn_nxt(DevDomain d, int spg_ts, int bt_fw, int euler, double atfp, T *ub, T *vb, T *un, T *vn, T *ua, T *va,
+                      const double *__restrict__ ua_b, const double *__restrict__ va_b,
+                      const double *__restrict__ un_adv, const double *__restrict__ vn_adv, double *__restrict__ ub_b,
+                      double *__restrict__ vb_b, double *__restrict__ un_b, double *__restrict__ vn_b,
+                      const double *__restrict__ r1_hu, const double *__restrict__ r1_hv)
 {
-    S_dyn_nxt2<T>::run(vb_hw(), d, euler, bt_fix, atfp, ub, vb, un, vn, ua, va, ub_b, vb_b, un_b, vn_b, r1_hu, r1_hv);
+    S_dyn_nxt<T, KMAX, E3U, RING>::run(vb_hw(), d, spg_ts, bt_fw, euler, atfp, ub, vb, un, vn, ua, va, ua_b, va_b, un_adv, vn_adv, ub_b, vb_b, un_b, vn_b, r1_hu, r1_hv);
 }
 
 // ---------------------------------------------------------------------------
@@ -403,7 +473,8 @@ int launch_div_hor(const T *un, const T *vn, T *hdivn)
     const DevDomain &d = nh::dom();
     Grid2 g = grid2(d.jpi, d.jpj);
     g.grid.z = (unsigned)((d.jpk + NXT_KB - 1) / NXT_KB);
-    LAUNCHB("div_hor", k_div_hor<T>, (S_div_hor<T>), g, d, un, vn, hdivn);
+    if (d.e3_sij == 0) LAUNCHB("div_hor", (k_div_hor<T, true>), (S_div_hor<T, true>), g, d, un, vn, hdivn);
+    else LAUNCHB("div_hor", (k_div_hor<T, false>), (S_div_hor<T, false>), g, d, un, vn, hdivn);
     return 0;
 }
 
@@ -413,7 +484,8 @@ int launch_ssh_nxt(double z2dt, double zcoef, const T *un, const T *vn, T *hdivn
 {
     const DevDomain &d = nh::dom();
     Grid2 g = grid2(d.jpi, d.jpj);
-    LAUNCHB("ssh_nxt", k_ssh_nxt<T>, (S_ssh_nxt<T>), g, d, z2dt, zcoef, un, vn, hdivn, sshb, emp_b, emp, ssha);
+    if (d.e3_sij == 0) LAUNCHB("ssh_nxt", (k_ssh_nxt<T, true>), (S_ssh_nxt<T, true>), g, d, z2dt, zcoef, un, vn, hdivn, sshb, emp_b, emp, ssha);
+    else LAUNCHB("ssh_nxt", (k_ssh_nxt<T, false>), (S_ssh_nxt<T, false>), g, d, z2dt, zcoef, un, vn, hdivn, sshb, emp_b, emp, ssha);
     return 0;
 }
 
@@ -450,11 +522,27 @@ int launch_dyn_nxt(int euler, T *ub, T *vb, T *un, T *vn, T *ua, T *va, const do
                    double *vn_b, const double *r1_hu, const double *r1_hv)
 {
     const DevDomain &d = nh::dom();
-    Grid2 g = grid2(d.jpi, d.jpj);
-    LAUNCHB("dyn_nxt", k_dyn_nxt1<T>, (S_dyn_nxt1<T>), g, d, d.ln_dynspg_ts, d.ln_bt_fw, ua, va, un, vn, ua_b, va_b, un_adv, vn_adv,
-           (const double *)un_b, (const double *)vn_b, r1_hu, r1_hv);
-    LAUNCHB("dyn_nxt", k_dyn_nxt2<T>, (S_dyn_nxt2<T>), g, d, euler, d.ln_dynspg_ts && d.ln_bt_fw, d.rn_atfp, ub, vb, un, vn,
-           (const T *)ua, (const T *)va, ub_b, vb_b, un_b, vn_b, r1_hu, r1_hv);
+    Grid2 g = grid2(d.jpi, d.jpj), gr = grid2(1, 1);
+    g.grid.z = gr.grid.z = 2;
+    gr.grid.x = (unsigned)((2 * (d.jpi + d.jpj) - 4 + NH_BLOCK - 1) / NH_BLOCK);
+#define NXT_LAUNCH3(KM, U, R, gg)                                                                                    \
+    LAUNCHB("dyn_nxt", (k_dyn_nxt<T, KM, U, R>), (S_dyn_nxt<T, KM, U, R>), gg, d, d.ln_dynspg_ts, d.ln_bt_fw, euler, \
+            d.rn_atfp, ub, vb, un, vn, ua, va, ua_b, va_b, un_adv, vn_adv, ub_b, vb_b, un_b, vn_b, r1_hu, r1_hv)
+#define NXT_LAUNCH2(KM)                                                                                   \
+    do {                                                                                                  \
+        if (d.e3_sij == 0) NXT_LAUNCH3(KM, true, false, g); else NXT_LAUNCH3(KM, false, false, g);         \
+        if (!d.iper && !d.jper) break;                                                                    \
+        if (d.e3_sij == 0) NXT_LAUNCH3(KM, true, true, gr); else NXT_LAUNCH3(KM, false, true, gr);         \
+    } while (0)
+    // levels kept in registers: as few as hold the column, for occupancy (in a
+    // plan the largest form, so that members of different depths share a launch)
+    const int nlev = d.jpk - 1;
+    if (nlev > 80) NXT_LAUNCH2(0);
+    else if (nlev > 48 || nh::planning()) NXT_LAUNCH2(80);
+    else if (nlev > 32) NXT_LAUNCH2(48);
+    else NXT_LAUNCH2(32);
+#undef NXT_LAUNCH2
+#undef NXT_LAUNCH3
     return 0;
 }
 
