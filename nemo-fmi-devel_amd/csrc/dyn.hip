@@ -45,10 +45,24 @@ __device__ __forceinline__ T keg_hw(const DevDomain &d, const T *un, const T *vn
     return r1_48 * (zv + zu);
 }
 
+// How the levels of a launch of nb workgroups per level chunk are shared out: the
+// whole column per workgroup where that gives every SIMD its waves (512
+// workgroups and more), else chunks of four levels or more towards 768 workgroups.
+// (32x22x31 FP64, five workgroups: k_step_dyn1 34 us in one chunk, 17 us
+// with its sums.)  In a plan the members fill the chip together.
+inline int lev_chunks(unsigned nb, int nlev)
+{
+    if (nh::planning() || nb >= 512u || nb == 0u) return nlev;
+    int n = (int)(768u / nb);
+    n = n > nlev / 4 ? nlev / 4 : n;
+    return n < 1 ? nlev : (nlev + n - 1) / n;
+}
+
+// One thread per column and chunk of kch levels (grid.z).
 template <typename T>
 struct S_dyn_keg_zad {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, int do_keg, int kscheme, int do_zad, const T * __restrict__ un, const T * __restrict__ vn, const T * __restrict__ wn, T * __restrict__ ua, T * __restrict__ va)
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, int do_keg, int kscheme, int do_zad, const T * __restrict__ un, const T * __restrict__ vn, const T * __restrict__ wn, T * __restrict__ ua, T * __restrict__ va, int kch)
     {
         THREAD_IJ_V(vb_, 2, 2);
         if (i > d.jpi - 1 || j > d.jpj - 1) return;
@@ -56,8 +70,20 @@ struct S_dyn_keg_zad {
         const size_t ij = IJ(i, j);
         const T e1u = m.e1u[ij], e2v = m.e2v[ij], r1_e1e2u = m.r1_e1e2u[ij], r1_e1e2v = m.r1_e1e2v[ij];
         const T e1e2t = m.e1e2t[ij], e1e2t_e = m.e1e2t[IJ(i + 1, j)], e1e2t_n = m.e1e2t[IJ(i, j + 1)];
-        T zwuw_k = T(0), zwvw_k = T(0);    // surface flux zero, dynzad.F90:93-94
-        for (int k = 1; k <= d.jpk - 1; k++) {
+        const int ka = (int)vb_.z * kch + 1, kb = min(ka + kch - 1, d.jpk - 1);
+        // dynzad's fluxes at w-level kk (zero at the surface, dynzad.F90:93-94)
+        const auto wflux = [&](int kk, T &cu, T &cv) {
+            cu = cv = T(0);
+            if (kk == 1 || kk > d.jpk - 1) return;
+            const T zww = T(0.25) * e1e2t * A3(wn, i, j, kk);
+            const T zww_e = T(0.25) * e1e2t_e * A3(wn, i + 1, j, kk);
+            const T zww_n = T(0.25) * e1e2t_n * A3(wn, i, j + 1, kk);
+            cu = (zww_e + zww) * (A3(un, i, j, kk - 1) - A3(un, i, j, kk));
+            cv = (zww_n + zww) * (A3(vn, i, j, kk - 1) - A3(vn, i, j, kk));
+        };
+        T zwuw_k = T(0), zwvw_k = T(0);
+        if (do_zad) wflux(ka, zwuw_k, zwvw_k);
+        for (int k = ka; k <= kb; k++) {
             const size_t p = IJK(i, j, k);
             T a = ua[p], b = va[p];
             if (do_keg) {
@@ -75,15 +101,8 @@ struct S_dyn_keg_zad {
                 b = b - (hn - h) / e2v;
             }
             if (do_zad) {
-                T zwuw_kp1 = T(0), zwvw_kp1 = T(0);
-                if (k + 1 <= d.jpk - 1) {
-                    const int kk = k + 1;
-                    const T zww = T(0.25) * e1e2t * A3(wn, i, j, kk);
-                    const T zww_e = T(0.25) * e1e2t_e * A3(wn, i + 1, j, kk);
-                    const T zww_n = T(0.25) * e1e2t_n * A3(wn, i, j + 1, kk);
-                    zwuw_kp1 = (zww_e + zww) * (A3(un, i, j, kk - 1) - A3(un, i, j, kk));
-                    zwvw_kp1 = (zww_n + zww) * (A3(vn, i, j, kk - 1) - A3(vn, i, j, kk));
-                }
+                T zwuw_kp1, zwvw_kp1;
+                wflux(k + 1, zwuw_kp1, zwvw_kp1);
                 a = a - (zwuw_k + zwuw_kp1) * r1_e1e2u / E3(m.e3u, ij, k);
                 b = b - (zwvw_k + zwvw_kp1) * r1_e1e2v / E3(m.e3v, ij, k);
                 zwuw_k = zwuw_kp1;
@@ -96,9 +115,9 @@ struct S_dyn_keg_zad {
 };
 template <typename T>
 KERNEL void k_dyn_keg_zad(DevDomain d, int do_keg, int kscheme, int do_zad, const T * __restrict__ un, const T * __restrict__ vn, const T * __restrict__ wn,
-                              T * __restrict__ ua, T * __restrict__ va)
+                              T * __restrict__ ua, T * __restrict__ va, int kch)
 {
-    S_dyn_keg_zad<T>::run(vb_hw(), d, do_keg, kscheme, do_zad, un, vn, wn, ua, va);
+    S_dyn_keg_zad<T>::run(vb_hw(), d, do_keg, kscheme, do_zad, un, vn, wn, ua, va, kch);
 }
 
 // ---------------------------------------------------------------------------
@@ -193,7 +212,9 @@ int launch_dyn_adv(int which, int kscheme, const T *un, const T *vn, const T *wn
         LAUNCHB("dyn_adv_cen2", k_dyn_adv_cen2<T>, (S_dyn_adv_cen2<T>), g, d, un, vn, wn, ua, va);
     } else {
         const char *nm = which == 1 ? "dyn_keg" : which == 2 ? "dyn_zad" : "dyn_adv";
-        LAUNCHB(nm, k_dyn_keg_zad<T>, (S_dyn_keg_zad<T>), g, d, (which & 1), kscheme, (which & 2) ? 1 : 0, un, vn, wn, ua, va);
+        const int kch = lev_chunks(g.grid.x * g.grid.y, d.jpk - 1);
+        g.grid.z = (unsigned)((d.jpk - 1 + kch - 1) / kch);
+        LAUNCHB(nm, k_dyn_keg_zad<T>, (S_dyn_keg_zad<T>), g, d, (which & 1), kscheme, (which & 2) ? 1 : 0, un, vn, wn, ua, va, kch);
     }
     return 0;
 }
@@ -228,40 +249,127 @@ __device__ __forceinline__ T fvor(const DevDomain &d, int kvor, const T *pu, con
                (A3(pu, p, q + 1, k) + A3(pu, p, q, k)) * m.dj_e1u_2e1e2f[pq];
     }
 }
-// vor_een's zwz: vorticity times 1/e3f, DYN/dynvor.F90:580-643
+// zwz of the ENT scheme (relative vorticity) after lbc_lnk('F')
 template <typename T>
-__device__ __forceinline__ T fvor_een(const DevDomain &d, int kvor, const T *pu, const T *pv, int p, int q, int k)
-{
-    const Metrics<T> &m = met<T>(d);
-    const size_t pq = IJ(p, q);
-    const T t1 = TMASK(T, p, q + 1, k), t2 = TMASK(T, p + 1, q + 1, k), t3 = TMASK(T, p, q, k), t4 = TMASK(T, p + 1, q, k);
-    const T ze3f = E3(m.e3t, IJ(p, q + 1), k) * t1 + E3(m.e3t, IJ(p + 1, q + 1), k) * t2 + E3(m.e3t, pq, k) * t3 +
-                   E3(m.e3t, IJ(p + 1, q), k) * t4;
-    T z1;
-    if (ze3f != T(0)) z1 = (d.nn_een_e3f == 0 ? T(4) : (t1 + t2 + t3 + t4)) / ze3f;
-    else z1 = T(0);
-    switch (kvor) {
-    case np_COR: return m.ff_f[pq] * z1;
-    case np_RVO: return curl_f(d, pu, pv, p, q, k) * m.r1_e1e2f[pq] * z1;
-    case np_MET:
-        return ((A3(pv, p + 1, q, k) + A3(pv, p, q, k)) * m.di_e2v_2e1e2f[pq] -
-                (A3(pu, p, q + 1, k) + A3(pu, p, q, k)) * m.dj_e1u_2e1e2f[pq]) * z1;
-    case np_CRV: return (m.ff_f[pq] + curl_f(d, pu, pv, p, q, k) * m.r1_e1e2f[pq]) * z1;
-    default:
-        return (m.ff_f[pq] + (A3(pv, p + 1, q, k) + A3(pv, p, q, k)) * m.di_e2v_2e1e2f[pq] -
-                (A3(pu, p, q + 1, k) + A3(pu, p, q, k)) * m.dj_e1u_2e1e2f[pq]) * z1;
-    }
-}
-// zwz after lbc_lnk('F') for the EEN/EET/ENT schemes
-template <typename T>
-__device__ __forceinline__ T zwz_f(const DevDomain &d, int scheme, int kvor, const T *pu, const T *pv, int p, int q, int k)
+__device__ __forceinline__ T zwz_ent(const DevDomain &d, const T *pu, const T *pv, int p, int q, int k)
 {
     int sp, sq;
     if (!lbc_src(d, 'F', p, q, sp, sq)) return T(0);
-    if (scheme == NEMO_NP_EEN) return fvor_een(d, kvor, pu, pv, sp, sq, k);
-    if (scheme == NEMO_NP_ENT) return curl_f(d, pu, pv, sp, sq, k) * met<T>(d).r1_e1e2f[IJ(sp, sq)];
-    return fvor(d, kvor, pu, pv, sp, sq, k);
+    return curl_f(d, pu, pv, sp, sq, k) * met<T>(d).r1_e1e2f[IJ(sp, sq)];
 }
+
+// zwz of the EEN and EET schemes after lbc_lnk('F') (vorticity, for EEN times
+// 1/e3f: DYN/dynvor.F90:580-643, 700-760) at the f-points around a workgroup's
+// 64 x 4 cells, one level at a time, in LDS.  A cell needs eight of them, each
+// with a division, four masks and eight loads: evaluated by every cell they took
+// 256 registers (one wave per SIMD) and eight times the work; here 1.55 times,
+// with the columns' metrics and masks in registers and the next level's
+// velocities in flight.  362x149x46 FP64 in k_step_dyn1: 333 us, 97 us;
+// 182x149x31 FP32 in k_dyn_vor: 226 us, 17.5 us (both with the levels shared
+// out over workgroups, lev_chunks).
+template <typename T, int SCHEME, int KVOR>
+struct ZwzTile {
+    static constexpr int TX = 64, W = TX + 2, H = NH_BLOCK / TX + 2, NR = (W * H + NH_BLOCK - 1) / NH_BLOCK;
+    static constexpr bool CURL = KVOR == np_RVO || KVOR == np_CRV, FF = KVOR == np_COR || KVOR == np_CRV || KVOR == np_CME;
+    static constexpr bool EEN = SCHEME == NEMO_NP_EEN;
+    typedef T Lds[2][H][W];
+    uint32_t pq[NR], t1[NR], t2[NR], t3[NR], t4[NR];
+    T ff[NR], ve[NR], vc[NR], un[NR], uc[NR], r1f[NR];   // f; curl: e2v, e1u; else di, dj in ve, un
+    T u0[NR], u1[NR], v0[NR], v1[NR];                    // the velocities of the next level
+    bool ok[NR];
+
+    __device__ __forceinline__ static int tid() { return (int)(threadIdx.y * TX + threadIdx.x); }
+    // (i0, j0): the workgroup's first cell
+    __device__ __forceinline__ ZwzTile(const DevDomain &d, int i0, int j0)
+    {
+        const Metrics<T> &m = met<T>(d);
+        const uint32_t w = (uint32_t)d.jpi;
+    #pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const int n = tid() + r * NH_BLOCK, p = i0 - 1 + n % W, q = j0 - 1 + n / W;
+            int sp = 2, sq = 2;
+            ok[r] = n < W * H && p >= 1 && p <= d.jpi && q >= 1 && q <= d.jpj && lbc_src(d, 'F', p, q, sp, sq);
+            const uint32_t c = ok[r] ? IJ32(sp, sq) : IJ32(2, 2);
+            pq[r] = c;
+            if (EEN) {
+                t1[r] = d.ktu[c + w]; t2[r] = d.ktu[c + w + 1u]; t3[r] = d.ktu[c]; t4[r] = d.ktu[c + 1u];
+            }
+            if (FF) ff[r] = m.ff_f[c];
+            if (CURL) {
+                ve[r] = m.e2v[c + 1u]; vc[r] = m.e2v[c]; un[r] = m.e1u[c + w]; uc[r] = m.e1u[c];
+                r1f[r] = m.r1_e1e2f[c];
+            } else if (KVOR != np_COR) {
+                ve[r] = m.di_e2v_2e1e2f[c]; un[r] = m.dj_e1u_2e1e2f[c];
+            }
+        }
+    }
+    // the deepest wet level around the workgroup's f-points (EEN: zwz is zero
+    // below); s: a word of LDS.  Ends with a barrier.
+    __device__ __forceinline__ int bottom(int *s) const
+    {
+        if (tid() == 0) *s = 0;
+        __syncthreads();
+        int k = 0;
+    #pragma unroll
+        for (int r = 0; r < NR; r++)
+            if (ok[r]) k = max(k, (int)max(max((t1[r] >> 8) & 255u, (t2[r] >> 8) & 255u), max((t3[r] >> 8) & 255u, (t4[r] >> 8) & 255u)));
+        atomicMax(s, k);
+        __syncthreads();
+        return *s;
+    }
+    __device__ __forceinline__ void fetch(const DevDomain &d, const T *pu, const T *pv, int k)
+    {
+        if (KVOR == np_COR) return;
+        const T *u = plane_ptr(pu, d.n2, k), *v = plane_ptr(pv, d.n2, k);
+    #pragma unroll
+        for (int r = 0; r < NR; r++) {
+            u0[r] = ldp(u, pq[r]); u1[r] = ldp(u, pq[r] + (uint32_t)d.jpi);
+            v0[r] = ldp(v, pq[r]); v1[r] = ldp(v, pq[r] + 1u);
+        }
+    }
+    __device__ __forceinline__ T vor(int r) const
+    {
+        if (KVOR == np_COR) return ff[r];
+        if (CURL) {
+            const T c = ve[r] * v1[r] - vc[r] * v0[r] - un[r] * u1[r] + uc[r] * u0[r];
+            return KVOR == np_RVO ? c * r1f[r] : ff[r] + c * r1f[r];
+        }
+        if (KVOR == np_MET) return (v1[r] + v0[r]) * ve[r] - (u1[r] + u0[r]) * un[r];
+        return ff[r] + (v1[r] + v0[r]) * ve[r] - (u1[r] + u0[r]) * un[r];
+    }
+    // level k from the fetched velocities
+    __device__ __forceinline__ void put(const DevDomain &d, int k, Lds &z) const
+    {
+        const T *e3t = met<T>(d).e3t;
+        const bool uni = d.e3_sij == 0;
+        const uint32_t w = (uint32_t)d.jpi;
+    #pragma unroll
+        for (int r = 0; r < NR; r++) {
+            T x = T(0);
+            if constexpr (EEN) {
+                const auto in = [&](uint32_t t) { return k >= (int)(t & 255u) && k <= (int)((t >> 8) & 255u) ? T(1) : T(0); };
+                const T m1 = in(t1[r]), m2 = in(t2[r]), m3 = in(t3[r]), m4 = in(t4[r]), n = m1 + m2 + m3 + m4;
+                if (ok[r] && n != T(0)) {
+                    T ze3f;
+                    if (uni) {
+                        const T e = uld(e3t, k - 1);
+                        ze3f = e * m1 + e * m2 + e * m3 + e * m4;
+                    } else {
+                        ze3f = E3(e3t, pq[r] + w, k) * m1 + E3(e3t, pq[r] + w + 1u, k) * m2 + E3(e3t, pq[r], k) * m3 +
+                               E3(e3t, pq[r] + 1u, k) * m4;
+                    }
+                    T z1 = T(0);
+                    if (ze3f != T(0)) z1 = (d.nn_een_e3f == 0 ? T(4) : n) / ze3f;
+                    x = vor(r) * z1;
+                }
+            } else {
+                if (ok[r]) x = vor(r);
+            }
+            const int q = tid() + r * NH_BLOCK;
+            if (q < W * H) z[k & 1][q / W][q % W] = x;
+        }
+    }
+};
 
 template <typename T>
 __device__ __forceinline__ void vor_ene_pt(const DevDomain &d, int kvor, const T *pu, const T *pv, int i, int j, int k,
@@ -295,18 +403,32 @@ __device__ __forceinline__ void vor_ens_pt(const DevDomain &d, int kvor, const T
     a = a + zuav * (z_s + z_c);
     b = b + zvau * (z_w + z_c);
 }
-// EEN (use_e3f) and EET: triads of f-point vorticity around t-points
+// EEN (use_e3f) and EET: triads of f-point vorticity around t-points.  The
+// metrics of a cell's four u- and four v-points stay in registers: loaded in the
+// level loop they would be loads again, since the kernel stores.
 template <typename T>
-__device__ __forceinline__ void vor_een_pt(const DevDomain &d, int scheme, int kvor, const T *pu, const T *pv, int i,
-                                           int j, int k, T &a, T &b)
+struct EenCol {
+    T yc, ye, ys, yse, xw, xnw, xc, xn, ru, rv;
+    __device__ __forceinline__ EenCol(const DevDomain &d, uint32_t c)
+    {
+        const Metrics<T> &m = met<T>(d);
+        const uint32_t w = (uint32_t)d.jpi;
+        yc = m.e1v[c]; ye = m.e1v[c + 1u]; ys = m.e1v[c - w]; yse = m.e1v[c - w + 1u];
+        xw = m.e2u[c - 1u]; xnw = m.e2u[c + w - 1u]; xc = m.e2u[c]; xn = m.e2u[c + w];
+        const T r1_12 = T(1) / T(12);
+        ru = r1_12 * m.r1_e1u[c];
+        rv = r1_12 * m.r1_e2v[c];
+    }
+};
+// (x, y): the cell within the workgroup; z: the level's f-points (ZwzTile)
+template <typename T, int SCHEME, int W>
+__device__ __forceinline__ void vor_een_pt(const DevDomain &d, const EenCol<T> &e, const T (*z)[W], int x, int y,
+                                           const T *pu, const T *pv, uint32_t c, int k, T &a, T &b)
 {
     const Metrics<T> &m = met<T>(d);
-    // zwz(i-1..i+1, j-1..j+1) except (i+1,j+1)
-    T z[3][3];
-    for (int dj = -1; dj <= 1; dj++)
-        for (int di = -1; di <= 1; di++)
-            z[dj + 1][di + 1] = (di == 1 && dj == 1) ? T(0) : zwz_f(d, scheme, kvor, pu, pv, i + di, j + dj, k);
-#define ZW(di, dj) z[(dj) + 1][(di) + 1]
+    const uint32_t w = (uint32_t)d.jpi;
+    const T *u = plane_ptr(pu, d.n2, k), *v = plane_ptr(pv, d.n2, k);
+#define ZW(di, dj) z[y + (dj) + 1][x + (di) + 1]
     // triads at t-point (i+oi, j+oj)
     auto tne = [&](int oi, int oj) { return ZW(oi - 1, oj) + ZW(oi, oj) + ZW(oi, oj - 1); };
     auto tnw = [&](int oi, int oj) { return ZW(oi - 1, oj - 1) + ZW(oi - 1, oj) + ZW(oi, oj); };
@@ -314,20 +436,17 @@ __device__ __forceinline__ void vor_een_pt(const DevDomain &d, int scheme, int k
     auto tsw = [&](int oi, int oj) { return ZW(oi, oj - 1) + ZW(oi - 1, oj - 1) + ZW(oi - 1, oj); };
     T ne00 = tne(0, 0), nw10 = tnw(1, 0), se00 = tse(0, 0), sw10 = tsw(1, 0);
     T sw01 = tsw(0, 1), se01 = tse(0, 1), nw00 = tnw(0, 0);
-    if (scheme == NEMO_NP_EET) {
-        const T z00 = T(1) / E3(m.e3t, IJ(i, j), k), z10 = T(1) / E3(m.e3t, IJ(i + 1, j), k),
-                z01 = T(1) / E3(m.e3t, IJ(i, j + 1), k);
+    if (SCHEME == NEMO_NP_EET) {
+        const T z00 = T(1) / E3(m.e3t, c, k), z10 = T(1) / E3(m.e3t, c + 1u, k), z01 = T(1) / E3(m.e3t, c + w, k);
         ne00 = ne00 * z00; nw10 = nw10 * z10; se00 = se00 * z00; sw10 = sw10 * z10;
         sw01 = sw01 * z01; se01 = se01 * z01; nw00 = nw00 * z00;
     }
 #undef ZW
-    auto zwx = [&](int p, int q) { return m.e2u[IJ(p, q)] * E3(m.e3u, IJ(p, q), k) * A3(pu, p, q, k); };
-    auto zwy = [&](int p, int q) { return m.e1v[IJ(p, q)] * E3(m.e3v, IJ(p, q), k) * A3(pv, p, q, k); };
-    const T r1_12 = T(1) / T(12);
-    const T zua = r1_12 * m.r1_e1u[IJ(i, j)] *
-                  (ne00 * zwy(i, j) + nw10 * zwy(i + 1, j) + se00 * zwy(i, j - 1) + sw10 * zwy(i + 1, j - 1));
-    const T zva = -(r1_12 * m.r1_e2v[IJ(i, j)] *
-                    (sw01 * zwx(i - 1, j + 1) + se01 * zwx(i, j + 1) + nw00 * zwx(i - 1, j) + ne00 * zwx(i, j)));
+    const bool uni = d.e3_sij == 0;
+    const auto zwx = [&](T e2u, uint32_t q) { return e2u * (uni ? uld(m.e3u, k - 1) : E3(m.e3u, q, k)) * ldp(u, q); };
+    const auto zwy = [&](T e1v, uint32_t q) { return e1v * (uni ? uld(m.e3v, k - 1) : E3(m.e3v, q, k)) * ldp(v, q); };
+    const T zua = e.ru * (ne00 * zwy(e.yc, c) + nw10 * zwy(e.ye, c + 1u) + se00 * zwy(e.ys, c - w) + sw10 * zwy(e.yse, c - w + 1u));
+    const T zva = -(e.rv * (sw01 * zwx(e.xnw, c + w - 1u) + se01 * zwx(e.xn, c + w) + nw00 * zwx(e.xw, c - 1u) + ne00 * zwx(e.xc, c)));
     a = a + zua;
     b = b + zva;
 }
@@ -342,16 +461,16 @@ __device__ __forceinline__ T ent_zwt(const DevDomain &d, int kvor, const T *pu, 
     switch (kvor) {
     case np_COR: return m.ff_t[pq] * m.e1e2t[pq] * e3t;
     case np_RVO: {
-        const T s = zwz_f(d, NEMO_NP_ENT, kvor, pu, pv, p - 1, q, k) + zwz_f(d, NEMO_NP_ENT, kvor, pu, pv, p, q, k) +
-                    zwz_f(d, NEMO_NP_ENT, kvor, pu, pv, p - 1, q - 1, k) + zwz_f(d, NEMO_NP_ENT, kvor, pu, pv, p, q - 1, k);
+        const T s = zwz_ent(d, pu, pv, p - 1, q, k) + zwz_ent(d, pu, pv, p, q, k) +
+                    zwz_ent(d, pu, pv, p - 1, q - 1, k) + zwz_ent(d, pu, pv, p, q - 1, k);
         return r1_4 * s * m.e1e2t[pq] * e3t;
     }
     case np_MET:
         return ((A3(pv, p, q, k) + A3(pv, p, q - 1, k)) * m.di_e2u_2[pq] -
                 (A3(pu, p, q, k) + A3(pu, p - 1, q, k)) * m.dj_e1v_2[pq]) * e3t;
     case np_CRV: {
-        const T s = zwz_f(d, NEMO_NP_ENT, kvor, pu, pv, p - 1, q, k) + zwz_f(d, NEMO_NP_ENT, kvor, pu, pv, p, q, k) +
-                    zwz_f(d, NEMO_NP_ENT, kvor, pu, pv, p - 1, q - 1, k) + zwz_f(d, NEMO_NP_ENT, kvor, pu, pv, p, q - 1, k);
+        const T s = zwz_ent(d, pu, pv, p - 1, q, k) + zwz_ent(d, pu, pv, p, q, k) +
+                    zwz_ent(d, pu, pv, p - 1, q - 1, k) + zwz_ent(d, pu, pv, p, q - 1, k);
         return (m.ff_t[pq] + r1_4 * s) * m.e1e2t[pq] * e3t;
     }
     default:
@@ -376,52 +495,80 @@ __device__ __forceinline__ void vor_ent_pt(const DevDomain &d, int kvor, const T
 // The scheme and the vorticity kinds are template parameters: each
 // instantiation carries only its own stencil, which keeps register use (and so
 // occupancy) at what that scheme needs.
+// One thread per column and chunk of kch levels (grid.z, lev_chunks).
 template <typename T, int SCHEME, int NCOR, int NRVM, int NTOT>
 struct S_dyn_vor {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const T * __restrict__ un, const T * __restrict__ vn, T * __restrict__ ua, T * __restrict__ va)
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const T * __restrict__ un, const T * __restrict__ vn, T * __restrict__ ua, T * __restrict__ va, int kch)
     {
         THREAD_IJ_V(vb_, 2, 2);
-        if (i > d.jpi - 1 || j > d.jpj - 1) return;
-        for (int k = 1; k <= d.jpk - 1; k++) {
-            const size_t p = IJK(i, j, k);
-            T a = ua[p], b = va[p];
-            switch (SCHEME) {
-            case NEMO_NP_ENE: vor_ene_pt(d, NTOT, un, vn, i, j, k, a, b); break;
-            case NEMO_NP_ENS: vor_ens_pt(d, NTOT, un, vn, i, j, k, a, b); break;
-            case NEMO_NP_MIX:
-                vor_ens_pt(d, NRVM, un, vn, i, j, k, a, b);
-                vor_ene_pt(d, NCOR, un, vn, i, j, k, a, b);
-                break;
-            case NEMO_NP_ENT: vor_ent_pt(d, NTOT, un, vn, i, j, k, a, b); break;
-            default: vor_een_pt(d, SCHEME, NTOT, un, vn, i, j, k, a, b); break;
+        const bool on = i <= d.jpi - 1 && j <= d.jpj - 1;
+        const int ka = (int)vb_.z * kch + 1;
+        int kb = min(ka + kch - 1, d.jpk - 1);
+        if constexpr (SCHEME == NEMO_NP_EEN || SCHEME == NEMO_NP_EET) {
+            typedef ZwzTile<T, SCHEME, NTOT> Z;
+            __shared__ typename Z::Lds z;
+            __shared__ int s_bot;
+            Z f(d, (int)(bx_ * Z::TX) + 2, (int)(by_ * (Z::H - 2)) + 2);
+            if (Z::EEN) kb = min(kb, f.bottom(&s_bot));   // below, the trend is zero
+            if (kb < ka) return;
+            const uint32_t c = on ? IJ32(i, j) : IJ32(2, 2);
+            const EenCol<T> e(d, c);
+            f.fetch(d, un, vn, ka);
+            for (int k = ka; k <= kb; k++) {
+                f.put(d, k, z);
+                f.fetch(d, un, vn, min(k + 1, kb));
+                __syncthreads();
+                if (!on) continue;
+                T *pa = plane_ptr(ua, d.n2, k), *pb = plane_ptr(va, d.n2, k);
+                T a = ldp((const T *)pa, c), b = ldp((const T *)pb, c);
+                vor_een_pt<T, SCHEME, Z::W>(d, e, z[k & 1], (int)threadIdx.x, (int)threadIdx.y, un, vn, c, k, a, b);
+                stp(pa, c, a);
+                stp(pb, c, b);
             }
-            ua[p] = a;
-            va[p] = b;
+        } else {
+            if (!on) return;
+            for (int k = ka; k <= kb; k++) {
+                const size_t p = IJK(i, j, k);
+                T a = ua[p], b = va[p];
+                switch (SCHEME) {
+                case NEMO_NP_ENE: vor_ene_pt(d, NTOT, un, vn, i, j, k, a, b); break;
+                case NEMO_NP_ENS: vor_ens_pt(d, NTOT, un, vn, i, j, k, a, b); break;
+                case NEMO_NP_MIX:
+                    vor_ens_pt(d, NRVM, un, vn, i, j, k, a, b);
+                    vor_ene_pt(d, NCOR, un, vn, i, j, k, a, b);
+                    break;
+                default: vor_ent_pt(d, NTOT, un, vn, i, j, k, a, b); break;
+                }
+                ua[p] = a;
+                va[p] = b;
+            }
         }
     }
 };
 template <typename T, int SCHEME, int NCOR, int NRVM, int NTOT>
 KERNEL void k_dyn_vor(DevDomain d, const T * __restrict__ un, const T * __restrict__ vn, T * __restrict__ ua,
-                      T * __restrict__ va)
+                      T * __restrict__ va, int kch)
 {
-    S_dyn_vor<T, SCHEME, NCOR, NRVM, NTOT>::run(vb_hw(), d, un, vn, ua, va);
+    S_dyn_vor<T, SCHEME, NCOR, NRVM, NTOT>::run(vb_hw(), d, un, vn, ua, va, kch);
 }
 
 template <typename T, int SCHEME>
 static int launch_dyn_vor_s(const DevDomain &d, const T *un, const T *vn, T *ua, T *va)
 {
     Grid2 g = grid2(d.jpi - 2, d.jpj - 2);
+    const int kch = lev_chunks(g.grid.x * g.grid.y, d.jpk - 1);
+    g.grid.z = (unsigned)((d.jpk - 1 + kch - 1) / kch);
     // (nrvm, ntot) from the momentum advection form, DYN/dynvor.F90:903-939
     switch (d.n_dynadv) {
     case NEMO_NP_LIN_DYN:
-        LAUNCHB("dyn_vor", (k_dyn_vor<T, SCHEME, np_COR, np_COR, np_COR>), (S_dyn_vor<T, SCHEME, np_COR, np_COR, np_COR>), g, d, un, vn, ua, va);
+        LAUNCHB("dyn_vor", (k_dyn_vor<T, SCHEME, np_COR, np_COR, np_COR>), (S_dyn_vor<T, SCHEME, np_COR, np_COR, np_COR>), g, d, un, vn, ua, va, kch);
         break;
     case NEMO_NP_VEC_C2:
-        LAUNCHB("dyn_vor", (k_dyn_vor<T, SCHEME, np_COR, np_RVO, np_CRV>), (S_dyn_vor<T, SCHEME, np_COR, np_RVO, np_CRV>), g, d, un, vn, ua, va);
+        LAUNCHB("dyn_vor", (k_dyn_vor<T, SCHEME, np_COR, np_RVO, np_CRV>), (S_dyn_vor<T, SCHEME, np_COR, np_RVO, np_CRV>), g, d, un, vn, ua, va, kch);
         break;
     default:
-        LAUNCHB("dyn_vor", (k_dyn_vor<T, SCHEME, np_COR, np_MET, np_CME>), (S_dyn_vor<T, SCHEME, np_COR, np_MET, np_CME>), g, d, un, vn, ua, va);
+        LAUNCHB("dyn_vor", (k_dyn_vor<T, SCHEME, np_COR, np_MET, np_CME>), (S_dyn_vor<T, SCHEME, np_COR, np_MET, np_CME>), g, d, un, vn, ua, va, kch);
         break;
     }
     return 0;
@@ -917,35 +1064,84 @@ template int launch_dyn_zdf<float>(double, const float *, const float *, float *
 template <typename T, int ADV, int KEG, int SCHEME, int NCOR, int NRVM, int NTOT>
 struct S_step_dyn1 {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const T *__restrict__ un, const T *__restrict__ vn, const T *__restrict__ wn, T *__restrict__ ua, T *__restrict__ va, const double *__restrict__ r1_hu_n, const double *__restrict__ r1_hv_n, const double *__restrict__ un_b, const double *__restrict__ vn_b, double *__restrict__ zu_frc, double *__restrict__ zv_frc, double *__restrict__ su_s, double *__restrict__ sv_s, double *__restrict__ zwxb, double *__restrict__ zwyb)
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const T *__restrict__ un, const T *__restrict__ vn, const T *__restrict__ wn, T *__restrict__ ua, T *__restrict__ va, const double *__restrict__ r1_hu_n, const double *__restrict__ r1_hv_n, const double *__restrict__ un_b, const double *__restrict__ vn_b, double *__restrict__ zu_frc, double *__restrict__ zv_frc, double *__restrict__ su_s, double *__restrict__ sv_s, double *__restrict__ zwxb, double *__restrict__ zwyb, int kch)
     {
         THREAD_IJ_V(vb_, 1, 1);
-        if (i > d.jpi || j > d.jpj) return;
-        const size_t ij = IJ(i, j);
+        constexpr bool TILE = SCHEME == NEMO_NP_EEN || SCHEME == NEMO_NP_EET;
         const int jpk = d.jpk;
-        if (!is_interior(d, i, j)) {
-            for (int k = 1; k <= jpk; k++) {
+        // the chunk's levels; a workgroup of whole columns also sums them
+        const int ka = (int)vb_.z * kch + 1, kb = min(ka + kch - 1, jpk - 1);
+        const bool whole = kch >= jpk - 1;
+        const bool in = i <= d.jpi && j <= d.jpj, inner = in && is_interior(d, i, j);
+        const uint32_t ij = in ? IJ32(i, j) : 0u;
+        if (in && !inner) {
+            for (int k = ka; k <= (kb == jpk - 1 ? jpk : kb); k++) {
                 A3(ua, i, j, k) = T(0);
                 A3(va, i, j, k) = T(0);
             }
-            double su = 0.0, sv = 0.0;
-            su = su * r1_hu_n[ij];
-            sv = sv * r1_hv_n[ij];
-            zu_frc[ij] = su; su_s[ij] = su;
-            zv_frc[ij] = sv; sv_s[ij] = sv;
-            return;
+            if (whole) {
+                double su = 0.0, sv = 0.0;
+                su = su * r1_hu_n[ij];
+                sv = sv * r1_hv_n[ij];
+                zu_frc[ij] = su; su_s[ij] = su;
+                zv_frc[ij] = sv; sv_s[ij] = sv;
+            }
+        }
+        if (!TILE && !inner) return;
+        typedef ZwzTile<T, TILE ? SCHEME : NEMO_NP_EET, NTOT> Z;
+        __shared__ typename Z::Lds zf;
+        __shared__ int s_bot;
+        // threads without a cell of their own work on the f-points: cell (2,2)
+        const uint32_t c = inner ? ij : IJ32(2, 2);
+        int kvor = kb;
+        [[maybe_unused]] typename std::conditional<TILE, Z, int>::type f = [&] {
+            if constexpr (TILE) return Z(d, (int)(bx_ * Z::TX) + 1, (int)(by_ * (Z::H - 2)) + 1);
+            else return 0;
+        }();
+        [[maybe_unused]] typename std::conditional<TILE, EenCol<T>, int>::type e = [&] {
+            if constexpr (TILE) return EenCol<T>(d, c);
+            else return 0;
+        }();
+        if constexpr (TILE) {
+            if (Z::EEN) kvor = min(kb, f.bottom(&s_bot));   // below, the vorticity trend is zero
+            if (kvor >= ka) f.fetch(d, un, vn, ka);
         }
         const Metrics<T> &m = met<T>(d);
-        const T e1u = m.e1u[ij], e2v = m.e2v[ij], r1_e1e2u = m.r1_e1e2u[ij], r1_e1e2v = m.r1_e1e2v[ij];
-        const T e1e2t = m.e1e2t[ij], e1e2t_e = m.e1e2t[IJ(i + 1, j)], e1e2t_n = m.e1e2t[IJ(i, j + 1)];
-        // vertical flux carried between levels: zad (dynzad.F90:93-94) or cen2 surface flux (dynadv_cen2.F90:105-112)
+        const T e1u = m.e1u[c], e2v = m.e2v[c], r1_e1e2u = m.r1_e1e2u[c], r1_e1e2v = m.r1_e1e2v[c];
+        const T e1e2t = m.e1e2t[c], e1e2t_e = m.e1e2t[c + 1u], e1e2t_n = m.e1e2t[c + (uint32_t)d.jpi];
+        // vertical fluxes at w-level kk: zad (zero at the surface, dynzad.F90:93-94)
+        // or cen2 (surface flux, dynadv_cen2.F90:105-112), carried between levels
+        const auto wflux = [&](int kk, T &cu, T &cv) {
+            cu = cv = T(0);
+            if (ADV == NEMO_NP_VEC_C2 && kk > 1 && kk <= jpk - 1) {
+                const T zww = T(0.25) * e1e2t * A3(wn, i, j, kk);
+                const T zww_e = T(0.25) * e1e2t_e * A3(wn, i + 1, j, kk);
+                const T zww_n = T(0.25) * e1e2t_n * A3(wn, i, j + 1, kk);
+                cu = (zww_e + zww) * (A3(un, i, j, kk - 1) - A3(un, i, j, kk));
+                cv = (zww_n + zww) * (A3(vn, i, j, kk - 1) - A3(vn, i, j, kk));
+            }
+            if (ADV == NEMO_NP_FLX_C2 && kk == 1) {
+                cu = T(0.5) * (e1e2t * A3(wn, i, j, 1) + e1e2t_e * A3(wn, i + 1, j, 1)) * A3(un, i, j, 1);
+                cv = T(0.5) * (e1e2t * A3(wn, i, j, 1) + e1e2t_n * A3(wn, i, j + 1, 1)) * A3(vn, i, j, 1);
+            }
+            if (ADV == NEMO_NP_FLX_C2 && kk > 1 && kk <= jpk - 1) {
+                const T fw = cen2_zfw(d, wn, i, j, kk);
+                cu = (fw + cen2_zfw(d, wn, i + 1, j, kk)) * (A3(un, i, j, kk) + A3(un, i, j, kk - 1));
+                cv = (fw + cen2_zfw(d, wn, i, j + 1, kk)) * (A3(vn, i, j, kk) + A3(vn, i, j, kk - 1));
+            }
+        };
         T cu_k = T(0), cv_k = T(0);
-        if (ADV == NEMO_NP_FLX_C2) {
-            cu_k = T(0.5) * (e1e2t * A3(wn, i, j, 1) + e1e2t_e * A3(wn, i + 1, j, 1)) * A3(un, i, j, 1);
-            cv_k = T(0.5) * (e1e2t * A3(wn, i, j, 1) + e1e2t_n * A3(wn, i, j + 1, 1)) * A3(vn, i, j, 1);
-        }
+        if (inner) wflux(ka, cu_k, cv_k);
         double su = 0.0, sv = 0.0;
-        for (int k = 1; k <= jpk - 1; k++) {
+        for (int k = ka; k <= kb; k++) {
+            if constexpr (TILE) {
+                if (k <= kvor) {
+                    f.put(d, k, zf);
+                    f.fetch(d, un, vn, min(k + 1, kvor));
+                    __syncthreads();
+                }
+                if (!inner) continue;
+            }
             T a = T(0), b = T(0);
             if (ADV == NEMO_NP_VEC_C2) {
                 T h, he, hn;
@@ -956,15 +1152,8 @@ struct S_step_dyn1 {
                 }
                 a = a - (he - h) / e1u;
                 b = b - (hn - h) / e2v;
-                T cu_kp1 = T(0), cv_kp1 = T(0);
-                if (k + 1 <= jpk - 1) {
-                    const int kk = k + 1;
-                    const T zww = T(0.25) * e1e2t * A3(wn, i, j, kk);
-                    const T zww_e = T(0.25) * e1e2t_e * A3(wn, i + 1, j, kk);
-                    const T zww_n = T(0.25) * e1e2t_n * A3(wn, i, j + 1, kk);
-                    cu_kp1 = (zww_e + zww) * (A3(un, i, j, kk - 1) - A3(un, i, j, kk));
-                    cv_kp1 = (zww_n + zww) * (A3(vn, i, j, kk - 1) - A3(vn, i, j, kk));
-                }
+                T cu_kp1, cv_kp1;
+                wflux(k + 1, cu_kp1, cv_kp1);
                 a = a - (cu_k + cu_kp1) * r1_e1e2u / E3(m.e3u, ij, k);
                 b = b - (cv_k + cv_kp1) * r1_e1e2v / E3(m.e3v, ij, k);
                 cu_k = cu_kp1;
@@ -989,13 +1178,8 @@ struct S_step_dyn1 {
                 const T zfv_t_j = (fv_jm1 + fv_i) * (v_jm1 + v_j);
                 a = a - (zfu_t_ip1 - zfu_t_i + zfv_f_j - zfv_f_jm1) * r1_e1e2u / E3(m.e3u, ij, k);
                 b = b - (zfu_f_i - zfu_f_im1 + zfv_t_jp1 - zfv_t_j) * r1_e1e2v / E3(m.e3v, ij, k);
-                T cu_kp1 = T(0), cv_kp1 = T(0);
-                if (k + 1 <= jpk - 1) {
-                    const int kk = k + 1;
-                    const T fw = cen2_zfw(d, wn, i, j, kk);
-                    cu_kp1 = (fw + cen2_zfw(d, wn, i + 1, j, kk)) * (A3(un, i, j, kk) + A3(un, i, j, kk - 1));
-                    cv_kp1 = (fw + cen2_zfw(d, wn, i, j + 1, kk)) * (A3(vn, i, j, kk) + A3(vn, i, j, kk - 1));
-                }
+                T cu_kp1, cv_kp1;
+                wflux(k + 1, cu_kp1, cv_kp1);
                 a = a - (cu_k - cu_kp1) * r1_e1e2u / E3(m.e3u, ij, k);
                 b = b - (cv_k - cv_kp1) * r1_e1e2v / E3(m.e3v, ij, k);
                 cu_k = cu_kp1;
@@ -1009,7 +1193,12 @@ struct S_step_dyn1 {
                 vor_ene_pt(d, NCOR, un, vn, i, j, k, a, b);
                 break;
             case NEMO_NP_ENT: vor_ent_pt(d, NTOT, un, vn, i, j, k, a, b); break;
-            default: vor_een_pt(d, SCHEME, NTOT, un, vn, i, j, k, a, b); break;
+            default:
+                if constexpr (TILE) {
+                    if (k <= kvor)
+                        vor_een_pt<T, SCHEME, Z::W>(d, e, zf[k & 1], (int)threadIdx.x, (int)threadIdx.y, un, vn, c, k, a, b);
+                }
+                break;
             }
             const size_t p = IJK(i, j, k);
             ua[p] = a;
@@ -1017,8 +1206,12 @@ struct S_step_dyn1 {
             su = su + (double)E3(m.e3u, ij, k) * (double)a * UMASK(double, i, j, k);
             sv = sv + (double)E3(m.e3v, ij, k) * (double)b * VMASK(double, i, j, k);
         }
-        A3(ua, i, j, jpk) = T(0);
-        A3(va, i, j, jpk) = T(0);
+        if (!inner) return;
+        if (kb == jpk - 1) {
+            A3(ua, i, j, jpk) = T(0);
+            A3(va, i, j, jpk) = T(0);
+        }
+        if (!whole) return;   // k_step_sum
         su = su * r1_hu_n[ij];
         sv = sv * r1_hv_n[ij];
         zu_frc[ij] = su; su_s[ij] = su;
@@ -1033,9 +1226,59 @@ KERNEL void k_step_dyn1(DevDomain d, const T *__restrict__ un, const T *__restri
                         const double *__restrict__ r1_hv_n, const double *__restrict__ un_b,
                         const double *__restrict__ vn_b, double *__restrict__ zu_frc, double *__restrict__ zv_frc,
                         double *__restrict__ su_s, double *__restrict__ sv_s, double *__restrict__ zwxb,
-                        double *__restrict__ zwyb)
+                        double *__restrict__ zwyb, int kch)
 {
-    S_step_dyn1<T, ADV, KEG, SCHEME, NCOR, NRVM, NTOT>::run(vb_hw(), d, un, vn, wn, ua, va, r1_hu_n, r1_hv_n, un_b, vn_b, zu_frc, zv_frc, su_s, sv_s, zwxb, zwyb);
+    S_step_dyn1<T, ADV, KEG, SCHEME, NCOR, NRVM, NTOT>::run(vb_hw(), d, un, vn, wn, ua, va, r1_hu_n, r1_hv_n, un_b, vn_b, zu_frc, zv_frc, su_s, sv_s, zwxb, zwyb, kch);
+}
+
+
+// the sums of k_step_dyn1 where its levels are shared out: one thread per column
+// and component (grid.z), eight levels' loads together
+template <typename T>
+struct S_step_sum {
+    static constexpr int NTHR = NH_BLOCK, WAVES = 1, KB = 8;
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, const T *__restrict__ un, const T *__restrict__ vn, const T *__restrict__ ua, const T *__restrict__ va, const double *__restrict__ r1_hu_n, const double *__restrict__ r1_hv_n, const double *__restrict__ un_b, const double *__restrict__ vn_b, double *__restrict__ zu_frc, double *__restrict__ zv_frc, double *__restrict__ su_s, double *__restrict__ sv_s, double *__restrict__ zwxb, double *__restrict__ zwyb)
+    {
+        THREAD_IJ_V(vb_, 1, 1);
+        if (i > d.jpi || j > d.jpj) return;
+        const bool cv = vb_.z != 0;
+        const uint32_t ij = IJ32(i, j);
+        const Metrics<T> &m = met<T>(d);
+        const T *a = cv ? va : ua, *e3 = cv ? m.e3v : m.e3u;
+        const uint32_t w = cv ? d.kvf[ij] : d.ktu[ij] >> 16;
+        const int m0 = (int)(w & 255u), m1 = (int)((w >> 8) & 255u);
+        const bool inner = is_interior(d, i, j), uni = d.e3_sij == 0;
+        double s = 0.0;
+        if (inner) {
+            for (int k0 = 1; k0 <= d.jpk - 1; k0 += KB) {
+                T av[KB];
+    #pragma unroll
+                for (int q = 0; q < KB; q++) av[q] = ldp(plane_ptr(a, d.n2, min(k0 + q, d.jpk - 1)), ij);
+    #pragma unroll
+                for (int q = 0; q < KB; q++) {
+                    const int k = k0 + q;
+                    if (k > d.jpk - 1) break;
+                    s = s + (double)(uni ? uld(e3, k - 1) : E3(e3, ij, k)) * (double)av[q] * (k >= m0 && k <= m1 ? 1.0 : 0.0);
+                }
+            }
+        }
+        s = s * (cv ? r1_hv_n : r1_hu_n)[ij];
+        (cv ? zv_frc : zu_frc)[ij] = s;
+        (cv ? sv_s : su_s)[ij] = s;
+        if (!inner) return;
+        if (cv) zwyb[ij] = (double)A3(vn, i, j, d.mbkv[ij]) - vn_b[ij];
+        else zwxb[ij] = (double)A3(un, i, j, d.mbku[ij]) - un_b[ij];
+    }
+};
+template <typename T>
+KERNEL void k_step_sum(DevDomain d, const T *__restrict__ un, const T *__restrict__ vn, const T *__restrict__ ua,
+                       const T *__restrict__ va, const double *__restrict__ r1_hu_n,
+                       const double *__restrict__ r1_hv_n, const double *__restrict__ un_b,
+                       const double *__restrict__ vn_b, double *__restrict__ zu_frc, double *__restrict__ zv_frc,
+                       double *__restrict__ su_s, double *__restrict__ sv_s, double *__restrict__ zwxb,
+                       double *__restrict__ zwyb)
+{
+    S_step_sum<T>::run(vb_hw(), d, un, vn, ua, va, r1_hu_n, r1_hv_n, un_b, vn_b, zu_frc, zv_frc, su_s, sv_s, zwxb, zwyb);
 }
 
 // ua after dyn_spg_ts: interior columns remove the vertical mean of the
@@ -1130,19 +1373,26 @@ static int launch_step_dyn1_s(const DevDomain &d, Grid2 g, const T *un, const T 
                               const nemo_hip_spg_ts_t *st, double **w)
 {
     const double *r1u = st->r1_hu_n, *r1v = st->r1_hv_n, *ub = st->un_b, *vb = st->vn_b;
+    const int kch = lev_chunks(g.grid.x * g.grid.y, d.jpk - 1);
+    g.grid.z = (unsigned)((d.jpk - 1 + kch - 1) / kch);
     switch (ADV) {
     case NEMO_NP_LIN_DYN:
         LAUNCHB("step_dyn", (k_step_dyn1<T, ADV, KEG, SCHEME, np_COR, np_COR, np_COR>), (S_step_dyn1<T, ADV, KEG, SCHEME, np_COR, np_COR, np_COR>), g, d, un, vn, wn, ua, va, r1u,
-               r1v, ub, vb, w[0], w[1], w[2], w[3], w[4], w[5]);
+               r1v, ub, vb, w[0], w[1], w[2], w[3], w[4], w[5], kch);
         break;
     case NEMO_NP_VEC_C2:
         LAUNCHB("step_dyn", (k_step_dyn1<T, ADV, KEG, SCHEME, np_COR, np_RVO, np_CRV>), (S_step_dyn1<T, ADV, KEG, SCHEME, np_COR, np_RVO, np_CRV>), g, d, un, vn, wn, ua, va, r1u,
-               r1v, ub, vb, w[0], w[1], w[2], w[3], w[4], w[5]);
+               r1v, ub, vb, w[0], w[1], w[2], w[3], w[4], w[5], kch);
         break;
     default:
         LAUNCHB("step_dyn", (k_step_dyn1<T, ADV, KEG, SCHEME, np_COR, np_MET, np_CME>), (S_step_dyn1<T, ADV, KEG, SCHEME, np_COR, np_MET, np_CME>), g, d, un, vn, wn, ua, va, r1u,
-               r1v, ub, vb, w[0], w[1], w[2], w[3], w[4], w[5]);
+               r1v, ub, vb, w[0], w[1], w[2], w[3], w[4], w[5], kch);
         break;
+    }
+    if (g.grid.z > 1) {
+        g.grid.z = 2;
+        LAUNCHB("step_dyn", k_step_sum<T>, (S_step_sum<T>), g, d, un, vn, (const T *)ua, (const T *)va, r1u, r1v, ub, vb, w[0], w[1], w[2],
+                w[3], w[4], w[5]);
     }
     return 0;
 }
