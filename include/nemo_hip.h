@@ -439,6 +439,13 @@ int nemo_hip_tra_adv_fct_coef(double p2dt, const double *pun, const double *pvn,
 int nemo_hip_tra_adv_fct_tl(double p2dt, const double *pun, const double *pvn, const double *pwn, const double *ptb,
                             const double *ptn, int kn_fct_h, int kn_fct_v, const double *pcx, const double *pcy,
                             const double *pcz, double *pta);
+/* tra_adv_fct_coef, then tra_adv_fct_tl with those factors, from one
+   evaluation of the fluxes */
+int nemo_hip_tra_adv_fct_coef_tl(double p2dt, const double *pun, const double *pvn, const double *pwn,
+                                 const double *ptb, const double *ptn, int kn_fct_h, int kn_fct_v, double *pcx,
+                                 double *pcy, double *pcz, double *pta);
+/* tra_nxt (TRA/tranxt.F90:66-237) of one tracer */
+int nemo_hip_tra_nxt_one(int kt, double *tb, double *tn, double *ta);
 /* ptb_ad, ptn_ad += the transpose of tra_adv_fct_tl applied to pta_ad */
 int nemo_hip_tra_adv_fct_ad(const double *pun, const double *pvn, const double *pwn, int kn_fct_h, int kn_fct_v,
                             const double *pcx, const double *pcy, const double *pcz, const double *pta_ad,

@@ -1422,15 +1422,15 @@ static int do_wzv(int kt, const T *hdivn, T *wn)
 }
 
 template <typename T>
-static int do_tra_nxt(int kt, T *tsb, T *tsn, T *tsa)
+static int do_tra_nxt(int kt, T *tsb, T *tsn, T *tsa, int ntr = 2)
 {
     NEED_DOMAIN();
     NEED_STEADY(kt);
     NEED_PTR(tsb); NEED_PTR(tsn); NEED_PTR(tsa);
-    const size_t n4 = g_c->dom.n3 * 2;
+    const size_t n4 = g_c->dom.n3 * (size_t)ntr;
     Stager S;
     T *b = S.inout(tsb, n4), *n = S.inout(tsn, n4), *a = S.inout(tsa, n4);
-    int rc = S.status ? S.status : launch_tra_nxt<T>(euler_step(kt), b, n, a);
+    int rc = S.status ? S.status : launch_tra_nxt<T>(euler_step(kt), b, n, a, ntr);
     return S.finish(rc);
 }
 
@@ -1908,6 +1908,7 @@ int nemo_hip_ssh_swp(int kt, double *sshb, double *sshn, const double *ssha)
     return S.finish(rc);
 }
 int nemo_hip_tra_nxt(int kt, double *tsb, double *tsn, double *tsa) { return do_tra_nxt<double>(kt, tsb, tsn, tsa); }
+int nemo_hip_tra_nxt_one(int kt, double *tb, double *tn, double *ta) { return do_tra_nxt<double>(kt, tb, tn, ta, 1); }
 int nemo_hip_dyn_nxt(int kt, double *ub, double *vb, double *un, double *vn, double *ua, double *va,
                      const double *ua_b, const double *va_b, const double *un_adv, const double *vn_adv,
                      double *ub_b, double *vb_b, double *un_b, double *vn_b, const double *r1_hu_n,
@@ -2201,6 +2202,22 @@ int nemo_hip_tra_adv_fct_tl(double p2dt, const double *pun, const double *pvn, c
     int rc = S.status ? S.status
                       : launch_fct_frozen(1, p2dt, u, v, w, tb, tn, kn_fct_h, kn_fct_v, (double *)cx, (double *)cy,
                                           (double *)cz, ta);
+    return S.finish(rc);
+}
+
+int nemo_hip_tra_adv_fct_coef_tl(double p2dt, const double *pun, const double *pvn, const double *pwn,
+                                 const double *ptb, const double *ptn, int kn_fct_h, int kn_fct_v, double *pcx,
+                                 double *pcy, double *pcz, double *pta)
+{
+    NEED_DOMAIN();
+    NEED_FCT_ORDERS(kn_fct_h, kn_fct_v);
+    NEED_PTR(pun); NEED_PTR(pvn); NEED_PTR(pwn); NEED_PTR(ptb); NEED_PTR(ptn); NEED_PTR(pcx); NEED_PTR(pcy);
+    NEED_PTR(pcz); NEED_PTR(pta);
+    const size_t n3 = g_c->dom.n3;
+    Stager S;
+    const double *u = S.in(pun, n3), *v = S.in(pvn, n3), *w = S.in(pwn, n3), *tb = S.in(ptb, n3), *tn = S.in(ptn, n3);
+    double *cx = S.inout(pcx, n3), *cy = S.inout(pcy, n3), *cz = S.inout(pcz, n3), *ta = S.inout(pta, n3);
+    int rc = S.status ? S.status : launch_fct_frozen(2, p2dt, u, v, w, tb, tn, kn_fct_h, kn_fct_v, cx, cy, cz, ta);
     return S.finish(rc);
 }
 

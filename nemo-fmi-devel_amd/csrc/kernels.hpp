@@ -51,7 +51,7 @@ int launch_ssh_nxt(double z2dt, double zcoef, const T *un, const T *vn, T *hdivn
                    const double *emp_b, const double *emp, double *ssha);
 template <typename T> int launch_wzv(int first, double z1_2dt, const T *hdivn, T *wn);
 int launch_ssh_swp(int euler, double *sshb, double *sshn, const double *ssha);
-template <typename T> int launch_tra_nxt(int euler, T *tsb, T *tsn, T *tsa);
+template <typename T> int launch_tra_nxt(int euler, T *tsb, T *tsn, T *tsa, int ntr = 2);
 template <typename T>
 int launch_dyn_nxt(int euler, T *ub, T *vb, T *un, T *vn, T *ua, T *va, const double *ua_b, const double *va_b,
                    const double *un_adv, const double *vn_adv, double *ub_b, double *vb_b, double *un_b,

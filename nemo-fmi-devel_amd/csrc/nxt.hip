@@ -229,7 +229,7 @@ KERNEL void k_ssh_swp(DevDomain d, int euler, double atfp, double *__restrict__ 
 // tra_nxt, TRA/tranxt.F90:66-192 with tra_nxt_fix, lines 195-237: lbc_lnk of
 // tsa; Euler: tsn = tsa on levels 1..jpkm1; leapfrog: Asselin filter on the
 // interior, then lbc_lnk of tsb, tsn, tsa.  One thread per cell and tracer
-// (grid.z = jpk * 2).
+// (grid.z = jpk times the tracers).
 // ---------------------------------------------------------------------------
 template <typename T>
 struct S_tra_nxt {
@@ -507,11 +507,11 @@ int launch_ssh_swp(int euler, double *sshb, double *sshn, const double *ssha)
 }
 
 template <typename T>
-int launch_tra_nxt(int euler, T *tsb, T *tsn, T *tsa)
+int launch_tra_nxt(int euler, T *tsb, T *tsn, T *tsa, int ntr)
 {
     const DevDomain &d = nh::dom();
     Grid2 g = grid2(d.jpi, d.jpj);
-    g.grid.z = (unsigned)(2 * d.jpk);
+    g.grid.z = (unsigned)(ntr * d.jpk);
     LAUNCHB("tra_nxt", k_tra_nxt<T>, (S_tra_nxt<T>), g, d, euler, d.rn_atfp, tsb, tsn, tsa);
     return 0;
 }
@@ -811,7 +811,7 @@ int launch_istate_bt(const T *un, const T *vn, const T *ub, const T *vb, const d
     template int launch_ssh_nxt<T>(double, double, const T *, const T *, T *, const double *, const double *,    \
                                    const double *, double *);                                                    \
     template int launch_wzv<T>(int, double, const T *, T *);                                                     \
-    template int launch_tra_nxt<T>(int, T *, T *, T *);                                                          \
+    template int launch_tra_nxt<T>(int, T *, T *, T *, int);                                                          \
     template int launch_dyn_nxt<T>(int, T *, T *, T *, T *, T *, T *, const double *, const double *,            \
                                    const double *, const double *, double *, double *, double *, double *,      \
                                    const double *, const double *);                                              \

@@ -814,7 +814,9 @@ KERNEL void k_fct_coef(DevDomain d, const double *__restrict__ paa, const double
 }
 
 // k_fct_final with the factors given: each limited flux is the flux times
-// its factor, at the flux's lbc source, as nonosc and its lbc_lnk give it
+// its factor, at the flux's lbc source, as nonosc and its lbc_lnk give it.  In
+// blocks of FIN_KB levels as k_fct_final (256x256x75: 141 us by whole columns,
+// 63 us)
 KERNEL void k_fct_final_frozen(DevDomain d, const double *__restrict__ paa, const double *__restrict__ pbb,
                                const double *__restrict__ pcc, const double *__restrict__ cx,
                                const double *__restrict__ cy, const double *__restrict__ cz, double *__restrict__ ta)
@@ -834,18 +836,26 @@ KERNEL void k_fct_final_frozen(DevDomain d, const double *__restrict__ paa, cons
         const bool ok = lbc_src_safe(d, 'V', p, q, sp, sq);
         return ok ? A3(pbb, sp, sq, k) * A3(cy, sp, sq, k) : 0.0;
     };
-    double lz_k = A3(pcc, i, j, 1);
-    for (int k = 1; k <= d.jpk - 1; k++) {
+    const int k0 = (int)blockIdx.z * FIN_KB + 1, k1 = min(k0 + FIN_KB - 1, d.jpk - 1);
+    double lz_k = k0 == 1 ? A3(pcc, i, j, 1) : A3(pcc, i, j, k0) * A3(cz, i, j, k0);
+    double tv[FIN_KB];
+#pragma unroll
+    for (int q = 0; q < FIN_KB; q++) tv[q] = A3(ta, i, j, min(k0 + q, k1));
+#pragma unroll
+    for (int q = 0; q < FIN_KB; q++) {
+        const int k = k0 + q;
+        if (k > k1) break;
         const double lz_kp1 = A3(pcc, i, j, k + 1) * A3(cz, i, j, k + 1);
         const size_t p = IJK(i, j, k);
-        ta[p] = ta[p] - (lx(i, j, k) - lx(i - 1, j, k) + ly(i, j, k) - ly(i, j - 1, k) + lz_k - lz_kp1) * r1_e1e2t /
+        ta[p] = tv[q] - (lx(i, j, k) - lx(i - 1, j, k) + ly(i, j, k) - ly(i, j - 1, k) + lz_k - lz_kp1) * r1_e1e2t /
                             E3(m.e3t, ij, k);
         lz_k = lz_kp1;
     }
 }
 
 // mode 0: the factors of the state (tb, tn) into cx, cy, cz; mode 1: pta +=
-// the FCT trend with the factors cx, cy, cz
+// the FCT trend with the factors cx, cy, cz; mode 2: both, from one evaluation
+// of the fluxes (256x256x75: 182 us, which the two calls spend twice)
 int launch_fct_frozen(int mode, double p2dt, const double *pun, const double *pvn, const double *pwn,
                       const double *tb, const double *tn, int kn_h, int kn_v, double *cx, double *cy, double *cz,
                       double *pta)
@@ -873,14 +883,16 @@ int launch_fct_frozen(int mode, double p2dt, const double *pun, const double *pv
         if ((st = launch_lbc<double>(zwy, d.jpk, 'V', 0.0))) return st;
         if ((st = launch_lbc<double>(zwz, d.jpk, 'W', 0.0))) return st;
     }
-    if (mode == 1) {
-        LAUNCH("tra_adv_fct", k_fct_final_frozen, gi, d, zwx, zwy, zwz, cx, cy, cz, pta);
-        return 0;
+    if (mode != 1) {
+        LAUNCHB("tra_adv_fct", (k_fct_beta<double, FctKB<double>::beta>), (S_fct_beta<double, FctKB<double>::beta>), gk, d, p2dt, tb, zwi, zwx, zwy, zwz, zbu, zbd);
+        if ((st = launch_lbc<double>(zbu, d.jpk, 'T', 0.0))) return st;
+        if ((st = launch_lbc<double>(zbd, d.jpk, 'T', 0.0))) return st;
+        LAUNCH("tra_adv_fct", k_fct_coef, gi, d, zwx, zwy, zwz, zbu, zbd, cx, cy, cz);
+        if (mode == 0) return 0;
     }
-    LAUNCHB("tra_adv_fct", (k_fct_beta<double, FctKB<double>::beta>), (S_fct_beta<double, FctKB<double>::beta>), gk, d, p2dt, tb, zwi, zwx, zwy, zwz, zbu, zbd);
-    if ((st = launch_lbc<double>(zbu, d.jpk, 'T', 0.0))) return st;
-    if ((st = launch_lbc<double>(zbd, d.jpk, 'T', 0.0))) return st;
-    LAUNCH("tra_adv_fct", k_fct_coef, gi, d, zwx, zwy, zwz, zbu, zbd, cx, cy, cz);
+    Grid2 gf = gi;
+    gf.grid.z = (unsigned)((d.jpk - 1 + FIN_KB - 1) / FIN_KB);
+    LAUNCH("tra_adv_fct", k_fct_final_frozen, gf, d, zwx, zwy, zwz, cx, cy, cz, pta);
     return 0;
 }
 
@@ -1924,7 +1936,7 @@ struct S_fct_h {
         const size_t n3 = d.n3;
         const T zp2dt = (T)p2dt;
         const uint32_t c = IJ32(i, j);
-        const uint32_t tc = d.ktu[c];
+        const uint32_t tc = d.ktu[c], te = d.ktu[c + 1u], tn_ = d.ktu[c + (uint32_t)d.jpi];
         const T u = tr_u<TRP>(d, pu, i, j, k), v = tr_v<TRP>(d, pv, i, j, k);
         T um = T(0), vm = T(0), e3t = T(1), tm = T(0), r1_e1e2t = T(0);
         if (inner) {
@@ -1933,8 +1945,8 @@ struct S_fct_h {
         }
         // a transport through the face of a dry cell: the limiter may not stop early
         const bool wet = kin<0>(tc, k);
-        if ((!(u == T(0)) && !(wet && kin<0>(d.ktu[c + 1u], k))) || (!(v == T(0)) && !(wet && kin<0>(d.ktu[c + (uint32_t)d.jpi], k))))
-            *dry.flag = dry.gen;
+        const bool we = wet & kin<0>(te, k), wn = wet & kin<0>(tn_, k);
+        if ((!(u == T(0)) & !we) | (!(v == T(0)) & !wn)) *dry.flag = dry.gen;
         // a dry wave whose transports are zero, as they are unless a caller's are
         // not masked: zero fluxes, and a first guess that is masked
         if (!__any(wet) && !__any(!(u == T(0) && v == T(0) && um == T(0) && vm == T(0)))) {
@@ -1963,7 +1975,7 @@ struct S_fct_h {
         T mu_w = T(0), mu_c = T(0), mu_e = T(0), mv_s = T(0), mv_c = T(0), mv_n = T(0);
         if (NH4) {
             mu_w = kin<16>(d.ktu[w_], k) ? T(1) : T(0); mu_c = kin<16>(tc, k) ? T(1) : T(0);
-            mu_e = kin<16>(d.ktu[e1], k) ? T(1) : T(0);
+            mu_e = kin<16>(te, k) ? T(1) : T(0);
             mv_s = kin<0>(d.kvf[s_], k) ? T(1) : T(0); mv_c = kin<0>(d.kvf[c], k) ? T(1) : T(0);
             mv_n = kin<0>(d.kvf[n1], k) ? T(1) : T(0);
         }

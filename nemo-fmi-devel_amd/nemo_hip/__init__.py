@@ -489,6 +489,15 @@ class NemoHip:
         self._check(self.L.nemo_hip_tra_adv_fct_tl(C.c_double(p2dt), p(pun), p(pvn), p(pwn), p(ptb), p(ptn),
                                                    C.c_int(kn[0]), C.c_int(kn[1]), p(cx), p(cy), p(cz), p(pta)))
 
+    def tra_adv_fct_coef_tl(self, p2dt, pun, pvn, pwn, ptb, ptn, cx, cy, cz, pta, kn=(2, 2)):
+        p = self._p
+        self._check(self.L.nemo_hip_tra_adv_fct_coef_tl(C.c_double(p2dt), p(pun), p(pvn), p(pwn), p(ptb), p(ptn),
+                                                        C.c_int(kn[0]), C.c_int(kn[1]), p(cx), p(cy), p(cz), p(pta)))
+
+    def tra_nxt_one(self, kt, tb, tn, ta):
+        p = self._p
+        self._check(self.L.nemo_hip_tra_nxt_one(C.c_int(kt), p(tb), p(tn), p(ta)))
+
     def tra_adv_fct_ad(self, pun, pvn, pwn, cx, cy, cz, ta_ad, tb_ad, tn_ad, kn=(2, 2)):
         p = self._p
         self._check(self.L.nemo_hip_tra_adv_fct_ad(p(pun), p(pvn), p(pwn), C.c_int(kn[0]), C.c_int(kn[1]), p(cx),

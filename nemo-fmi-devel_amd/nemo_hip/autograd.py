@@ -5,7 +5,7 @@ The tracer step is the one the adjoint entry points of the C-ABI transpose
 one tracer in FP64, tra_adv_fct (orders kn) with the limiter factors of
 nonosc (TRA/traadv_fct.F90:404-426), tra_ldf_lap, tra_zdf_imp and the
 leapfrog tra_nxt, the velocities and diffusivities fixed.  Forward computes
-the factors of the state (nemo_hip_tra_adv_fct_coef) and applies them, which
+the factors of the state and applies them (nemo_hip_tra_adv_fct_coef_tl), which
 is the nonlinear step bit for bit; backward applies the adjoint entry points
 with those factors frozen (the transpose of the step linearised with the
 limiter held).  Nothing here computes: every operation is a library call on
@@ -45,23 +45,31 @@ class TracerModel:
 
     def step(self, c, tb, tn):
         """one step with the limiter factors c: (tb, tn) -> (tb', tn')"""
-        h, n3 = self.h, self.n3
         ta = self._z()
-        h.tra_adv_fct_tl(self.p2dt, self.zun, self.zvn, self.zwn, tb, tn, *c, ta, kn=self.kn)
+        self.h.tra_adv_fct_tl(self.p2dt, self.zun, self.zvn, self.zwn, tb, tn, *c, ta, kn=self.kn)
+        return self._diffuse_and_swap(tb, tn, ta)
+
+    def factors_and_step(self, tb, tn):
+        """factors(tb, tn) and step with them, the fluxes evaluated once"""
+        c, ta = [self._z() for _ in range(3)], self._z()
+        self.h.tra_adv_fct_coef_tl(self.p2dt, self.zun, self.zvn, self.zwn, tb, tn, *c, ta, kn=self.kn)
+        return c, self._diffuse_and_swap(tb, tn, ta)
+
+    def _diffuse_and_swap(self, tb, tn, ta):
+        h = self.h
         h.tra_ldf_lap(self.kt, 1, "TRA", self.ahtu, self.ahtv, tb, ta, 1, 1)
         h.tra_zdf_imp(self.kt, 1, "TRA", self.p2dt, tb, ta, 1, self.avt, self.avt)
-        B, N, A = self._z(2), self._z(2), self._z(2)
-        B[:n3].copy_(tb)
-        N[:n3].copy_(tn)
-        A[:n3].copy_(ta)
-        h.tra_nxt(self.kt, B, N, A)
-        return B[:n3].clone(), N[:n3].clone()
+        nb, nn = torch.empty_like(ta), torch.empty_like(ta)
+        nb.copy_(tb)
+        nn.copy_(tn)
+        h.tra_nxt_one(self.kt, nb, nn, ta)
+        return nb, nn
 
     def step_ad(self, c, lb, ln):
         """the adjoint of step with the factors c frozen: (lb', ln') -> (lb, ln)"""
         h = self.h
         lb, ln = lb.contiguous().clone(), ln.contiguous().clone()
-        la = self._z()
+        la = torch.empty_like(lb)   # tra_nxt_ad sets all of it
         h.tra_nxt_ad(lb, ln, la)
         h.tra_zdf_imp_ad(self.p2dt, self.avt, la, lb)
         h.tra_ldf_lap_ad(self.ahtu, self.ahtv, la, lb)
@@ -78,8 +86,7 @@ class TracerStep(torch.autograd.Function):
         cur = torch.cuda.current_stream()
         model.stream.wait_stream(cur)          # the inputs are ready
         with torch.cuda.stream(model.stream):
-            c = model.factors(tb, tn)
-            nb, nn = model.step(c, tb, tn)
+            c, (nb, nn) = model.factors_and_step(tb, tn)
         cur.wait_stream(model.stream)          # the outputs are ready
         for t in (nb, nn):
             t.record_stream(cur)
@@ -92,8 +99,7 @@ class TracerStep(torch.autograd.Function):
         cur = torch.cuda.current_stream()
         model.stream.wait_stream(cur)
         with torch.cuda.stream(model.stream):
-            z = torch.zeros(model.n3, dtype=torch.float64, device="cuda")
-            lb, ln = model.step_ad(ctx.c, z if gb is None else gb, z if gn is None else gn)
+            lb, ln = model.step_ad(ctx.c, model._z() if gb is None else gb, model._z() if gn is None else gn)
         cur.wait_stream(model.stream)
         for t in (lb, ln):
             t.record_stream(cur)
