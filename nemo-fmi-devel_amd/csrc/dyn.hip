@@ -984,31 +984,42 @@ __device__ __forceinline__ void zdf_column_reg(const DevDomain &d, double r2dt, 
 // 75 of the full-size configurations
 #define ZDF_REG_KMAX 76
 
+// The u and v columns of a point by one thread after the other, or, where the
+// columns leave SIMDs idle (two waves each: 512 workgroups; with a remainder,
+// 1024), by two workgroups (grid.z 2), with a checkpoint array each.  k_step_dyn2
+// 32x22x31 FP64: 68 us in turn, 36 us; 362x149x46 FP64 113 and 81 us;
+// 251x333x56 FP32 146 and 101 us.  In a plan the members fill the chip.
+inline unsigned zdf_comps(unsigned nb) { return nh::planning() || nb >= 1024u ? 1u : 2u; }
 template <typename T, bool REG, bool E3U>
 struct S_dyn_zdf {
     static constexpr int NTHR = NH_BLOCK, WAVES = 2;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double r2dt, const T * __restrict__ ub, const T * __restrict__ vb, T * __restrict__ ua, T * __restrict__ va, const T * __restrict__ avm, const double * __restrict__ rCdU_bot, const double * __restrict__ ua_b, const double * __restrict__ va_b, const double * __restrict__ utau, const double * __restrict__ utau_b, const double * __restrict__ vtau, const double * __restrict__ vtau_b, double * __restrict__ zwd_s)
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double r2dt, const T * __restrict__ ub, const T * __restrict__ vb, T * __restrict__ ua, T * __restrict__ va, const T * __restrict__ avm, const double * __restrict__ rCdU_bot, const double * __restrict__ ua_b, const double * __restrict__ va_b, const double * __restrict__ utau, const double * __restrict__ utau_b, const double * __restrict__ vtau, const double * __restrict__ vtau_b, double * __restrict__ zwd_s, double * __restrict__ zwd2_s)
     {
         THREAD_IJ_V(vb_, 1, 1);
         const bool on = i <= d.jpi && j <= d.jpj;
-        if constexpr (REG) {
-            if (!on) return;
-            zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b);
-            zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b);
-        } else {
-            const ZdfLev lu = zdf_levels(d, 0, i, j, on), lv = zdf_levels(d, 1, i, j, on);
-            if (!on) return;
-            zdf_column<E3U>(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b, zwd_s, lu);
-            zdf_column<E3U>(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b, zwd_s, lv);
-        }
+        const auto comp = [&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            const T *xb = c ? vb : ub;
+            T *xa = c ? va : ua;
+            const double *xa_b = c ? va_b : ua_b, *tau = c ? vtau : utau, *tau_b = c ? vtau_b : utau_b;
+            if constexpr (REG) {
+                if (!on) return;
+                zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, c, i, j, xb, xa, avm, rCdU_bot, xa_b, tau, tau_b);
+            } else {
+                const ZdfLev l = zdf_levels(d, c, i, j, on);
+                if (on) zdf_column<E3U>(d, r2dt, c, i, j, xb, xa, avm, rCdU_bot, xa_b, tau, tau_b, c ? zwd2_s : zwd_s, l);
+            }
+        };
+        if (vb_.z == 0) comp(std::integral_constant<int, 0>());
+        if (vb_.z == 1 || vb_.gz == 1) comp(std::integral_constant<int, 1>());
     }
 };
 template <typename T, bool REG, bool E3U>
 KERNEL_W(2) void k_dyn_zdf(DevDomain d, double r2dt, const T * __restrict__ ub, const T * __restrict__ vb, T * __restrict__ ua, T * __restrict__ va, const T * __restrict__ avm,
                           const double * __restrict__ rCdU_bot, const double * __restrict__ ua_b, const double * __restrict__ va_b, const double * __restrict__ utau,
-                          const double * __restrict__ utau_b, const double * __restrict__ vtau, const double * __restrict__ vtau_b, double * __restrict__ zwd_s)
+                          const double * __restrict__ utau_b, const double * __restrict__ vtau, const double * __restrict__ vtau_b, double * __restrict__ zwd_s, double * __restrict__ zwd2_s)
 {
-    S_dyn_zdf<T, REG, E3U>::run(vb_hw(), d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau, utau_b, vtau, vtau_b, zwd_s);
+    S_dyn_zdf<T, REG, E3U>::run(vb_hw(), d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau, utau_b, vtau, vtau_b, zwd_s, zwd2_s);
 }
 // the register form applies: FP32 storage, jpk <= ZDF_REG_KMAX, switch zdf_reg
 template <typename T>
@@ -1024,18 +1035,19 @@ int launch_dyn_zdf(double r2dt, const T *ub, const T *vb, T *ua, T *va, const T 
 {
     const DevDomain &d = nh::dom();
     Grid2 g = grid2(d.jpi, d.jpj);
-    double *zwd = (double *)nh::scratch3(nh::S_ZWT);
+    g.grid.z = zdf_comps(g.grid.x * g.grid.y);
+    double *zwd = (double *)nh::scratch3(nh::S_ZWT), *zwd2 = (double *)nh::scratch3(nh::S_ZWT2);
     // forward-substituted values stay in ua/va at storage precision
     if constexpr (sizeof(T) == 4) {
         if (zdf_reg<T>(d)) {
             LAUNCHB("dyn_zdf", (k_dyn_zdf<T, true, false>), (S_dyn_zdf<T, true, false>), g, d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau,
-                   utau_b, vtau, vtau_b, zwd);
+                   utau_b, vtau, vtau_b, zwd, zwd2);
             return 0;
         }
     }
 #define ZDF_LAUNCH(U) \
     LAUNCHB("dyn_zdf", (k_dyn_zdf<T, false, U>), (S_dyn_zdf<T, false, U>), g, d, r2dt, ub, vb, ua, va, avm, rCdU_bot, ua_b, va_b, utau, \
-           utau_b, vtau, vtau_b, zwd)
+           utau_b, vtau, vtau_b, zwd, zwd2)
     if (d.e3_sij == 0) ZDF_LAUNCH(true);
     else ZDF_LAUNCH(false);
 #undef ZDF_LAUNCH
@@ -1301,54 +1313,46 @@ struct PreSpg {
 template <typename T, bool REG, bool E3U>
 struct S_step_dyn2 {
     static constexpr int NTHR = NH_BLOCK, WAVES = 2;
-    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double r2dt, double r1_2dt_b, const T *__restrict__ ub, const T *__restrict__ vb, T *__restrict__ ua, T *__restrict__ va, T *__restrict__ un, T *__restrict__ vn, const T *__restrict__ avm, const double *__restrict__ rCdU_bot, const double *__restrict__ ua_b, const double *__restrict__ va_b, const double *__restrict__ ub_b, const double *__restrict__ vb_b, const double *__restrict__ un_adv, const double *__restrict__ vn_adv, const double *__restrict__ r1_hu_n, const double *__restrict__ r1_hv_n, const double *__restrict__ un_b, const double *__restrict__ vn_b, const double *__restrict__ su_s, const double *__restrict__ sv_s, const double *__restrict__ utau, const double *__restrict__ utau_b, const double *__restrict__ vtau, const double *__restrict__ vtau_b, double *__restrict__ zwd_s)
+    __device__ __forceinline__ static void run(const VB &vb_, const DevDomain &d, double r2dt, double r1_2dt_b, const T *__restrict__ ub, const T *__restrict__ vb, T *__restrict__ ua, T *__restrict__ va, T *__restrict__ un, T *__restrict__ vn, const T *__restrict__ avm, const double *__restrict__ rCdU_bot, const double *__restrict__ ua_b, const double *__restrict__ va_b, const double *__restrict__ ub_b, const double *__restrict__ vb_b, const double *__restrict__ un_adv, const double *__restrict__ vn_adv, const double *__restrict__ r1_hu_n, const double *__restrict__ r1_hv_n, const double *__restrict__ un_b, const double *__restrict__ vn_b, const double *__restrict__ su_s, const double *__restrict__ sv_s, const double *__restrict__ utau, const double *__restrict__ utau_b, const double *__restrict__ vtau, const double *__restrict__ vtau_b, double *__restrict__ zwd_s, double *__restrict__ zwd2_s)
     {
         THREAD_IJ_V(vb_, 1, 1);
         const bool on = i <= d.jpi && j <= d.jpj;
-        const ZdfLev lu = zdf_levels(d, 0, i, j, on), lv = zdf_levels(d, 1, i, j, on);
-        if (!on) return;
-        const size_t ij = IJ(i, j);
         const size_t plane = d.n2;
-        const uint32_t ij32 = IJ32(i, j);
-        // phase 3 on the now velocities, lines 1254-1259: zero where masked
-        {
-            const double cu = un_adv[ij] * r1_hu_n[ij], cv = vn_adv[ij] * r1_hv_n[ij];
-            const double ubn = un_b[ij], vbn = vn_b[ij];
-            const int u0 = d.kU.k0[ij], u1 = d.kU.k1[ij], v0 = d.kV.k0[ij], v1 = d.kV.k1[ij];
-            const int ke = max(lu.end, lv.end);
-            constexpr int KB = 8;   // levels loaded together, ahead of the stores
-            for (int k0 = 1; k0 <= ke; k0 += KB) {
-                T uo[KB], vo[KB];
+        const uint32_t ij = on ? IJ32(i, j) : 0u;
+        const auto comp = [&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            const ZdfLev l = zdf_levels(d, c, i, j, on);
+            if (!on) return;
+            const int *m0 = c ? d.kV.k0 : d.kU.k0, *m1 = c ? d.kV.k1 : d.kU.k1;
+            const int x0 = m0[ij], x1 = m1[ij];
+            // phase 3 on the now velocity, lines 1254-1259: zero where masked
+            {
+                T *xn = c ? vn : un;
+                const double cx = (c ? vn_adv : un_adv)[ij] * (c ? r1_hv_n : r1_hu_n)[ij], xbn = (c ? vn_b : un_b)[ij];
+                constexpr int KB = 8;   // levels loaded together, ahead of the stores
+                for (int k0 = 1; k0 <= l.end; k0 += KB) {
+                    T xo[KB];
     #pragma unroll
-                for (int q = 0; q < KB; q++) {
-                    const int k = min(k0 + q, ke);
-                    uo[q] = ldp((const T *)plane_ptr(un, plane, k), ij32);
-                    vo[q] = ldp((const T *)plane_ptr(vn, plane, k), ij32);
-                }
+                    for (int q = 0; q < KB; q++) xo[q] = ldp((const T *)plane_ptr(xn, plane, min(k0 + q, l.end)), ij);
     #pragma unroll
-                for (int q = 0; q < KB; q++) {
-                    const int k = k0 + q;
-                    if (k > ke) break;
-                    const double um = (k >= u0 && k <= u1) ? 1.0 : 0.0, vm = (k >= v0 && k <= v1) ? 1.0 : 0.0;
-                    stp(plane_ptr(un, plane, k), ij32, (T)(((double)uo[q] + cu - ubn) * um));
-                    stp(plane_ptr(vn, plane, k), ij32, (T)(((double)vo[q] + cv - vbn) * vm));
+                    for (int q = 0; q < KB; q++) {
+                        const int k = k0 + q;
+                        if (k > l.end) break;
+                        const double xm = (k >= x0 && k <= x1) ? 1.0 : 0.0;
+                        stp(plane_ptr(xn, plane, k), ij, (T)(((double)xo[q] + cx - xbn) * xm));
+                    }
                 }
+                for (int k = l.end + 1; k <= d.jpk - 1; k++) stp(plane_ptr(xn, plane, k), ij, T(0));
             }
-            for (int k = ke + 1; k <= d.jpk - 1; k++) {
-                stp(plane_ptr(un, plane, k), ij32, T(0));
-                stp(plane_ptr(vn, plane, k), ij32, T(0));
-            }
-        }
-        const bool inner = is_interior(d, i, j);
-        PreSpg<T> pu{su_s[ij], (ua_b[ij] - ub_b[ij]) * r1_2dt_b, 0.0, d.kU.k0[ij], d.kU.k1[ij], inner};
-        PreSpg<T> pv{sv_s[ij], (va_b[ij] - vb_b[ij]) * r1_2dt_b, 0.0, d.kV.k0[ij], d.kV.k1[ij], inner};
-        if constexpr (REG) {
-            zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b, pu);
-            zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b, pv);
-        } else {
-            zdf_column<E3U>(d, r2dt, 0, i, j, ub, ua, avm, rCdU_bot, ua_b, utau, utau_b, zwd_s, lu, pu);
-            zdf_column<E3U>(d, r2dt, 1, i, j, vb, va, avm, rCdU_bot, va_b, vtau, vtau_b, zwd_s, lv, pv);
-        }
+            const double *xa_b = c ? va_b : ua_b, *xb_b = c ? vb_b : ub_b, *tau = c ? vtau : utau, *tau_b = c ? vtau_b : utau_b;
+            const T *xb = c ? vb : ub;
+            T *xa = c ? va : ua;
+            const PreSpg<T> px{(c ? sv_s : su_s)[ij], (xa_b[ij] - xb_b[ij]) * r1_2dt_b, 0.0, x0, x1, is_interior(d, i, j)};
+            if constexpr (REG) zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, c, i, j, xb, xa, avm, rCdU_bot, xa_b, tau, tau_b, px);
+            else zdf_column<E3U>(d, r2dt, c, i, j, xb, xa, avm, rCdU_bot, xa_b, tau, tau_b, c ? zwd2_s : zwd_s, l, px);
+        };
+        if (vb_.z == 0) comp(std::integral_constant<int, 0>());
+        if (vb_.z == 1 || vb_.gz == 1) comp(std::integral_constant<int, 1>());
     }
 };
 template <typename T, bool REG, bool E3U>
@@ -1363,9 +1367,9 @@ KERNEL_W(2) void k_step_dyn2(DevDomain d, double r2dt, double r1_2dt_b, const T 
                         const double *__restrict__ su_s, const double *__restrict__ sv_s,
                         const double *__restrict__ utau, const double *__restrict__ utau_b,
                         const double *__restrict__ vtau, const double *__restrict__ vtau_b,
-                        double *__restrict__ zwd_s)
+                        double *__restrict__ zwd_s, double *__restrict__ zwd2_s)
 {
-    S_step_dyn2<T, REG, E3U>::run(vb_hw(), d, r2dt, r1_2dt_b, ub, vb, ua, va, un, vn, avm, rCdU_bot, ua_b, va_b, ub_b, vb_b, un_adv, vn_adv, r1_hu_n, r1_hv_n, un_b, vn_b, su_s, sv_s, utau, utau_b, vtau, vtau_b, zwd_s);
+    S_step_dyn2<T, REG, E3U>::run(vb_hw(), d, r2dt, r1_2dt_b, ub, vb, ua, va, un, vn, avm, rCdU_bot, ua_b, va_b, ub_b, vb_b, un_adv, vn_adv, r1_hu_n, r1_hv_n, un_b, vn_b, su_s, sv_s, utau, utau_b, vtau, vtau_b, zwd_s, zwd2_s);
 }
 
 template <typename T, int ADV, int KEG, int SCHEME>
@@ -1433,19 +1437,20 @@ int launch_step_dyn(int kt, double r2dt, const T *ub, const T *vb, const T *wn, 
     if (rc) return rc;
     if ((rc = launch_dyn_spg_ts<T>(kt, st, 1))) return rc;
     const double z2dt_bf = (kt == d.nit000 && d.neuler == 0) ? d.rdt : 2.0 * d.rdt;
-    double *zwd = (double *)nh::scratch3(nh::S_ZWT);
+    g.grid.z = zdf_comps(g.grid.x * g.grid.y);
+    double *zwd = (double *)nh::scratch3(nh::S_ZWT), *zwd2 = (double *)nh::scratch3(nh::S_ZWT2);
     if constexpr (sizeof(T) == 4) {
         if (zdf_reg<T>(d)) {
             LAUNCHB("step_dyn", (k_step_dyn2<T, true, false>), (S_step_dyn2<T, true, false>), g, d, r2dt, 1.0 / z2dt_bf, ub, vb, ua, va, un, vn, avm,
                    st->rCdU_bot, st->ua_b, st->va_b, st->ub_b, st->vb_b, st->un_adv, st->vn_adv, st->r1_hu_n,
-                   st->r1_hv_n, st->un_b, st->vn_b, w[2], w[3], st->utau, utau_b, st->vtau, vtau_b, zwd);
+                   st->r1_hv_n, st->un_b, st->vn_b, w[2], w[3], st->utau, utau_b, st->vtau, vtau_b, zwd, zwd2);
             return 0;
         }
     }
 #define DYN2_LAUNCH(U) \
     LAUNCHB("step_dyn", (k_step_dyn2<T, false, U>), (S_step_dyn2<T, false, U>), g, d, r2dt, 1.0 / z2dt_bf, ub, vb, ua, va, un, vn, avm, \
            st->rCdU_bot, st->ua_b, st->va_b, st->ub_b, st->vb_b, st->un_adv, st->vn_adv, st->r1_hu_n, st->r1_hv_n, \
-           st->un_b, st->vn_b, w[2], w[3], st->utau, utau_b, st->vtau, vtau_b, zwd)
+           st->un_b, st->vn_b, w[2], w[3], st->utau, utau_b, st->vtau, vtau_b, zwd, zwd2)
     if (d.e3_sij == 0) DYN2_LAUNCH(true);
     else DYN2_LAUNCH(false);
 #undef DYN2_LAUNCH

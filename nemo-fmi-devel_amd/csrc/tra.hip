@@ -816,7 +816,7 @@ KERNEL void k_fct_coef(DevDomain d, const double *__restrict__ paa, const double
 // k_fct_final with the factors given: each limited flux is the flux times
 // its factor, at the flux's lbc source, as nonosc and its lbc_lnk give it.  In
 // blocks of FIN_KB levels as k_fct_final (256x256x75: 141 us by whole columns,
-// 63 us)
+// 64 us)
 KERNEL void k_fct_final_frozen(DevDomain d, const double *__restrict__ paa, const double *__restrict__ pbb,
                                const double *__restrict__ pcc, const double *__restrict__ cx,
                                const double *__restrict__ cy, const double *__restrict__ cz, double *__restrict__ ta)
