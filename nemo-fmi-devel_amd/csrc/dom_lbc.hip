@@ -38,7 +38,10 @@ int launch_dom_msk(double *tmask, double *umask, double *vmask, double *fmask, d
 
 // ---------------------------------------------------------------------------
 // lbc_lnk on (jpi,jpj,nk): one block per level; the east-west fill completes
-// (barrier) before the north-south fill copies whole rows.
+// (barrier) before the north-south fill copies whole rows.  The nk levels may be
+// those of several arrays one after the other (two tracers, both betas), so a
+// level is addressed from its own 64-bit base: only one array of a domain is
+// sure to stay below the 4 GiB that a 32-bit offset reaches.
 // ---------------------------------------------------------------------------
 template <typename T>
 struct S_lbc {
@@ -47,25 +50,26 @@ struct S_lbc {
     {
         const int k = (int)vb_.x + 1;
         if (k > nk) return;
+        T *__restrict__ q = plane_ptr(p, d.n2, k);
         for (int j = (int)threadIdx.x + 1; j <= d.jpj; j += blockDim.x) {
             if (d.iper) {
-                T a = A3(p, d.jpi - 1, j, k), b = A3(p, 2, j, k);
-                A3(p, 1, j, k) = a;
-                A3(p, d.jpi, j, k) = b;
+                T a = ldp((const T *)q, IJ32(d.jpi - 1, j)), b = ldp((const T *)q, IJ32(2, j));
+                stp(q, IJ32(1, j), a);
+                stp(q, IJ32(d.jpi, j), b);
             } else {
-                if (nat != 'F') A3(p, 1, j, k) = pval;
-                A3(p, d.jpi, j, k) = pval;
+                if (nat != 'F') stp(q, IJ32(1, j), pval);
+                stp(q, IJ32(d.jpi, j), pval);
             }
         }
         __syncthreads();
         for (int i = (int)threadIdx.x + 1; i <= d.jpi; i += blockDim.x) {
             if (d.jper) {
-                T a = A3(p, i, d.jpj - 1, k), b = A3(p, i, 2, k);
-                A3(p, i, 1, k) = a;
-                A3(p, i, d.jpj, k) = b;
+                T a = ldp((const T *)q, IJ32(i, d.jpj - 1)), b = ldp((const T *)q, IJ32(i, 2));
+                stp(q, IJ32(i, 1), a);
+                stp(q, IJ32(i, d.jpj), b);
             } else {
-                if (nat != 'F') A3(p, i, 1, k) = pval;
-                A3(p, i, d.jpj, k) = pval;
+                if (nat != 'F') stp(q, IJ32(i, 1), pval);
+                stp(q, IJ32(i, d.jpj), pval);
             }
         }
     }
