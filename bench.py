@@ -643,7 +643,7 @@ def kernel_times(h):
                         "k_fct_beta", "k_fct_final", "k_fct_low", "k_fct_ad"],
         "tra_ldf_iso": ["k_ldf_iso_coef", "k_tra_ldf_iso", "k_fill3"], "tra_zdf": ["k_tra_zdf", "k_tra_zdf_reg", "k_clamp_ring"],
         "lbc_lnk": ["k_lbc", "k_lbc4"],
-        "step_dyn": ["k_step_dyn1", "k_step_dyn2"],
+        "step_dyn": ["k_step_dyn1", "k_step_sum", "k_step_dyn2"],
         "step_tra": ["k_fct_fused", "k_fct_cpt_fwd", "k_fct_h", "k_fct_hh", "k_fct_v", "k_fct_vz_reg", "k_fct_lim", "k_fct_vlim",
                      "k_fct_beta", "k_fct_final", "k_zero_ring", "k_tra_zdf", "k_tra_zdf_reg"],
         "div_hor": ["k_div_hor"], "ssh_nxt": ["k_ssh_nxt"], "wzv": ["k_wzv"], "ssh_swp": ["k_ssh_swp"],
@@ -1075,6 +1075,7 @@ KERNEL_BYTES = {
     "k_spg_blk": lambda w, i, j, k, f: 45 * 8 * i * j,
     # fused momentum step
     "k_step_dyn1": _b(5),        # r un vn wn, w ua va
+    "k_step_sum": _b(2),         # r ua va
     "k_step_dyn2": _b(11),       # r ua va un vn ub vb avm, w ua va un vn
     # time-step closure
     "k_div_hor": _b(3),          # r un vn, w hdivn

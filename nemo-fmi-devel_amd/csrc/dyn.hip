@@ -1298,7 +1298,7 @@ KERNEL void k_step_sum(DevDomain d, const T *__restrict__ un, const T *__restric
 // correction (phase 3, rounded to storage)
 template <typename T>
 struct PreSpg {
-    double s, dd, xm0;
+    double s, dd;
     int x0, x1;
     bool inner;
     __device__ __forceinline__ T operator()(int k, T x) const
@@ -1347,7 +1347,7 @@ struct S_step_dyn2 {
             const double *xa_b = c ? va_b : ua_b, *xb_b = c ? vb_b : ub_b, *tau = c ? vtau : utau, *tau_b = c ? vtau_b : utau_b;
             const T *xb = c ? vb : ub;
             T *xa = c ? va : ua;
-            const PreSpg<T> px{(c ? sv_s : su_s)[ij], (xa_b[ij] - xb_b[ij]) * r1_2dt_b, 0.0, x0, x1, is_interior(d, i, j)};
+            const PreSpg<T> px{(c ? sv_s : su_s)[ij], (xa_b[ij] - xb_b[ij]) * r1_2dt_b, x0, x1, is_interior(d, i, j)};
             if constexpr (REG) zdf_column_reg<ZDF_REG_KMAX>(d, r2dt, c, i, j, xb, xa, avm, rCdU_bot, xa_b, tau, tau_b, px);
             else zdf_column<E3U>(d, r2dt, c, i, j, xb, xa, avm, rCdU_bot, xa_b, tau, tau_b, c ? zwd2_s : zwd_s, l, px);
         };

@@ -11,8 +11,9 @@
 //
 // lbc_lnk is folded into the kernels.  A read-only input (un, vn for the
 // divergence) lets a ring point compute its value at its lbc source point.
-// Fields updated in place (tsb/tsn/tsa, ua) are written to the ring by the
-// thread of the interior source point (lbc_targets), so no thread reads a
+// The tracers, updated in place, are written to the ring by the thread of the
+// interior source point (lbc_targets); dyn_nxt's cyclic ring columns follow in a
+// second launch that reads the finished source columns.  So no thread reads a
 // value another thread of the same launch overwrites.
 #include "common.hpp"
 #include "kernels.hpp"
