@@ -148,23 +148,51 @@ KERNEL void k_slp_mxl(DevDomain d, SlpIn<T> in, const int32_t *__restrict__ nmln
 // one (the reference's lbc_lnk of zwz/zww, lines 231 and 315): there the region
 // runs on past the domain's last column to its first, both ring columns
 // included, so the source is two points away across the seam and the region
-// has two more points on each side.  The output's ring is the final lbc_lnk
-// (line 361), a separate pass.
+// has two more points on the side of the seam (slp_tile).  The output's ring is
+// the final lbc_lnk (line 361), a separate pass.
 //
 // The terms of the mixed layer (a division and the depths) are formed only at
 // levels where a column of the wave is in it, -7e3/e3 once per level where the
-// scale factors are horizontally uniform, and levels below the region's deepest
-// column are stored as the zeros the masks give.
+// scale factors are horizontally uniform (E3U; where they vary, they are loaded
+// with the level's fields, ahead of the barrier), and levels below the region's
+// deepest column are stored as the zeros the masks give.
 //
 // Bound by FP64 vector instructions (six divisions per point).  One level of
 // a 64x4 tile per workgroup, staged in LDS with its two-point halo, ran 1020
 // instructions per cell: 512x509x75 FP32 790 -> 330 us, 203x157x31 cyclic FP64
-// 74 -> 39 us.
+// 74 -> 39 us; all wet, and the mixed layer down to the bottom, 600x500x60 FP32
+// 773 -> 695 us, 300x200x60 cyclic both ways FP64 203 -> 175 us (277 us with the
+// wide halo on every side of every tile); e3 varying, 512x512x75 FP32 847 -> 407
+// us (551 us with e3 loaded where used).
 // ---------------------------------------------------------------------------
 #define SLP_RX 32
 #define SLP_RY 16
 #define SLP_MAXKB 24
-template <typename T>
+// The n interior points of a direction over tiles, each the middle of a region of
+// R columns: a halo of two points on each side, four where the tile meets a
+// seam, which the first and the last tile of a cyclic direction do.  Tile t of nt
+// owns cnt points from o on (0-based), the first of them at region column h.
+inline int slp_tiles(int n, int R, int per)
+{
+    if (!per) return (n + R - 5) / (R - 4);
+    if (n <= R - 8) return 1;
+    const int r = n - 2 * (R - 6);
+    return r <= 0 ? 2 : 2 + (r + R - 5) / (R - 4);
+}
+__device__ inline void slp_tile(int t, int nt, int n, int R, int per, int &o, int &cnt, int &h)
+{
+    h = per && t == 0 ? 4 : 2;
+    if (!per) {
+        o = t * (R - 4);
+        cnt = min(R - 4, n - o);
+        return;
+    }
+    const int e = nt == 1 ? n : nt == 2 ? (n + 1) / 2 : R - 6;    // the first tile's points
+    const int w = nt > 2 ? (n - 2 * e + nt - 3) / (nt - 2) : 0;   // a middle one's
+    o = t == 0 ? 0 : t < nt - 1 ? e + (t - 1) * w : nt == 2 ? e : n - e;
+    cnt = t == 0 ? e : t < nt - 1 ? min(w, n - e - o) : n - o;
+}
+template <typename T, bool E3U>
 __global__ __launch_bounds__(SLP_RX * SLP_RY, 4) void k_slp(DevDomain d, SlpIn<T> in, const T *__restrict__ gdept,
                                                              const T *__restrict__ gdepw,
                                                              const int32_t *__restrict__ nmln,
@@ -185,14 +213,14 @@ __global__ __launch_bounds__(SLP_RX * SLP_RY, 4) void k_slp(DevDomain d, SlpIn<T
     xcd_tile(bx, by);
     const int jpi = d.jpi, jpj = d.jpj, jpkm1 = d.jpk - 1;
     const int q = (int)threadIdx.x, lx = q % SLP_RX, ly = q / SLP_RX;
-    // the tile of interior points the workgroup owns, and its halo
-    const int hx = d.iper ? 4 : 2, hy = d.jper ? 4 : 2, wx = SLP_RX - 2 * hx, wy = SLP_RY - 2 * hy;
-    int i = 2 + (int)bx * wx + lx - hx, j = 2 + (int)by * wy + ly - hy;
-    const bool own = lx >= hx && lx < SLP_RX - hx && ly >= hy && ly < SLP_RY - hy && i <= jpi - 1 && j <= jpj - 1;
+    int ox, cx, hx, oy, cy, hy;
+    slp_tile((int)bx, (int)gridDim.x, jpi - 2, SLP_RX, d.iper, ox, cx, hx);
+    slp_tile((int)by, (int)gridDim.y, jpj - 2, SLP_RY, d.jper, oy, cy, hy);
+    int i = 2 + ox + lx - hx, j = 2 + oy + ly - hy;
+    const bool own = lx >= hx && lx < hx + cx && ly >= hy && ly < hy + cy;
     if (d.iper) i = ((i - 1) % jpi + jpi) % jpi + 1;
     if (d.jper) j = ((j - 1) % jpj + jpj) % jpj + 1;
     const int k0 = 2 + (int)blockIdx.z * kb, k1 = min(k0 + kb - 1, jpkm1);
-    const bool uni = d.e3_sij == 0;
     const bool inner = i >= 2 && i <= jpi - 1 && j >= 2 && j <= jpj - 1;
     // columns off the domain read its nearest one and are not used
     const int ic = min(max(i, 1), jpi), jc = min(max(j, 1), jpj);
@@ -204,7 +232,7 @@ __global__ __launch_bounds__(SLP_RX * SLP_RY, 4) void k_slp(DevDomain d, SlpIn<T
     if (q == 0) s_end = 0;
     __syncthreads();
     atomicMax(&s_end, (int)((tc >> 8) & 255u));
-    if (uni && q < k1 - k0 + 1) {
+    if (E3U && q < k1 - k0 + 1) {
         q3u[q] = -7.e+3 / m.e3u[k0 + q - 1];
         q3v[q] = -7.e+3 / m.e3v[k0 + q - 1];
         q3w[q] = -7.e+3 / m.e3w[k0 + q - 1];
@@ -245,6 +273,12 @@ __global__ __launch_bounds__(SLP_RX * SLP_RY, 4) void k_slp(DevDomain d, SlpIn<T
         for (int k = k0; k <= kend; k++) {
             const int kn = min(k + 1, d.jpk);
             const double p_n = ld(in.prd, kn), n_pn = ld(in.pn2, min(k + 2, d.jpk));   // the next level's
+            double e3u = 1., e3v = 1., e3w = 1.;
+            if (!E3U) {
+                e3u = E3(m.e3u, c, k);
+                e3v = E3(m.e3v, c, k);
+                e3w = E3(m.e3w, c, k);
+            }
             const bool um_w = um(tw, k), vm_s = vm(vs, k), um_cp = um(tc, k + 1), vm_cp = vm(vc, k + 1);
             const bool tm_p = vm(tc, k + 1), wm = tm_c && tm_m;
             const double dz = zm1_g * (p_k + 1.) * (n_k + n_p) * (tm_p ? 0.5 : 1.);   // zdzr, lines 162-170
@@ -257,9 +291,9 @@ __global__ __launch_bounds__(SLP_RX * SLP_RY, 4) void k_slp(DevDomain d, SlpIn<T
             if (raw) {
                 const double gu_c = msk(um_c, sp[q + 1] - p_k), gu_w = msk(um_w, p_k - sp[q - 1]);
                 const double gv_c = msk(vm_c, sp[q + SLP_RX] - p_k), gv_s = msk(vm_s, p_k - sp[q - SLP_RX]);
-                const double e3u7 = uni ? q3u[k - k0] : -7.e+3 / E3(m.e3u, c, k);
-                const double e3v7 = uni ? q3v[k - k0] : -7.e+3 / E3(m.e3v, c, k);
-                const double e3w7 = uni ? q3w[k - k0] : -7.e+3 / E3(m.e3w, c, k);
+                const double e3u7 = E3U ? q3u[k - k0] : -7.e+3 / e3u;
+                const double e3v7 = E3U ? q3v[k - k0] : -7.e+3 / e3v;
+                const double e3w7 = E3U ? q3w[k - k0] : -7.e+3 / e3w;
                 // I. u, v slopes, lines 197-219
                 const double zau = gu_c * r1_e1u, zav = gv_c * r1_e2v;
                 double zbu = 0.5 * (dz + sdz[q + 1]), zbv = 0.5 * (dz + sdz[q + SLP_RX]);
@@ -370,18 +404,25 @@ int launch_ldf_slp(const T *prd, const T *pn2, const T *gdept, const T *gdepw, c
     LAUNCH("ldf_slp", k_slp_mxl<T>, g2, d, in, nmln, hmlpt, z1_slpmax, zsu, zsv, wiml, wjml);
     Grid2 g;
     g.block = dim3(SLP_RX * SLP_RY, 1, 1);
-    const int wx = SLP_RX - (d.iper ? 8 : 4), wy = SLP_RY - (d.jper ? 8 : 4);
-    g.grid = dim3((unsigned)((d.jpi - 2 + wx - 1) / wx), (unsigned)((d.jpj - 2 + wy - 1) / wy), 1);
+    g.grid = dim3((unsigned)slp_tiles(d.jpi - 2, SLP_RX, d.iper), (unsigned)slp_tiles(d.jpj - 2, SLP_RY, d.jper), 1);
     // levels per workgroup: long marches repeat fewer first levels, short ones
-    // fill the chip (two workgroups per CU) on small domains
+    // fill the chip (two workgroups per CU, 512).  Where four levels each would
+    // leave it unfilled, as few as fill it (FP64, four levels and one: 32x22x31
+    // 27.3 and 16.6 us, 60x50x40 27.8 and 18.2 us)
     const int tiles = (int)(g.grid.x * g.grid.y), nlev = d.jpk - 2;
     int nz = (1536 + tiles - 1) / tiles;
     nz = nz < 1 ? 1 : nz > (nlev + 3) / 4 ? (nlev + 3) / 4 : nz;
     if ((nlev + nz - 1) / nz > SLP_MAXKB) nz = (nlev + SLP_MAXKB - 1) / SLP_MAXKB;
-    const int kb = (nlev + nz - 1) / nz;
+    int kb = (nlev + nz - 1) / nz;
+    const int kfill = (tiles * nlev + 256) / 512;
+    if (kfill < 4) kb = kfill < 1 ? 1 : kfill;
     g.grid.z = (unsigned)((nlev + kb - 1) / kb);
-    LAUNCH("ldf_slp", k_slp<T>, g, d, in, gdept, gdepw, nmln, (const double *)zsu, (const double *)zsv, hmlp,
-           (const double *)wiml, (const double *)wjml, z1_slpmax, kb, uslp, vslp, wslpi, wslpj);
+#define SLP_LAUNCH(U)                                                                                               \
+    LAUNCH("ldf_slp", (k_slp<T, U>), g, d, in, gdept, gdepw, nmln, (const double *)zsu, (const double *)zsv, hmlp, \
+           (const double *)wiml, (const double *)wjml, z1_slpmax, kb, uslp, vslp, wslpi, wslpj)
+    if (d.e3_sij == 0) SLP_LAUNCH(true);
+    else SLP_LAUNCH(false);
+#undef SLP_LAUNCH
     return launch_lbc4<T>(uslp, vslp, wslpi, wslpj, d.jpk);
 }
 
