@@ -363,14 +363,12 @@ int launch_dyn_ldf_lap(double zsign, const T *pub, const T *pvb, T *pua, T *pva,
     g.block = dim3(LDF_RX * LDF_RY, 1, 1);
     g.grid = dim3((unsigned)((d.jpi - 2 + LDF_RX - 3) / (LDF_RX - 2)), (unsigned)((d.jpj - 2 + LDF_RY - 3) / (LDF_RY - 2)), 1);
     // levels per workgroup: two rounds of the two workgroups that fit a CU (1024),
-    // the metrics read once for up to 16 levels, in equal shares.  (At four rounds
+    // the metrics read once for up to 16 levels.  (At four rounds
     // 1500x40x40 FP64 took 62 us and 251x233x20 35, slower than a workgroup per
     // level of a 64x4 tile, 50 and 28; now 45 and 28)
     const int tiles = (int)(g.grid.x * g.grid.y), nlev = d.jpk - 1;
     int kb = (int)(((long)tiles * nlev + 512) / 1024);
     kb = kb < 1 ? 1 : kb > 16 ? 16 : kb;
-    const int nz = (nlev + kb - 1) / kb;
-    kb = (nlev + nz - 1) / nz;
     g.grid.z = (unsigned)((nlev + kb - 1) / kb);
     LAUNCH("dyn_ldf", k_dyn_ldf_lap<T>, g, d, zsign, kb, pub, pvb, pua, pva, ahmt, ahmf);
     return 0;
