@@ -306,8 +306,19 @@ KERNEL void k_tra_nxt(DevDomain d, int euler, double atfp, T *__restrict__ tsb, 
 // again, for deeper columns.
 // lbc_lnk('U'/'V') of line 139: ring points without a source (closed sides) are
 // columns of zeros in the same launch; the ones with a source (cyclic sides)
-// follow in a launch of their own (RING), which reads the finished source.
+// follow in a launch of their own (RING), which reads the finished source.  The
+// ring's columns along j are jpi points apart, a cache line per lane, and few:
+// one for every NXT_RING-th lane makes a wave's accesses as many times cheaper and
+// spreads them over more waves.  With one per lane their launch took 51 of the 134
+// us of 362x149x46 FP64, e3 varying (88 now); of the rows along i one per lane
+// (300x260x40 FP32, cyclic along j: 48 us, every 8th lane 57).
+// Scale factors that vary are loaded with each KB levels' other operands: loaded
+// where used, after the stores of the level before, 512x512x75 FP32 took 428 us
+// (385 now).
 // ---------------------------------------------------------------------------
+#define NXT_RING 8
+// threads for the ring's rows (with a source where the domain is cyclic along j), whole waves
+__host__ __device__ inline int nxt_ring_rows(const DevDomain &d) { return d.jper ? (2 * d.jpi + 63) / 64 * 64 : 0; }
 template <typename T, int KMAX, bool E3U, bool RING>
 struct S_dyn_nxt {
     static constexpr int NTHR = NH_BLOCK, WAVES = 1;
@@ -315,10 +326,18 @@ struct S_dyn_nxt {
     {
         int i, j;
         if constexpr (RING) {
-            const int p = (int)(vb_.x * NH_BLOCK + threadIdx.y * blockDim.x + threadIdx.x), q = p - 2 * d.jpi;
-            i = q >= 0 ? ((q & 1) ? d.jpi : 1) : p < d.jpi ? p + 1 : p - d.jpi + 1;
-            j = q >= 0 ? 2 + q / 2 : p < d.jpi ? 1 : d.jpj;
-            if (q >= 0 && j > d.jpj - 1) return;
+            const int t = (int)(vb_.x * NH_BLOCK + threadIdx.y * blockDim.x + threadIdx.x), nr = nxt_ring_rows(d);
+            if (t < nr) {
+                if (t >= 2 * d.jpi) return;
+                i = t < d.jpi ? t + 1 : t - d.jpi + 1;
+                j = t < d.jpi ? 1 : d.jpj;
+            } else {
+                if ((t - nr) % NXT_RING) return;
+                const int q = (t - nr) / NXT_RING;
+                i = (q & 1) ? d.jpi : 1;
+                j = 2 + q / 2;
+                if (j > d.jpj - 1) return;
+            }
         } else {
             unsigned bx, by;
             xcd_tile_v(vb_, bx, by);
@@ -351,6 +370,12 @@ struct S_dyn_nxt {
     #pragma unroll
             for (int q = 0; q < KB; q++) v[q] = ldp(plane_ptr(p, d.n2, min(k0 + q, nlev - 1) + 1), c);
         };
+        // scale factors that vary: KB at a time, with the levels' other operands
+        const auto load_e3 = [&](int k0, double *v) {
+    #pragma unroll
+            for (int q = 0; q < KB; q++) v[q] = E3U ? 1.0 : E3(e3x, ij, min(k0 + q, nlev - 1) + 1);
+        };
+        const auto e3_of = [&](int k, double v) { return E3U ? uld(e3x, k - 1) : v; };
         // A
         T x[NB * KB];
         double mean = 0.0;
@@ -388,13 +413,15 @@ struct S_dyn_nxt {
         double sn = 0.0, sb = 0.0;   // depth sums of un and ub
         const auto filter = [&](int k0, T *v) {
             T nv[KB], bv[KB];
+            double e3[KB];
             load(un, ij, k0, nv);
             load(ub, ij, k0, bv);
+            load_e3(k0, e3);
     #pragma unroll
             for (int q = 0; q < KB; q++) {
                 const int k = k0 + q + 1;
                 if (k > nlev) break;
-                const double mk = mask(k), e3 = NXT_E3(e3x, ij, k);
+                const double mk = mask(k), e3k = e3_of(k, e3[q]);
                 T a = v[q];
                 if (fix) a = (T)(((double)a - mean + uab) * mk);
                 if (zero) a = T(0);
@@ -407,7 +434,7 @@ struct S_dyn_nxt {
                 }
                 stp(plane_ptr(un, d.n2, k), ij, a);
                 v[q] = f;
-                const double tn = e3 * (double)a * mk, tb = e3 * (double)f * mk;
+                const double tn = e3k * (double)a * mk, tb = e3k * (double)f * mk;
                 sn = k == 1 ? tn : sn + tn;
                 sb = k == 1 ? tb : sb + tb;
             }
@@ -429,6 +456,8 @@ struct S_dyn_nxt {
         if (bt_fix) {
             const double cu = sb * r1h - unb;
             const auto correct = [&](int k0, const T *v) {
+                double e3[KB];
+                load_e3(k0, e3);
     #pragma unroll
                 for (int q = 0; q < KB; q++) {
                     const int k = k0 + q + 1;
@@ -436,7 +465,7 @@ struct S_dyn_nxt {
                     const double mk = mask(k);
                     const T nb = (T)((double)v[q] - cu * mk);
                     stp(plane_ptr(ub, d.n2, k), ij, nb);
-                    const double tb = NXT_E3(e3x, ij, k) * (double)nb * mk;
+                    const double tb = e3_of(k, e3[q]) * (double)nb * mk;
                     sb = k == 1 ? tb : sb + tb;
                 }
             };
@@ -525,7 +554,7 @@ int launch_dyn_nxt(int euler, T *ub, T *vb, T *un, T *vn, T *ua, T *va, const do
     const DevDomain &d = nh::dom();
     Grid2 g = grid2(d.jpi, d.jpj), gr = grid2(1, 1);
     g.grid.z = gr.grid.z = 2;
-    gr.grid.x = (unsigned)((2 * (d.jpi + d.jpj) - 4 + NH_BLOCK - 1) / NH_BLOCK);
+    gr.grid.x = (unsigned)((nxt_ring_rows(d) + (d.iper ? NXT_RING * 2 * (d.jpj - 2) : 0) + NH_BLOCK - 1) / NH_BLOCK);
 #define NXT_LAUNCH3(KM, U, R, gg)                                                                                    \
     LAUNCHB("dyn_nxt", (k_dyn_nxt<T, KM, U, R>), (S_dyn_nxt<T, KM, U, R>), gg, d, d.ln_dynspg_ts, d.ln_bt_fw, euler, \
             d.rn_atfp, ub, vb, un, vn, ua, va, ua_b, va_b, un_adv, vn_adv, ub_b, vb_b, un_b, vn_b, r1_hu, r1_hv)
