@@ -41,7 +41,9 @@ __device__ __forceinline__ void lbc_targets(const DevDomain &d, int i, int j, F 
 // and after both: ssh_nxt 471 -> 246 us, div_hor 389 -> 244 us, with 942 MB
 // each to move.  (wzv, one load per level, gains nothing from it.)
 #define NXT_KB 8
-// (Scale factors that vary take registers of their own: half as many levels.)
+// (Scale factors that vary are as many loads again, of 8 bytes each: two levels.
+// Four or eight crowd the caches, 260x230x50 FP64 44, 48 and 37 us for 4, 8 and 2;
+// level by level 49.)
 #define NXT_E3(p, ij, k) (E3U ? uld(p, (k) - 1) : E3(p, ij, k))
 
 // horizontal divergence at the interior point (i,j), DYN/divhor.F90:79-83.
@@ -49,7 +51,7 @@ __device__ __forceinline__ void lbc_targets(const DevDomain &d, int i, int j, F 
 // k0 (the last one repeated beyond kmax) with the reference's operation order.
 template <typename T, bool E3U>
 struct HdivCol {
-    static constexpr int KB = E3U ? NXT_KB : NXT_KB / 2;
+    static constexpr int KB = E3U ? NXT_KB : 2;
     double a1, a0, b1, b0, r;
     uint32_t ij;
     const T *un, *vn;
