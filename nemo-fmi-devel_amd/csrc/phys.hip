@@ -6,9 +6,13 @@
 // Arithmetic is FP64 in both storage forms, rounded once on store, in the
 // reference's operation order, so the FP64 form reproduces it bit for bit.
 //
-// The per-cell kernels of the density multiply by the t- or w-mask: a wave that
-// is dry at its level stores the zeros that gives and reads nothing.  512x509x75
-// FP32 TEOS-10: k_rab_poly 154 -> 134 us, k_eos_poly 121 -> 113.
+// The per-cell kernels of the density multiply by the t- or w-mask.  On domains
+// with enough dry waves (DRY, DevDomain::dry) a wave that is dry at its level
+// stores the zeros that gives and reads nothing: 512x509x75 FP32 TEOS-10, half of
+// it dry, k_rab_poly 154 -> 134 us, k_eos_poly 121 -> 113.  A wet wave then waits
+// for its mask before it asks for its operands, which an all-wet domain would pay
+// for nothing (600x500x60 FP32, TEOS-10: k_rab_poly 137 -> 160 us, k_eos_poly 107
+// -> 122; S-EOS: k_rab 83 -> 95, k_eos 66 -> 83): there the mask is loaded last.
 #include "common.hpp"
 #include "eos_poly.h"
 #include "kernels.hpp"
@@ -50,7 +54,7 @@ __device__ __forceinline__ double poly_z(const double (&c)[4][7][7], double zt, 
 // lines 399-437: polynomial TEOS-10 (SCH = 0) / EOS-80 (SCH = 1).  One
 // thread per cell, levels 1..jpkm1.
 // ---------------------------------------------------------------------------
-template <typename T, int POT, int SCH>
+template <typename T, int POT, int SCH, bool DRY>
 KERNEL void k_eos_poly(DevDomain d, const T *__restrict__ pts, T *__restrict__ prd, T *__restrict__ prhop,
                        const T *__restrict__ pdep)
 {
@@ -59,8 +63,9 @@ KERNEL void k_eos_poly(DevDomain d, const T *__restrict__ pts, T *__restrict__ p
     if (i > d.jpi || j > d.jpj) return;
     const nemo_eos_poly_t &P = EOS_POLY[SCH];
     const uint32_t p = IJK32(i, j, k);
-    const double ztm = TMASK(double, i, j, k);
-    if (!__any(ztm != 0.)) {
+    double ztm = 0.;
+    if (DRY) ztm = TMASK(double, i, j, k);
+    if (DRY && !__any(ztm != 0.)) {
         if (POT) at32(prhop, p) = T(0);
         at32(prd, p) = T(0);
         return;
@@ -69,6 +74,7 @@ KERNEL void k_eos_poly(DevDomain d, const T *__restrict__ pts, T *__restrict__ p
     const double zh = (double)at32(pdep, p) * P.r1_Z0;
     const double zt = (double)at32(pts, p) * P.r1_T0;
     const double zs = sqrt(fabs((double)at32(pts + d.n3, p) + P.rdeltaS) * P.r1_S0);
+    if (!DRY) ztm = TMASK(double, i, j, k);   // after the operands' loads
     double zn0;
     const double zn = poly_z<6, 4, 2, 1>(P.rho, zt, zs, zh, zn0);
     if (POT) at32(prhop, p) = (T)(zn0 * ztm);
@@ -76,7 +82,7 @@ KERNEL void k_eos_poly(DevDomain d, const T *__restrict__ pts, T *__restrict__ p
 }
 
 // rab_3d, TRA/eosbn2.F90:588-643: alpha and beta of the polynomial schemes
-template <typename T, int SCH>
+template <typename T, int SCH, bool DRY>
 KERNEL void k_rab_poly(DevDomain d, const T *__restrict__ pts, T *__restrict__ pab, const T *__restrict__ gdept)
 {
     THREAD_IJ(1, 1);
@@ -84,8 +90,9 @@ KERNEL void k_rab_poly(DevDomain d, const T *__restrict__ pts, T *__restrict__ p
     if (i > d.jpi || j > d.jpj) return;
     const nemo_eos_poly_t &P = EOS_POLY[SCH];
     const uint32_t p = IJK32(i, j, k);
-    const double ztm = TMASK(double, i, j, k);
-    if (!__any(ztm != 0.)) {
+    double ztm = 0.;
+    if (DRY) ztm = TMASK(double, i, j, k);
+    if (DRY && !__any(ztm != 0.)) {
         at32(pab, p) = T(0);
         at32(pab + d.n3, p) = T(0);
         return;
@@ -94,6 +101,7 @@ KERNEL void k_rab_poly(DevDomain d, const T *__restrict__ pts, T *__restrict__ p
     const double zh = (double)at32(gdept, p) * P.r1_Z0;
     const double zt = (double)at32(pts, p) * P.r1_T0;
     const double zs = sqrt(fabs((double)at32(pts + d.n3, p) + P.rdeltaS) * P.r1_S0);
+    if (!DRY) ztm = TMASK(double, i, j, k);   // after the operands' loads
     double z0;
     const double za = poly_z<5, 3, 1, 0>(P.alp, zt, zs, zh, z0);
     at32(pab, p) = (T)(za * r1_rau0 * ztm);
@@ -105,7 +113,7 @@ KERNEL void k_rab_poly(DevDomain d, const T *__restrict__ pts, T *__restrict__ p
 // eos_insitu (POT = 0), TRA/eosbn2.F90:276-299, and eos_insitu_pot (POT = 1),
 // lines 440-462, S-EOS.  One thread per cell, levels 1..jpkm1.
 // ---------------------------------------------------------------------------
-template <typename T, int POT>
+template <typename T, int POT, bool DRY>
 KERNEL void k_eos(DevDomain d, SeosPar e, const T *__restrict__ pts, T *__restrict__ prd, T *__restrict__ prhop,
                   const T *__restrict__ pdep)
 {
@@ -113,8 +121,9 @@ KERNEL void k_eos(DevDomain d, SeosPar e, const T *__restrict__ pts, T *__restri
     const int k = (int)blockIdx.z + 1;
     if (i > d.jpi || j > d.jpj) return;
     const uint32_t p = IJK32(i, j, k);
-    const double ztm = TMASK(double, i, j, k);
-    if (!__any(ztm != 0.)) {
+    double ztm = 0.;
+    if (DRY) ztm = TMASK(double, i, j, k);
+    if (DRY && !__any(ztm != 0.)) {
         if (POT) at32(prhop, p) = T(0);
         at32(prd, p) = T(0);
         return;
@@ -123,6 +132,7 @@ KERNEL void k_eos(DevDomain d, SeosPar e, const T *__restrict__ pts, T *__restri
     const double zt = (double)at32(pts, p) - 10.;
     const double zs = (double)at32(pts + d.n3, p) - 35.;
     const double zh = (double)at32(pdep, p);
+    if (!DRY) ztm = TMASK(double, i, j, k);
     if (POT) {
         double zn = -e.a0 * (1. + 0.5 * e.lambda1 * zt) * zt + e.b0 * (1. - 0.5 * e.lambda2 * zs) * zs -
                     e.nu * zt * zs;
@@ -137,7 +147,7 @@ KERNEL void k_eos(DevDomain d, SeosPar e, const T *__restrict__ pts, T *__restri
 }
 
 // rab_3d, TRA/eosbn2.F90:645-662 (S-EOS): alpha and beta at t-points
-template <typename T>
+template <typename T, bool DRY>
 KERNEL void k_rab(DevDomain d, SeosPar e, const T *__restrict__ pts, T *__restrict__ pab,
                   const T *__restrict__ gdept)
 {
@@ -145,8 +155,9 @@ KERNEL void k_rab(DevDomain d, SeosPar e, const T *__restrict__ pts, T *__restri
     const int k = (int)blockIdx.z + 1;
     if (i > d.jpi || j > d.jpj) return;
     const uint32_t p = IJK32(i, j, k);
-    const double ztm = TMASK(double, i, j, k);
-    if (!__any(ztm != 0.)) {
+    double ztm = 0.;
+    if (DRY) ztm = TMASK(double, i, j, k);
+    if (DRY && !__any(ztm != 0.)) {
         at32(pab, p) = T(0);
         at32(pab + d.n3, p) = T(0);
         return;
@@ -155,6 +166,7 @@ KERNEL void k_rab(DevDomain d, SeosPar e, const T *__restrict__ pts, T *__restri
     const double zt = (double)at32(pts, p) - 10.;
     const double zs = (double)at32(pts + d.n3, p) - 35.;
     const double zh = (double)at32(gdept, p);
+    if (!DRY) ztm = TMASK(double, i, j, k);
     double zn = e.a0 * (1. + e.lambda1 * zt + e.mu1 * zh) + e.nu * zs;
     at32(pab, p) = (T)(zn * r1_rau0 * ztm);
     zn = e.b0 * (1. - e.lambda2 * zs - e.mu2 * zh) - e.nu * zt;
@@ -304,35 +316,46 @@ __global__ __launch_bounds__(LDF_RX * LDF_RY, 4) void k_dyn_ldf_lap(DevDomain d,
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-template <typename T>
-int launch_eos(int neos, const SeosPar &e, int pot, const T *pts, T *prd, T *prhop, const T *pdep)
+template <typename T, bool DRY>
+static int launch_eos_d(int neos, const SeosPar &e, int pot, const T *pts, T *prd, T *prhop, const T *pdep)
 {
     const DevDomain &d = nh::dom();
     Grid2 g = grid2(d.jpi, d.jpj);
     g.grid.z = (unsigned)(d.jpk - 1);
     if (neos == NEMO_NP_TEOS10) {
-        if (pot) LAUNCH("eos", (k_eos_poly<T, 1, NEMO_EOS_POLY_TEOS10>), g, d, pts, prd, prhop, pdep);
-        else LAUNCH("eos", (k_eos_poly<T, 0, NEMO_EOS_POLY_TEOS10>), g, d, pts, prd, prhop, pdep);
+        if (pot) LAUNCH("eos", (k_eos_poly<T, 1, NEMO_EOS_POLY_TEOS10, DRY>), g, d, pts, prd, prhop, pdep);
+        else LAUNCH("eos", (k_eos_poly<T, 0, NEMO_EOS_POLY_TEOS10, DRY>), g, d, pts, prd, prhop, pdep);
     } else if (neos == NEMO_NP_EOS80) {
-        if (pot) LAUNCH("eos", (k_eos_poly<T, 1, NEMO_EOS_POLY_EOS80>), g, d, pts, prd, prhop, pdep);
-        else LAUNCH("eos", (k_eos_poly<T, 0, NEMO_EOS_POLY_EOS80>), g, d, pts, prd, prhop, pdep);
+        if (pot) LAUNCH("eos", (k_eos_poly<T, 1, NEMO_EOS_POLY_EOS80, DRY>), g, d, pts, prd, prhop, pdep);
+        else LAUNCH("eos", (k_eos_poly<T, 0, NEMO_EOS_POLY_EOS80, DRY>), g, d, pts, prd, prhop, pdep);
     } else {
-        if (pot) LAUNCH("eos", (k_eos<T, 1>), g, d, e, pts, prd, prhop, pdep);
-        else LAUNCH("eos", (k_eos<T, 0>), g, d, e, pts, prd, prhop, pdep);
+        if (pot) LAUNCH("eos", (k_eos<T, 1, DRY>), g, d, e, pts, prd, prhop, pdep);
+        else LAUNCH("eos", (k_eos<T, 0, DRY>), g, d, e, pts, prd, prhop, pdep);
     }
     return 0;
 }
-
 template <typename T>
-int launch_rab(int neos, const SeosPar &e, const T *pts, T *pab, const T *gdept)
+int launch_eos(int neos, const SeosPar &e, int pot, const T *pts, T *prd, T *prhop, const T *pdep)
+{
+    return nh::dom().dry ? launch_eos_d<T, true>(neos, e, pot, pts, prd, prhop, pdep)
+                         : launch_eos_d<T, false>(neos, e, pot, pts, prd, prhop, pdep);
+}
+
+template <typename T, bool DRY>
+static int launch_rab_d(int neos, const SeosPar &e, const T *pts, T *pab, const T *gdept)
 {
     const DevDomain &d = nh::dom();
     Grid2 g = grid2(d.jpi, d.jpj);
     g.grid.z = (unsigned)(d.jpk - 1);
-    if (neos == NEMO_NP_TEOS10) LAUNCH("rab", (k_rab_poly<T, NEMO_EOS_POLY_TEOS10>), g, d, pts, pab, gdept);
-    else if (neos == NEMO_NP_EOS80) LAUNCH("rab", (k_rab_poly<T, NEMO_EOS_POLY_EOS80>), g, d, pts, pab, gdept);
-    else LAUNCH("rab", k_rab<T>, g, d, e, pts, pab, gdept);
+    if (neos == NEMO_NP_TEOS10) LAUNCH("rab", (k_rab_poly<T, NEMO_EOS_POLY_TEOS10, DRY>), g, d, pts, pab, gdept);
+    else if (neos == NEMO_NP_EOS80) LAUNCH("rab", (k_rab_poly<T, NEMO_EOS_POLY_EOS80, DRY>), g, d, pts, pab, gdept);
+    else LAUNCH("rab", (k_rab<T, DRY>), g, d, e, pts, pab, gdept);
     return 0;
+}
+template <typename T>
+int launch_rab(int neos, const SeosPar &e, const T *pts, T *pab, const T *gdept)
+{
+    return nh::dom().dry ? launch_rab_d<T, true>(neos, e, pts, pab, gdept) : launch_rab_d<T, false>(neos, e, pts, pab, gdept);
 }
 
 template <typename T>
