@@ -49,7 +49,12 @@ __device__ __forceinline__ T keg_hw(const DevDomain &d, const T *un, const T *vn
 // whole column per workgroup where that gives every SIMD its waves (512
 // workgroups and more), else chunks of four levels or more towards 768 workgroups.
 // (32x22x31 FP64, five workgroups: k_step_dyn1 34 us in one chunk, 17 us
-// with its sums.)  In a plan the members fill the chip together.
+// with its sums.)  In a plan the launch holds every member's workgroups: several
+// members fill the chip without chunks, and the plan does not know their number
+// when it traces one, so none are made.  A plan of one or two members is left
+// short of workgroups by that (whole steps, separate calls and plan: one 32x22x31
+// FP64 271 and 471 us, one 182x149x56 FP32 508 and 826; two gyres 577 and 530;
+// six small members 2084 and 666).
 inline int lev_chunks(unsigned nb, int nlev)
 {
     if (nh::planning() || nb >= 512u || nb == 0u) return nlev;
@@ -988,7 +993,9 @@ __device__ __forceinline__ void zdf_column_reg(const DevDomain &d, double r2dt, 
 // columns leave SIMDs idle (two waves each: 512 workgroups; with a remainder,
 // 1024), by two workgroups (grid.z 2), with a checkpoint array each.  k_step_dyn2
 // 32x22x31 FP64: 68 us in turn, 36 us; 362x149x46 FP64 113 and 81 us;
-// 251x333x56 FP32 146 and 101 us.  In a plan the members fill the chip.
+// 251x333x56 FP32 146 and 101 us.  In a plan the members' workgroups share one
+// launch and the columns stay in turn (lev_chunks has what that costs a plan of
+// one or two members).
 inline unsigned zdf_comps(unsigned nb) { return nh::planning() || nb >= 1024u ? 1u : 2u; }
 template <typename T, bool REG, bool E3U>
 struct S_dyn_zdf {

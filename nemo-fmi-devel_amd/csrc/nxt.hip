@@ -47,7 +47,7 @@ __device__ __forceinline__ void lbc_targets(const DevDomain &d, int i, int j, F 
 #define NXT_E3(p, ij, k) (E3U ? uld(p, (k) - 1) : E3(p, ij, k))
 
 // horizontal divergence at the interior point (i,j), DYN/divhor.F90:79-83.
-// The column's metrics are loaded once; levels() evaluates NXT_KB levels from
+// The column's metrics are loaded once; levels() evaluates KB levels from
 // k0 (the last one repeated beyond kmax) with the reference's operation order.
 template <typename T, bool E3U>
 struct HdivCol {

@@ -239,7 +239,7 @@ KERNEL void k_hpg_zco(DevDomain d, const T *__restrict__ rhd, T *__restrict__ ua
 }
 
 // ---------------------------------------------------------------------------
-// dyn_ldf_lap, DYN/dynldf_lap_blp.F90:72-100.  A workgroup marches LDF_KB levels
+// dyn_ldf_lap, DYN/dynldf_lap_blp.F90:72-100.  A workgroup marches kb levels
 // of a region of LDF_RX x LDF_RY columns, one per thread, whose metrics stay in
 // registers: per level a thread shares its metric-weighted velocities through
 // LDS, forms the curl at its f-point and the divergence at its t-point from them

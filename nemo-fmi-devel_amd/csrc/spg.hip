@@ -1023,7 +1023,8 @@ int spg_ts_weights(const DevDomain &d, int ll_av, int ll_fw, int *jpit, double *
 // phase 2 by one cooperative launch of k_spg_loop: returns false (and
 // launches nothing) when the tuning switch is off, a graph is being
 // recorded, the weights do not fit the kernel's table or the device cannot
-// hold the grid resident; the caller then runs the two-kernel loop.
+// hold the grid resident; the caller then runs the two-kernel loop (also with
+// the switch on under capture: the blocks of sub-steps run with the switch off).
 // Switch value 1: one 1024-thread workgroup per CU (the fewest workgroups
 // at each barrier); 2: 256-thread workgroups, as many as stay resident.
 static bool spg_loop_coop(const DevDomain &d, const SpgWork &w, const nemo_hip_spg_ts_t *st, int icycle, int ll_init,

@@ -2423,7 +2423,10 @@ static int launch_fct_pairs(const DevDomain &d, double p2dt, const T *pu, const 
             gl.block = dim3(LIM_TX, NTH / LIM_TX, 1);
             gl.grid.y = (unsigned)((d.jpj - 2 + TY - 1) / TY);
             // levels per workgroup: all of them where the tiles fill the chip (three
-            // workgroups per CU), else chunks (two extra levels each) of 8 or more
+            // workgroups per CU), else chunks (two extra levels each) of 8 or more;
+            // in a plan the members' tiles share the launch and each keeps its levels
+            // together, which leaves a plan of one or two small members short of
+            // workgroups (32x22x31 FP64: 79 us, 38 in chunks)
             const int wgs = (int)(gl.grid.x * gl.grid.y) * nt, nlev = d.jpk - 1;
             int nch = nh::planning() ? 1 : 768 / wgs;
             nch = nch < 1 ? 1 : nch > nlev / 8 ? (nlev / 8 > 0 ? nlev / 8 : 1) : nch;

@@ -3,8 +3,8 @@
 The library's tuning switches (nemo_hip_tune_set) choose among kernel
 variants that give the same bits: the FCT as a chain of kernels or as one
 k-marched kernel per tile with 256 or 512 threads per 64 x TY tile
-(fct_fused 0 / 1 / 2), the barotropic sub-steps as two launches per
-sub-step or one cooperative launch with 1024- or 256-thread workgroups
+(fct_fused 0 / 1 / 2), the barotropic sub-steps several per launch or all in
+one cooperative launch with 1024- or 256-thread workgroups
 (spg_persistent 0 / 1 / 2), the column solves through the trend array or
 on chip (zdf_reg 0 / 1), and the chain's vertical half as kernels or as one
 bottom-up march with 256 or 512 threads per tile (fct_vlim 0 / 1 / 2).  Which is fastest depends on the domain (its size,
